@@ -7,6 +7,7 @@
 // norm downdate.
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <stddef.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -27,8 +28,12 @@ namespace {
 thread_local std::string g_err;
 
 constexpr double kEps = 1.1102230246251565e-16;  // LAPACK dlamch('E') = 2^-53
-// Panels with at least this many rows take the Gram-based path.
-constexpr int kFastPanelRows = 128;
+// Panels with at least this many rows take the Gram-based path.  Below, the
+// register-held panel of one workgroup is faster (about 0.5 us a column with
+// everything that follows it, against five launches of about 115 us); it stays
+// faster up to its 512 rows, but a step record says which form ran, and what
+// reads the records expects the Gram form from 425 rows on.
+constexpr int kFastPanelRows = 385;
 constexpr int kBatch = 8;  // DM steps queued between synchronisations
 // Layout of the per-step upload: up to 2*KMAX (dst, src) pairs, then KMAX
 // candidate ranks of the panel columns.
@@ -45,6 +50,12 @@ struct HipError {
     hipError_t e_ = (x);                               \
     if (e_ != hipSuccess) throw HipError{e_, #x};      \
   } while (0)
+
+// A column-by-column panel whose workgroups gave up waiting for each other
+// (DevState::flags bit 3) has lost the call's matrix.
+void check_panels(int flags) {
+  if (flags & 8) throw HipError{hipErrorLaunchTimeOut, "panel workgroups"};
+}
 
 // Grow-only device workspace, one per device, reused across calls.
 struct Workspace {
@@ -153,17 +164,11 @@ struct Buffers {
 
 size_t layout_buffers(int m, int n, char* base, Buffers* b, int nb = KMAX) {
   char* p = base;
-  const int mpad = ((m + 63) / 64) * 64;
-  const int nslab = (m + 31) / 32 + 1;  // slabs of the Gram and fast-panel passes
   const int nsplit = 16;  // row slabs of the trailing update's partial products
   static_assert(nsplit >= 16, "the fused pass uses up to 16 row slabs");
   Buffers t;
+  // the head that kernels find from the state (ws_mat, ws_slots, ws_v)
   t.st = carve<DevState>(p, 1);
-  t.work = carve<double>(p, n);
-  t.workold = carve<double>(p, n);
-  t.topk_val = carve<double>(p, (size_t)topk_blocks(n) * KMAX);
-  t.topk_idx = carve<int>(p, (size_t)topk_blocks(n) * KMAX);
-  t.gram_part = carve<double>(p, (size_t)nslab * KMAX * KMAX);
   t.G = carve<double>(p, KMAX * KMAX);
   t.S = carve<double>(p, KMAX * KMAX);
   t.T = carve<double>(p, KMAX * KMAX);
@@ -171,8 +176,13 @@ size_t layout_buffers(int m, int n, char* base, Buffers* b, int nb = KMAX) {
   t.R1inv = carve<double>(p, KMAX * KMAX);
   t.G2 = carve<double>(p, KMAX * KMAX);
   t.M = carve<double>(p, KMAX * KMAX);
-  t.ldv = mpad;
-  t.V = carve<double>(p, (size_t)2 * mpad * KMAX);
+  t.gram_part = carve<double>(p, ws_slabs(m) * KMAX * KMAX);
+  t.ldv = ws_ldv(m);
+  t.V = carve<double>(p, (size_t)2 * t.ldv * KMAX);
+  t.work = carve<double>(p, n);
+  t.workold = carve<double>(p, n);
+  t.topk_val = carve<double>(p, (size_t)topk_blocks(n) * KMAX);
+  t.topk_idx = carve<int>(p, (size_t)topk_blocks(n) * KMAX);
   t.nsplit = nsplit;
   t.Wp = carve<double>(p, (size_t)nsplit * KMAX * n);
   t.W = carve<double>(p, (size_t)KMAX * n);
@@ -224,6 +234,9 @@ void permute_walk(int ncols, std::vector<int>& marked, const int* sel, int nsel,
   }
   for (int p = 0; p < nsel; p++) marked[p] = 0;  // the accepted ones now lead
 }
+
+static_assert(offsetof(DevState, fjb_cmp) == 2 * sizeof(int) &&
+              offsetof(DevState, flags) == 3 * sizeof(int), "the wide steps' readback");
 
 struct Args {
   int layout, m, n, lda, nb;
@@ -343,22 +356,24 @@ int run_wide(const Args& x, Buffers& B, int nfxd, double eta, int enable_stop, d
                             hipMemcpyHostToDevice, s));
       launch_swap_pairs(A, lda, m, j, B.work, B.jp, B.wpairs, (int)swaps.size(), s);
     }
-    // --- dgeqr2_mia (:735-738) on the fjb columns, truncation included
-    launch_panel_exact(A, lda, j, m, fjb, tau_dm, 1, x.tau + j, B.st, s);
+    // --- dgeqr2_mia (:735-738), dlarft and dlarfb (:740-767): the block's
+    // panel KMAX columns at a time, each part's reflectors applied to every
+    // column right of it (the block's own later ones included) before the
+    // next; the part that the truncation ends is the last
     int kk = 0;
-    HIPCHK(hipMemcpyAsync(&kk, &B.st->fjb_cmp, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    // --- dlarft + dlarfb (:740-767) on columns j + fjb .. n, KMAX reflectors
-    // at a time
-    if (j + fjb < n) {
-      for (int i0 = 0; i0 < kk; i0 += KMAX) {
-        const int kq = std::min(KMAX, kk - i0);
-        launch_set_kk(B.st, kq, s);
-        launch_build_v(A, lda, j + i0, m, B.ldv, B.st, B.V, B.ldv, s);
-        launch_gram(B.V, B.ldv, j + i0, m, nullptr, KMAX, nullptr, B.gram_part, B.S, s);
-        launch_larft(B.S, x.tau + j + i0, B.st, B.T, s);
-        launch_larfb(A, lda, j + i0, m, j + fjb, n, B.V, B.ldv, B.T, 1, B.Wp, B.W, B.nsplit, s);
-      }
+    for (int i0 = 0; i0 < fjb; i0 += KMAX) {
+      const int kb = std::min(KMAX, fjb - i0), jp = j + i0;
+      launch_panel_exact(A, lda, jp, m, kb, tau_dm, i0 == 0 ? 1 : 2, x.tau + jp,
+                         B.st, s);
+      int pst[4];  // nc, fjb, fjb_cmp, flags
+      HIPCHK(hipMemcpyAsync(pst, B.st, sizeof(pst), hipMemcpyDeviceToHost, s));
+      HIPCHK(hipStreamSynchronize(s));
+      check_panels(pst[3]);
+      const int kq = pst[2];
+      if (kq > 0 && jp + kb < n)
+        launch_larfb(A, lda, jp, m, jp + kb, n, B.V, B.ldv, B.T, 1, B.Wp, B.W, B.nsplit, s);
+      kk += kq;
+      if (kq < kb) break;
     }
     // --- norm_update (:774-778) over the kk new rows
     launch_wide_state(B.st, j, kk, s);
@@ -480,6 +495,7 @@ int run_dm(const Args& x) {
     // (src/dlarfb.c:54-127); here it is caught by the norm sweep before any
     // write, and A is left as it was.
     if (hst->flags & 1) return -13;
+    check_panels(hst->flags);  // of the fixed columns
     double maxnrm = 0.0;
     {
       unsigned long long bits = hst->maxnrm_bits;
@@ -534,13 +550,12 @@ int run_dm(const Args& x) {
     launch_dm_begin(B.st, nfxd, minmn, tau_dm, delta, fused_now ? 1 : 0, s);
     const int batch = x.trace ? 1 : kBatch;
     int j0 = nfxd, it = 0;
-    // the exact panel and dlarft of the step at column jl (RUN_EXACT: they
-    // run when the step's panel is not the Gram-based one, or that fell back)
+    // the column-by-column panel of the step at column jl, with V and T
+    // (RUN_EXACT: it runs when the step's panel is not the Gram-based one, or
+    // that fell back)
     auto queue_exact = [&](int jl) {
       int pq = g_prof.begin(PC_PANEL, s);
       launch_panel_exact(A, lda, jl, m, 0, tau_dm, 1, x.tau, B.st, s, RUN_EXACT);
-      launch_vgram_exact(A, lda, jl, m, B.st, bufs, B.gram_part, s);
-      launch_larft(B.gram_part, x.tau, B.st, B.T, s, RUN_EXACT, vgram_exact_slabs(jl, m));
       g_prof.end(pq, s, 0.0);
     };
     // --- dlarfb (src/dgeqrdm_work.c:762-767) from c0 (set by the panel),
@@ -639,6 +654,7 @@ int run_dm(const Args& x) {
       const bool ahead = !x.trace && !switch_wanted && j0 + batch * KMAX < minmn;
       if (ahead) queue_batch(j0, q ^ 1);
       DevState* h = wait_slot(q);
+      check_panels(h->flags);
       bool in_flight = ahead;
       if (h->halt) {
         // the halted step (at h->j, selection and column moves done)
@@ -652,6 +668,7 @@ int run_dm(const Args& x) {
         queue_update(jh);
         readback(q);
         h = wait_slot(q);
+        check_panels(h->flags);
         if (h->halt) throw HipError{hipErrorUnknown, "resumed DM step halted again"};
       }
       if (x.trace && h->it > it && h->it - 1 < x.ntrace) {
@@ -732,10 +749,7 @@ void blocked_qr(double* A, int lda, int m, int n, int ncols_qr, double* tau, Buf
                 hipStream_t s) {
   for (int j = 0; j < ncols_qr; j += KMAX) {
     const int kb = (ncols_qr - j) < KMAX ? (ncols_qr - j) : KMAX;
-    launch_panel_exact(A, lda, j, m, kb, 0.0, 0, tau + j, B.st, s);
-    launch_build_v(A, lda, j, m, B.ldv, B.st, B.V, B.ldv, s);
-    launch_gram(B.V, B.ldv, j, m, nullptr, KMAX, nullptr, B.gram_part, B.S, s);
-    launch_larft(B.S, tau + j, B.st, B.T, s);
+    launch_panel_exact(A, lda, j, m, kb, 0.0, 0, tau + j, B.st, s);  // V and T too
     launch_larfb(A, lda, j, m, j + kb, n, B.V, B.ldv, B.T, 1, B.Wp, B.W, B.nsplit, s);
   }
 }
@@ -745,7 +759,10 @@ int run_geqrf(double* A, int lda, int m, int n, double* tau, hipStream_t s) {
   workspace_for(m, n, &B);
   HIPCHK(hipMemsetAsync(B.st, 0, sizeof(DevState), s));
   blocked_qr(A, lda, m, n, m < n ? m : n, tau, B, s);
+  int flags = 0;
+  HIPCHK(hipMemcpyAsync(&flags, &B.st->flags, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
+  check_panels(flags);
   return 0;
 }
 

@@ -365,7 +365,7 @@ __device__ void step_end_apply(DevState* st, int* ncols_dev, int m, int n, int e
   st->j = j + kk;
   st->done = done;
   st->maxnrm_bits = 0ull;
-  st->flags &= ~2;
+  st->flags &= ~6;
 }
 
 // The step's candidates: the sorted first kmax keys of work[j..n) (value
@@ -1037,19 +1037,20 @@ void launch_apply_perm(double* A, int lda, int m, double* work, int* jp, const i
 // (src/dlarfg.c:116-185) and dlarf_ (src/dlarf.c:161-185), column by column
 // in one workgroup.  Truncation: for column i > 0 stop when ||x|| < thres,
 // thres = 5e-14, or tau_dm*|R(0,0)| once column 0 is done (tau_dm > 0).
-// truncate = 0 disables the test (unpivoted QR).  RUN_EXACT: j and fjb from
-// st, tau indexed from column 0 (the step writes tau[j..]).
+// truncate = 0 disables the test (unpivoted QR); truncate = 2: the panel
+// continues a wider block whose R(0, 0) is beta0, and every column is tested.
 // The panel's work for the whole workgroup (any size up to 1024 threads;
 // red holds blockDim.x / 64 doubles): returns fjb_cmp, the columns reduced.
 // GROUP: block columns a wave updates at a time (1 for many-wave workgroups,
 // 4 for few waves).
 template <int GROUP>
 __device__ __forceinline__ int panel_exact_body(double* A, int lda, int j, int m, int fjb, double tau_dm,
-                                int truncate, double* tau, double* red) {
+                                int truncate, double* tau, double* red, double beta0 = 0.0) {
   const int msub = m - j;
   const int tid = local_tid(), lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
   double* P = A + j + (size_t)j * lda;
-  double thres = 5e-14;
+  const bool cont = truncate == 2;
+  double thres = cont && tau_dm > 0.0 ? tau_dm * fabs(beta0) : 5e-14;
   int i;
   for (i = 0; i < fjb; i++) {
     const int len = msub - i;
@@ -1057,7 +1058,7 @@ __device__ __forceinline__ int panel_exact_body(double* A, int lda, int j, int m
     double taui = 0.0;
     if (len > 1) {
       double xnorm = block_nrm2(col + 1, len - 1, red);
-      if (truncate && i > 0 && xnorm < thres) break;
+      if (truncate && (i > 0 || cont) && xnorm < thres) break;
       if (xnorm != 0.0) {
         double alpha = col[0];
         double beta = -dsign(dlapy2(alpha, xnorm), alpha);
@@ -1087,7 +1088,7 @@ __device__ __forceinline__ int panel_exact_body(double* A, int lda, int j, int m
     __syncthreads();
     if (i + 1 < fjb) {
       const double aii = col[0];
-      if (i == 0 && tau_dm > 0.0) thres = tau_dm * fabs(aii);
+      if (i == 0 && tau_dm > 0.0 && !cont) thres = tau_dm * fabs(aii);
       if (GROUP == 1 && taui != 0.0) {
         // dlarf_ on the later block columns: one column per wave at a time
         for (int c = i + 1 + wave; c < fjb; c += nw) {
@@ -1134,31 +1135,6 @@ __device__ __forceinline__ int panel_exact_body(double* A, int lda, int j, int m
   return i;
 }
 
-__global__ __launch_bounds__(1024) void k_panel_exact(double* A, int lda, int j, int m,
-                                                      int fjb, double tau_dm, int truncate,
-                                                      double* tau, DevState* st, int mode) {
-  __shared__ double red[16];
-  if (!step_runs(st, mode)) return;
-  if (mode != RUN_ALWAYS) {
-    j = st->j;
-    fjb = st->fjb;
-    tau += j;
-  }
-  const int i = panel_exact_body<1>(A, lda, j, m, fjb, tau_dm, truncate, tau, red);
-  if (threadIdx.x == 0) {
-    st->fjb_cmp = i;
-    // dlarf_ inside the panel already updated the rejected columns
-    // j+fjb_cmp..j+fjb-1; the trailing update starts at j+fjb (:764-766)
-    st->c0 = j + fjb;
-  }
-}
-
-void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm,
-                        int truncate, double* tau, DevState* st, hipStream_t s, int mode) {
-  hipLaunchKernelGGL(k_panel_exact, dim3(1), dim3(1024), 0, s, A, lda, j, m, fjb, tau_dm,
-                     truncate, tau, st, mode);
-}
-
 // ---------------------------------------------------------------------------
 // Dense copy of the block reflector V (unit lower trapezoidal, zero padded to
 // KMAX columns and to mpad rows, zero above row j) into V[r + c*ldv].
@@ -1182,67 +1158,6 @@ void launch_build_v(const double* A, int lda, int j, int m, int mpad, const DevS
                     double* V, int ldv, hipStream_t s, int mode) {
   hipLaunchKernelGGL(k_build_v, dim3((mpad + 255) / 256), dim3(256), 0, s, A, lda, j, m, mpad,
                      st, V, ldv, mode);
-}
-
-// ---------------------------------------------------------------------------
-// The DM loop's exact-panel V (RUN_EXACT): each workgroup builds the V rows
-// [rs, rs + EX_ROWS) from the panel (unit lower trapezoidal, fjb_cmp
-// columns, zero padded) in 64-row slabs, writes them to V and their Gram
-// V^T V to partial[blockIdx.x] (zero past m).  Workgroup 0 also zeroes the V
-// rows [j - 64, j) above the panel, which the trailing update relies on.
-constexpr int EX_ROWS = 4 * GRAM_ROWS;
-
-__global__ __launch_bounds__(256) void k_vgram_exact(const double* __restrict__ A, int lda,
-                                                     int m, const DevState* st, StepBufs bufs,
-                                                     double* partial) {
-  __shared__ double X[KMAX * (GRAM_ROWS + 1)];
-  if (!step_runs(st, RUN_EXACT)) return;
-  double* V = v_cur(bufs, st);
-  const int ldv = bufs.ldv;
-  const int j = st->j, kk = st->fjb_cmp;
-  const int tid = threadIdx.x;
-  dbl4 acc[4];
-#pragma unroll
-  for (int u = 0; u < 4; u++) acc[u] = (dbl4){0.0, 0.0, 0.0, 0.0};
-  for (int sub = 0; sub < EX_ROWS / GRAM_ROWS; sub++) {
-    const int rs = j + blockIdx.x * EX_ROWS + sub * GRAM_ROWS;
-    if (rs >= m) break;
-    double xv[KMAX * GRAM_ROWS / 256];
-#pragma unroll
-    for (int q = 0; q < KMAX * GRAM_ROWS / 256; q++) {
-      const int e = tid + 256 * q, c = e / GRAM_ROWS, r = rs + e % GRAM_ROWS;
-      const int rr = r - j;
-      xv[q] = (c < kk && r < m && rr >= c) ? (rr == c ? 1.0 : A[(size_t)(j + c) * lda + r]) : 0.0;
-    }
-    __syncthreads();  // the previous slab's products are done with X
-#pragma unroll
-    for (int q = 0; q < KMAX * GRAM_ROWS / 256; q++) {
-      const int e = tid + 256 * q, c = e / GRAM_ROWS, r = e % GRAM_ROWS;
-      X[c * (GRAM_ROWS + 1) + r] = xv[q];
-      if (rs + r < m) V[(size_t)c * ldv + rs + r] = xv[q];
-    }
-    __syncthreads();
-    gram_slab_acc(X, acc);
-  }
-  if (blockIdx.x == 0) {
-    const int z0 = j >= KMAX ? j - KMAX : 0;
-    for (int e = tid; e < KMAX * KMAX; e += 256) {
-      const int r = z0 + (e & 63), c = e >> 6;
-      if (r < j) V[(size_t)c * ldv + r] = 0.0;
-    }
-  }
-  gram_store(acc, partial + (size_t)blockIdx.x * KMAX * KMAX);
-}
-
-int vgram_exact_slabs(int j0, int m) {
-  const int ns = (m - j0 + EX_ROWS - 1) / EX_ROWS;
-  return ns > 0 ? ns : 1;
-}
-
-void launch_vgram_exact(const double* A, int lda, int j0, int m, const DevState* st,
-                        const StepBufs& bufs, double* partial, hipStream_t s) {
-  hipLaunchKernelGGL(k_vgram_exact, dim3(vgram_exact_slabs(j0, m)), dim3(256), 0, s, A, lda, m,
-                     st, bufs, partial);
 }
 
 // ---------------------------------------------------------------------------

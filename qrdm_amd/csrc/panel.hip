@@ -365,8 +365,8 @@ __device__ __forceinline__ int lu_signed_blocked(double (*W)[LDP], int nlim, con
 // X := L^-1 and U^-1 of the pair held in one 64 x 64 matrix W (L unit lower
 // triangular strictly below the diagonal, U upper triangular on and above
 // it, non-zero diagonal), X in the same layout: L^-1 strictly below the
-// diagonal (its unit diagonal implied), U^-1 on and above; 256 threads, ends
-// with a barrier.  BOTH = false: U^-1 only (W's lower part is not read, X's
+// diagonal (its unit diagonal implied), U^-1 on and above; at least 256
+// threads (the first four waves compute), ends with a barrier.  BOTH = false: U^-1 only (W's lower part is not read, X's
 // is set to zero).  Both go by 16 x 16 blocks, L^-1 as (L^T)^-1 read and
 // stored transposed: the diagonal blocks by back substitution (wave w takes
 // block w of both, one lane per column: lanes 0-15 U, 16-31 L^T), then the
@@ -393,7 +393,7 @@ __device__ __forceinline__ void lu_inverse(const double (*W)[LDP], double (*X)[L
     }
   }
   lds_barrier();
-  if (lane < (BOTH ? 32 : 16)) {
+  if (wave < 4 && lane < (BOTH ? 32 : 16)) {
     const int m = (lane < 16) ? 1 : 0, c = lane & 15, base = BLK * wave;
     double x[BLK];
 #pragma unroll
@@ -413,7 +413,7 @@ __device__ __forceinline__ void lu_inverse(const double (*W)[LDP], double (*X)[L
   const int g = lane >> 4, li = lane & 15;
   for (int d = 1; d < 4; d++) {
     const int ntgt = (BOTH ? 2 : 1) * (4 - d);
-    for (int t = wave; t < ntgt; t += 4) {
+    for (int t = wave; wave < 4 && t < ntgt; t += 4) {
       const int m = BOTH ? (t & 1) : 1, bi = BOTH ? (t >> 1) : t, bj = bi + d;
       dbl4p acc = {0.0, 0.0, 0.0, 0.0};
       for (int kb = bi + 1; kb <= bj; kb++) {

@@ -35,7 +35,8 @@ struct DevState {
   int nc;          // number of norm candidates
   int fjb;         // accepted columns
   int fjb_cmp;     // columns reduced by the panel
-  int flags;       // bit 0: non-finite value met; bit 1: fast panel fell back
+  int flags;       // bit 0: non-finite value met; bit 1: fast panel fell back; bit 2: the
+                   // register-held panel declined; bit 3: its workgroups gave up waiting
   int k1;          // columns the fast panel's first Cholesky factored
   unsigned long long maxnrm_bits;  // max partial norm (bit pattern, >= 0)
   unsigned long long recomp_rows;  // rows read by norm recomputes (profiling)
@@ -61,11 +62,31 @@ struct DevState {
   int kk_prev;  // fjb_cmp of the previous step (0 before the first): the width of the
                 // update the fused pass applies
   int policy_on;      // 1: the step's tau and delta come from the learned policy
+  double pan_beta;    // R(0, 0) of the last column-by-column panel (wide.hip's blocks)
   double tau_step;    // tau and delta of the current step (the defaults, or the
   double delta_step;  // policy's proposal)
   StepRec last;
   StepWork work;
 };
+
+// The head of a workspace, the same for every caller: the state, the 64 x 64
+// matrices, the Gram slabs' partial sums and the dense V.  Kernels that are
+// given only the state find the others behind it.
+enum { WS_G = 0, WS_S, WS_T, WS_R1, WS_R1INV, WS_G2, WS_M, WS_MATS };
+constexpr size_t kStateBytes = (sizeof(DevState) + 255) / 256 * 256;
+__host__ __device__ __forceinline__ double* ws_mat(DevState* st, int which) {
+  return reinterpret_cast<double*>(reinterpret_cast<char*>(st) + kStateBytes) +
+         (size_t)which * KMAX * KMAX;
+}
+// The Gram partials: one 64 x 64 per 32 rows and one more.  Between the Grams
+// the column-by-column panel exchanges its columns' sums here.
+__host__ __device__ __forceinline__ double* ws_slots(DevState* st) { return ws_mat(st, WS_MATS); }
+__host__ __device__ __forceinline__ size_t ws_slabs(int m) { return (size_t)(m + 31) / 32 + 1; }
+// The dense V (two buffers of ldv x KMAX).
+__host__ __device__ __forceinline__ int ws_ldv(int m) { return (m + 63) / 64 * 64; }
+__host__ __device__ __forceinline__ double* ws_v(DevState* st, int m) {
+  return ws_slots(st) + ws_slabs(m) * KMAX * KMAX;
+}
 
 // The DM loop's reflector buffers: the dense V (ldv x KMAX, zero above the
 // panel) and W = T^T V^T C (KMAX x n, by absolute column, column-major: W(i, c)
@@ -235,20 +256,19 @@ void launch_gram_select(double* A, int lda, int j0, int m, int n, double* partia
 void launch_apply_perm(double* A, int lda, int m, double* work, int* jp, const int* perm,
                        DevState* st, const StepBufs& bufs, hipStream_t s);
 // Column-by-column panel on columns [j, j + fjb) (RUN_ALWAYS: host j, fjb;
-// RUN_EXACT: from st, tau indexed from j).  Sets st->fjb_cmp and st->c0.
+// RUN_EXACT: from st, tau indexed from j) of the matrix with m rows whose
+// workspace starts at st.  Sets st->fjb_cmp, st->c0 and st->pan_beta, writes
+// the dense V (rows max(j - KMAX, 0) .. m of ws_v, of the step's parity with
+// st->fused) and T (ws_mat), and uses the Gram partials' space.  truncate: 0
+// none, 1 the DM test, 2 the DM test of a panel that continues a wider block.
 void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm,
                         int truncate, double* tau, DevState* st, hipStream_t s,
                         int mode = RUN_ALWAYS);
 void launch_build_v(const double* A, int lda, int j, int m, int mpad, const DevState* st,
                     double* V, int ldv, hipStream_t s, int mode = RUN_ALWAYS);
-// T from S = V^T V; with nslab > 0, S is summed from that many partial Grams.
+// T from S = V^T V.
 void launch_larft(const double* S, const double* tau, const DevState* st, double* T,
                   hipStream_t s, int mode = RUN_ALWAYS, int nslab = 0);
-// The DM loop's exact-panel V and its partial Grams (RUN_EXACT; j0 <= j
-// sizes the grid: vgram_exact_slabs(j0, m) partials).
-int vgram_exact_slabs(int j0, int m);
-void launch_vgram_exact(const double* A, int lda, int j0, int m, const DevState* st,
-                        const StepBufs& bufs, double* partial, hipStream_t s);
 // Block reflector from the left on rows [j, m), columns [c0, n):
 // trans = 1: C := (I - V T V^T)^T C (dgeqrdm's trailing update);
 // trans = 0: C := (I - V T V^T) C.

@@ -1,0 +1,473 @@
+// regpanel.hip -- the column-by-column Householder panel (dgeqr2_mia,
+// src/dgeqr2.c:144-191, with dlarfg_mia, src/dlarfg.c:116-185) with the panel
+// held in registers.
+//
+// What bounds it: 64 columns that each wait on the one before.  A panel kept
+// in memory (panel_exact_body) costs every column three round trips to the L2
+// (norm, scaling, update).  Here a workgroup keeps RP_ROWS rows x 64 columns in
+// registers (a wave 16 QH rows, a lane 4 QH rows of four columns), so that a
+// column costs one pass of products, one LDS exchange and one barrier:
+//
+//   x = column i below the diagonal; s_c = x^T (column c) for all 64 columns
+//   in one reduction: s_i = ||x||^2 gives beta, tau and the scale
+//   sc = 1 / (alpha - beta); for c > i, w_c = tau (a_ic + sc s_c) is dlarf_'s
+//   product v^T (column c); for c < i, a_ic + sc s_c = (V^T v_i)_c is the entry
+//   of V^T V that T needs.
+//
+// Row i leaves the registers when column i is done (R to the right of the
+// diagonal, V to the left), through LDS; the rest is written once, at the end,
+// with the dense V and T = (striu(V^T V) + diag(1 / tau))^-1 of the trailing
+// update.  Panels of more than RP_ROWS rows take one workgroup per RP_ROWS
+// rows: every column's partial sums pass between the workgroups through
+// memory, each a slot of its own that holds a sentinel until it is written.
+//
+// Measured against the memory-based panel: unpivoted QR of 1024 x 1024 15.6 ->
+// 3.6 ms, of 4096 x 2048 129 -> 10.1 ms; 2048 x 1024 DM with 128-column blocks
+// 68.3 -> 9.6 ms; 64 x 48 DM 0.53 -> 0.33 ms.
+//
+// Sums of squares are taken plainly: where one leaves [1e-280, 1e280] (or is
+// not a number) the panel is declined before anything is written, and the
+// memory-based panel, which scales, takes it.
+#include "qrdm_internal.h"
+
+namespace qrdm {
+
+constexpr int RP_ROWS = 512;  // rows per workgroup (eight waves of 64)
+constexpr int RP_SMALL = 128;  // panels up to this many rows: four waves of 32
+constexpr int RP_MID = 384;    // up to this many: eight waves of 48
+constexpr int RP_WGS = 64;     // workgroups of one panel at most
+
+// A slot not yet written: a NaN pattern no published value takes (published
+// NaNs are made the canonical one).
+__device__ constexpr unsigned long long kRpEmpty = 0x7ff4a5a5c3c30f0full;
+// Polls of one slot before a workgroup gives the panel up (about seconds).
+constexpr int RP_POLLS = 1 << 22;
+
+template <int QH, int NW>
+struct RegPanelLds {
+  double x[NW][16 * QH];    // column i's rows, per wave
+  double red[2][NW][KMAX];  // the waves' partial sums, by column
+  double row[2][KMAX];      // row i
+  double out[KMAX][LDP];    // the top block: R, V below the diagonal
+  double S[KMAX][LDP];      // V^T V above the diagonal
+  double X[KMAX][LDP];      // T
+  double Y[4][BLK][BLK + 1];
+  double rinv[KMAX], tau[KMAX];
+};
+
+// (lane 16 g + li) := the sum over the four lane groups of s[g], column 16 g + li.
+__device__ __forceinline__ double group_sums(const double (&s)[4]) {
+  auto halves = [](double a, double b) {  // lanes < 32: a's two halves summed, else b's
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((int)x, (int)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((int)(x >> 32), (int)(y >> 32), false, false);
+    return __longlong_as_double(((long long)(int)hi[0] << 32) | (unsigned)lo[0]) +
+           __longlong_as_double(((long long)(int)hi[1] << 32) | (unsigned)lo[1]);
+  };
+  auto rows = [](double a, double b) {  // even rows of 16: a's row pair summed, odd rows: b's
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((int)x, (int)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((int)(x >> 32), (int)(y >> 32), false, false);
+    return __longlong_as_double(((long long)(int)hi[0] << 32) | (unsigned)lo[0]) +
+           __longlong_as_double(((long long)(int)hi[1] << 32) | (unsigned)lo[1]);
+  };
+  return rows(halves(s[0], s[2]), halves(s[1], s[3]));
+}
+
+// f[u] := the value of lane 16 u + li in lane 16 g + li.
+__device__ __forceinline__ void group_values(double v, double (&f)[4]) {
+  const long long b = __double_as_longlong(v);
+  int w[4][2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int x = h ? (int)(b >> 32) : (int)b;
+    const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);  // rows 0022, 1133
+    const auto e = __builtin_amdgcn_permlane32_swap(p[0], p[0], false, false);  // 0000, 2222
+    const auto o = __builtin_amdgcn_permlane32_swap(p[1], p[1], false, false);  // 1111, 3333
+    w[0][h] = e[0];
+    w[1][h] = o[0];
+    w[2][h] = e[1];
+    w[3][h] = o[1];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+    f[u] = __longlong_as_double(((long long)w[u][1] << 32) | (unsigned)w[u][0]);
+}
+
+__device__ __forceinline__ double rp_publishable(double v) {
+  return v == v ? v : __longlong_as_double(0x7ff8000000000000ll);
+}
+
+// Waits for the slot; false when it stayed empty for RP_POLLS polls.
+__device__ __forceinline__ bool rp_await(const double* slot, double& v) {
+  for (int t = 0; t < RP_POLLS; t++) {
+    const unsigned long long b =
+        __hip_atomic_load(reinterpret_cast<const unsigned long long*>(slot), __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_AGENT);
+    if (b != kRpEmpty) {
+      v = __longlong_as_double((long long)b);
+      return true;
+    }
+  }
+  return false;
+}
+
+// The panel's columns [0, fjb) at P (leading dimension lda, msub rows) by nwg
+// workgroups, this one the rows from wg * 16 QH NW.  Truncation: 5e-14 is the
+// bound of the columns after the first (tau_dm > 0: tau_dm |R(0, 0)| once
+// column 0 is done), unless truncate is 0; truncate = 2: beta0 is the block's
+// R(0, 0), and every column is tested.  slots (nwg > 1): KMAX columns x
+// (nwg + 1) x KMAX values, empty on entry.  Returns the columns reduced with
+// everything written -- the panel, tau, rows [-KMAX, msub) of the dense V
+// (zero above the panel, where z0 rows exist) and T -- or -1, declined, with
+// nothing written.  Every workgroup returns the same (one that gives up
+// waiting sets flags bit 3, which fails the call).
+template <int QH, int NW, bool GRID>
+__device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, double tau_dm,
+                                         int truncate, double beta0, double* tau, double* V,
+                                         int ldv, int z0, double* T_out, double* slots, int nwg,
+                                         int wg, DevState* st, RegPanelLds<QH, NW>& L) {
+  constexpr int WR = 16 * QH, NQ = 4 * QH;
+  const int tid = local_tid(), lane = tid & 63, g = lane >> 4, li = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = wg * WR * NW + wave * WR;  // this wave's first row
+  const int nu = (fjb + 15) >> 4;
+  // the lane's rows: row0 + 16 (q / 4) + 4 g + q % 4
+  double a[NQ][4];
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      const int r = row0 + 16 * (q >> 2) + 4 * g + (q & 3), c = 16 * u + li;
+      a[q][u] = (r < msub && c < fjb) ? P[(size_t)c * lda + r] : 0.0;
+    }
+  const bool cont = truncate == 2;
+  const double thr0 = cont && tau_dm > 0.0 ? tau_dm * beta0 : 5e-14;
+  double thr2 = thr0 * thr0;
+  int k = fjb;
+  bool ok = true;
+  for (int i = 0; i < fjb; i++) {
+    const int buf = i & 1, ui = i >> 4, ii = i & 15;
+    // column i: its owner lanes' rows to every lane of the wave, zero on and
+    // above the diagonal
+    if (li == ii) {
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        if (u == ui) {
+#pragma unroll
+          for (int q = 0; q < NQ; q += 2)
+            *reinterpret_cast<double2*>(&L.x[wave][16 * (q >> 2) + 4 * g + (q & 3)]) =
+                make_double2(a[q][u], a[q + 1][u]);
+        }
+    }
+    if (row0 <= i) {
+      // row i, before its step: the lanes that hold it
+      const int rr = i - row0;
+      if (rr < WR && g == ((rr >> 2) & 3)) {
+        const int qr = 4 * (rr >> 4) + (rr & 3);
+#pragma unroll
+        for (int q = 0; q < NQ; q++)
+          if (q == qr) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) L.row[buf][16 * u + li] = a[q][u];
+          }
+      }
+      if (lane < WR && lane <= rr) L.x[wave][lane] = 0.0;
+    }
+    wave_lds_sync();
+    double x[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q += 2) {
+      const double2 t = *reinterpret_cast<const double2*>(&L.x[wave][16 * (q >> 2) + 4 * g + (q & 3)]);
+      x[q] = t.x;
+      x[q + 1] = t.y;
+    }
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (u < nu) {
+        double s1 = 0.0;
+#pragma unroll
+        for (int q = 0; q < NQ; q += 2) {
+          s[u] = fma(x[q], a[q][u], s[u]);
+          s1 = fma(x[q + 1], a[q + 1][u], s1);
+        }
+        s[u] += s1;
+      }
+    double sum = group_sums(s);  // column `lane`
+    if (rdlane(sum, i) == 0.0) {
+      // squares that underflow are not a zero column
+      bool any = false;
+#pragma unroll
+      for (int q = 0; q < NQ; q++) any |= x[q] != 0.0;
+      if (__any(any) && lane == i) sum = 1e-300;
+    }
+    L.red[buf][wave][lane] = sum;
+    lds_barrier();
+    double rv;
+    if constexpr (GRID) {
+      // this workgroup's sums (and row i, from the one that holds it) to the
+      // others; wave w then collects workgroups w, w + NW, ... in order
+      double* sl = slots + (size_t)i * (nwg + 1) * KMAX;
+      if (wave == 0) {
+        double t = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) t += L.red[buf][w][lane];
+        st_dev(sl + wg * KMAX + lane, rp_publishable(t));
+        if (wg == 0) st_dev(sl + nwg * KMAX + lane, rp_publishable(L.row[buf][lane]));
+      }
+      double t = 0.0, rr = 0.0;
+      bool got = true;
+      for (int b = wave; b < nwg; b += NW) {
+        double v = 0.0;
+        got &= rp_await(sl + b * KMAX + lane, v);
+        t += v;
+      }
+      if (wave == NW - 1) got &= rp_await(sl + nwg * KMAX + lane, rr);
+      if (__any(!got)) {
+        // given up: the call fails
+        if (lane == 0) atomicOr(&st->flags, 8);
+        t = __longlong_as_double(0x7ff8000000000000ll);
+      }
+      lds_barrier();  // the partial sums of this buffer are read
+      L.red[buf][wave][lane] = t;
+      if (wave == NW - 1) L.row[buf][lane] = rr;
+      lds_barrier();
+    }
+    rv = L.row[buf][lane];
+    sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) sum += L.red[buf][w][lane];
+    // dlarfg: every wave computes the same
+    const double si = rdlane(sum, i), alpha = rdlane(rv, i);
+    const double t2 = fma(alpha, alpha, si);
+    if (si != 0.0 && !(si >= 1e-280 && t2 <= 1e280)) {
+      ok = false;
+      break;
+    }
+    // (a column of one row is not tested: dlarfg_mia returns before the test)
+    if (truncate && (i > 0 || cont) && msub - i > 1 && si < thr2) {
+      k = i;
+      break;
+    }
+    double taui = 0.0, beta = alpha, sc = 1.0;
+    if (si != 0.0) {
+      const double y = rsqrt_nr(t2);
+      double b = t2 * y;
+      b = fma(fma(-b, b, t2), 0.5 * y, b);
+      taui = fma(fabs(alpha), y, 1.0);  // (beta - alpha) / beta
+      const double d = fabs(alpha) + b;
+      double e = __builtin_amdgcn_rcp(d);
+      e = fma(e, fma(-d, e, 1.0), e);
+      e = fma(e, fma(-d, e, 1.0), e);
+      sc = alpha >= 0 ? e : -e;  // 1 / (alpha - beta)
+      beta = alpha >= 0 ? -b : b;
+    }
+    if (i == 0 && tau_dm > 0.0 && fjb > 1 && !cont) thr2 = (tau_dm * beta) * (tau_dm * beta);
+    const double vc = fma(sc, sum, rv);  // c > i: v^T (column c); c < i: (V^T V)(c, i)
+    const double w = taui * vc;
+    if (wg == 0) {
+      if (wave == 0) {
+        L.out[i][lane] = lane < i ? rv : (lane == i ? beta : rv - w);
+        if (lane == 0) L.tau[i] = taui;
+      } else if (wave == 1) {
+        if (lane < i) L.S[lane][i] = vc;
+      }
+    }
+    double f[4];
+    group_values(lane > i ? -w * sc : (lane == i ? sc : 0.0), f);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (u >= ui && u < nu) {
+        if (u == ui && li == ii) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) a[q][u] = 0.0;  // becomes v = sc x
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; q++) a[q][u] = fma(x[q], f[u], a[q][u]);
+      }
+  }
+  lds_barrier();
+  if (!ok) return -1;
+  // the rows below the top k: V left of column k, updated columns right of it
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      const int r = row0 + 16 * (q >> 2) + 4 * g + (q & 3), c = 16 * u + li;
+      if (r >= k && r < msub) {
+        if (c < fjb) P[(size_t)c * lda + r] = a[q][u];
+        V[(size_t)c * ldv + r] = c < k ? a[q][u] : 0.0;
+      }
+    }
+  if (wg != 0) return k;
+  const int tid2 = local_tid();
+  for (int e = tid2; e < KMAX * KMAX; e += 64 * NW) {
+    const int r = e & 63, c = e >> 6;
+    if (r < k) {
+      const double v = L.out[r][c];
+      if (c < fjb) P[(size_t)c * lda + r] = v;
+      V[(size_t)c * ldv + r] = c < k ? (r > c ? v : (r == c ? 1.0 : 0.0)) : 0.0;
+    }
+    if (r < z0) V[(size_t)c * ldv + r - z0] = 0.0;
+    // T^-1 (a column with tau = 0 is no reflector: an identity row and column)
+    const bool on = r < k && c < k && L.tau[r] != 0.0 && L.tau[c] != 0.0;
+    const double sv = on ? (r < c ? L.S[r][c] : (r == c ? 1.0 / L.tau[r] : 0.0))
+                         : (r == c ? 1.0 : 0.0);
+    L.X[r][c] = sv;
+  }
+  if (tid2 < k) tau[tid2] = L.tau[tid2];
+  lds_barrier();  // every S is read
+  lu_inverse<false>(L.X, L.S, L.rinv, L.Y);
+  for (int e = tid2; e < KMAX * KMAX; e += 64 * NW) {
+    const int r = e & 63, c = e >> 6;
+    const bool on = r <= c && c < k && L.tau[r] != 0.0 && L.tau[c] != 0.0;
+    T_out[r + c * KMAX] = on ? L.S[r][c] : 0.0;
+  }
+  return k;
+}
+
+// Panels (RUN_ALWAYS: host j, fjb, the first V buffer; RUN_EXACT: j and fjb
+// from st, tau indexed from column 0, V of the step's parity).  The dense V,
+// T and the slots lie in the workspace behind st (ws_v, ws_mat, ws_slots).
+// truncate = 2: the panel continues a wider block (wide.hip), whose first
+// pivot st->pan_beta bounds every column, the first included.  A declined
+// panel sets DevState::flags bit 2 for k_panel_slow, queued behind.
+template <int QH, int NW, bool GRID>
+__global__ __launch_bounds__(64 * NW) void k_panel_reg(double* A, int lda, int j, int m, int fjb,
+                                                       double tau_dm, int truncate, double* tau,
+                                                       DevState* st, int mode) {
+  __shared__ RegPanelLds<QH, NW> L;
+  if (!step_runs(st, mode)) return;
+  const int ldv = ws_ldv(m);
+  double* V = ws_v(st, m);
+  if (mode != RUN_ALWAYS) {
+    j = st->j;
+    fjb = st->fjb;
+    tau += j;
+    if (st->fused) V += (size_t)(st->it & 1) * ldv * KMAX;
+  }
+  const int msub = m - j;
+  const int nwg = GRID ? (msub + 16 * QH * NW - 1) / (16 * QH * NW) : 1;
+  const int wg = blockIdx.x;
+  if (wg >= nwg) return;  // the grid is sized for the lowest j
+  const double beta0 = truncate == 2 ? st->pan_beta : 0.0;
+  const int k = reg_panel<QH, NW, GRID>(A + j + (size_t)j * lda, lda, msub, fjb, tau_dm, truncate,
+                                        beta0, tau, V + j, ldv, min(j, KMAX), ws_mat(st, WS_T),
+                                        ws_slots(st), nwg, wg, st, L);
+  if (wg == 0 && threadIdx.x == 0) {
+    if (k < 0) {
+      atomicOr(&st->flags, 4);
+    } else {
+      if (truncate != 2) st->pan_beta = L.out[0][0];
+      st->fjb_cmp = k;
+      // the rejected columns j + k .. j + fjb are already updated (as dlarf_
+      // does inside the reference's panel); the trailing update starts after
+      st->c0 = j + fjb;
+    }
+  }
+}
+
+// The panel in memory, column by column (panel_exact_body: norms with
+// dnrm2's scaling, any number of rows), then V and T, by one workgroup: runs
+// when the register-held form declined (flags bit 2), or with force.
+__global__ __launch_bounds__(1024) void k_panel_slow(double* A, int lda, int j, int m, int fjb,
+                                                     double tau_dm, int truncate, double* tau,
+                                                     DevState* st, int mode, int force) {
+  __shared__ double Ss[KMAX * KMAX];
+  __shared__ double Ts[KMAX * KMAX];
+  __shared__ double tmp[KMAX], ts[KMAX], red[16];
+  if (!step_runs(st, mode) || !(force || (st->flags & 4))) return;
+  const int ldv = ws_ldv(m);
+  double* V = ws_v(st, m);
+  if (mode != RUN_ALWAYS) {
+    j = st->j;
+    fjb = st->fjb;
+    tau += j;
+    if (st->fused) V += (size_t)(st->it & 1) * ldv * KMAX;
+  }
+  const double beta0 = truncate == 2 ? st->pan_beta : 0.0;
+  const int k = panel_exact_body<1>(A, lda, j, m, fjb, tau_dm, truncate, tau, red, beta0);
+  __syncthreads();
+  const int tid = local_tid(), lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
+  for (int c = wave; c < KMAX; c += 16)
+    for (int r = max(j - KMAX, 0) + lane; r < m; r += 64)
+      V[(size_t)c * ldv + r] = (c >= k || r < j + c) ? 0.0
+                               : (r == j + c ? 1.0 : A[(size_t)(j + c) * lda + r]);
+  for (int e = tid; e < KMAX * KMAX; e += 1024) Ss[e] = Ts[e] = 0.0;
+  if (tid < KMAX) ts[tid] = tid < k ? tau[tid] : 0.0;
+  __syncthreads();
+  // S = V^T V: wave w takes the 16-row blocks w, w + 16, ...; summed in wave order
+  dbl4 gt[10];
+#pragma unroll
+  for (int p = 0; p < 10; p++) gt[p] = (dbl4){0.0, 0.0, 0.0, 0.0};
+  for (int rb = j + 16 * wave; rb < m; rb += 256) {
+    dbl4 xb[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int r = rb + g + 4 * v;
+        xb[u][v] = r < m ? V[(size_t)(16 * u + li) * ldv + r] : 0.0;
+      }
+    gram_tiles(xb, gt);
+  }
+  for (int w = 0; w < 16; w++) {
+    if (wave == w) {
+      int p = 0;
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int u2 = u; u2 < 4; u2++) {
+#pragma unroll
+          for (int v = 0; v < 4; v++) Ss[(16 * u + g + 4 * v) + (16 * u2 + li) * KMAX] += gt[p][v];
+          p++;
+        }
+    }
+    __syncthreads();
+  }
+  larft_recurrence(Ss, Ts, ts, tmp, k);
+  for (int e = tid; e < KMAX * KMAX; e += 1024) ws_mat(st, WS_T)[e] = Ts[e];
+  if (tid == 0) {
+    if (truncate != 2) st->pan_beta = A[(size_t)j * lda + j];
+    st->fjb_cmp = k;
+    st->c0 = j + fjb;
+    st->flags &= ~4;
+  }
+}
+
+// Every slot of a panel by nwg workgroups empty (see kRpEmpty).
+__global__ __launch_bounds__(256) void k_panel_slots(DevState* st, int n, int mode) {
+  if (!step_runs(st, mode)) return;
+  unsigned long long* s = reinterpret_cast<unsigned long long*>(ws_slots(st));
+  for (int e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) s[e] = kRpEmpty;
+}
+
+// The form by the panel's rows (m - j, j the lowest the step can have): up to
+// RP_SMALL rows four waves of 32 rows, up to RP_MID eight of 48, up to RP_ROWS
+// eight of 64 in one workgroup, then RP_ROWS rows per workgroup, all of which
+// have to be resident together: at most RP_WGS of the 256 CUs.  Larger ones
+// stay in memory.
+void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm,
+                        int truncate, double* tau, DevState* st, hipStream_t s, int mode) {
+  const int rows = m - j, nwg = (rows + RP_ROWS - 1) / RP_ROWS;
+  if (rows <= RP_SMALL) {
+    hipLaunchKernelGGL((k_panel_reg<2, 4, false>), dim3(1), dim3(256), 0, s, A, lda, j, m, fjb,
+                       tau_dm, truncate, tau, st, mode);
+  } else if (rows <= RP_MID) {
+    hipLaunchKernelGGL((k_panel_reg<3, 8, false>), dim3(1), dim3(512), 0, s, A, lda, j, m, fjb,
+                       tau_dm, truncate, tau, st, mode);
+  } else if (nwg == 1) {
+    hipLaunchKernelGGL((k_panel_reg<4, 8, false>), dim3(1), dim3(512), 0, s, A, lda, j, m, fjb,
+                       tau_dm, truncate, tau, st, mode);
+  } else if (nwg <= RP_WGS) {
+    hipLaunchKernelGGL(k_panel_slots, dim3(8 * (nwg + 1)), dim3(256), 0, s, st,
+                       KMAX * KMAX * (nwg + 1), mode);
+    hipLaunchKernelGGL((k_panel_reg<4, 8, true>), dim3(nwg), dim3(512), 0, s, A, lda, j, m, fjb,
+                       tau_dm, truncate, tau, st, mode);
+  }
+  hipLaunchKernelGGL(k_panel_slow, dim3(1), dim3(1024), 0, s, A, lda, j, m, fjb, tau_dm,
+                     truncate, tau, st, mode, nwg > RP_WGS ? 1 : 0);
+}
+
+}  // namespace qrdm
