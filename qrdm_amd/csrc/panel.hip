@@ -362,20 +362,13 @@ __device__ __forceinline__ int lu_signed_blocked(double (*W)[LDP], int nlim, con
   return nlim;
 }
 
-// X := L^-1 and U^-1 of the pair held in one 64 x 64 matrix W (L unit lower
-// triangular strictly below the diagonal, U upper triangular on and above
-// it, non-zero diagonal), X in the same layout: L^-1 strictly below the
-// diagonal (its unit diagonal implied), U^-1 on and above; at least 256
-// threads (the first four waves compute), ends with a barrier.  BOTH = false: U^-1 only (W's lower part is not read, X's
-// is set to zero).  Both go by 16 x 16 blocks, L^-1 as (L^T)^-1 read and
-// stored transposed: the diagonal blocks by back substitution (wave w takes
-// block w of both, one lane per column: lanes 0-15 U, 16-31 L^T), then the
-// blocks at block distance d = 1, 2, 3 on the matrix cores, one block per
-// wave: X_ij = -X_ii Y with Y = sum_{k = i+1..j} R_ik X_kj (R = U or L^T).
-// Ys: one 16 x 16 scratch tile per wave.
-template <bool BOTH = true>
-__device__ __forceinline__ void lu_inverse(const double (*W)[LDP], double (*X)[LDP], double* rinv,
-                                           double (*Ys)[BLK][BLK + 1]) {
+// The off-diagonal blocks of lu_inverse's X from its diagonal blocks: block
+// distance d = 1, 2, 3 on the matrix cores, one block per wave (the first four
+// waves): X_ij = -X_ii Y with Y = sum_{k = i+1..j} R_ik X_kj (R = U or L^T).
+// Ys: one 16 x 16 scratch tile per wave.  Ends with a barrier.
+template <bool BOTH>
+__device__ __forceinline__ void inverse_merge(const double (*W)[LDP], double (*X)[LDP],
+                                              double (*Ys)[BLK][BLK + 1]) {
   const int tid = local_tid(), lane = tid & 63, wave = tid >> 6;
   // R_m(i, l): m = 1 U, m = 0 L^T (unit diagonal); zero below the diagonal
   auto Rm = [&](int m, int i, int l) -> double {
@@ -385,31 +378,6 @@ __device__ __forceinline__ void lu_inverse(const double (*W)[LDP], double (*X)[L
   auto Xm = [&](int m, int i, int j) -> double {
     return m ? ((i <= j) ? X[i][j] : 0.0) : ((i < j) ? X[j][i] : (i == j ? 1.0 : 0.0));
   };
-  if (tid < KMAX) rinv[tid] = 1.0 / W[tid][tid];
-  if (!BOTH) {
-    for (int e = tid; e < KMAX * KMAX; e += NT1) {
-      const int r = e & 63, c = e >> 6;
-      if (r > c) X[r][c] = 0.0;
-    }
-  }
-  lds_barrier();
-  if (wave < 4 && lane < (BOTH ? 32 : 16)) {
-    const int m = (lane < 16) ? 1 : 0, c = lane & 15, base = BLK * wave;
-    double x[BLK];
-#pragma unroll
-    for (int i = BLK - 1; i >= 0; i--) {
-      double sacc = (i == c) ? 1.0 : 0.0;
-#pragma unroll
-      for (int l = i + 1; l < BLK; l++) sacc = fma(-Rm(m, base + i, base + l), x[l], sacc);
-      x[i] = m ? sacc * rinv[base + i] : sacc;
-    }
-#pragma unroll
-    for (int i = 0; i < BLK; i++) {
-      if (m && i <= c) X[base + i][base + c] = x[i];
-      if (!m && i < c) X[base + c][base + i] = x[i];
-    }
-  }
-  lds_barrier();
   const int g = lane >> 4, li = lane & 15;
   for (int d = 1; d < 4; d++) {
     const int ntgt = (BOTH ? 2 : 1) * (4 - d);
@@ -445,6 +413,51 @@ __device__ __forceinline__ void lu_inverse(const double (*W)[LDP], double (*X)[L
     }
     lds_barrier();
   }
+}
+
+// X := L^-1 and U^-1 of the pair held in one 64 x 64 matrix W (L unit lower
+// triangular strictly below the diagonal, U upper triangular on and above
+// it, non-zero diagonal), X in the same layout: L^-1 strictly below the
+// diagonal (its unit diagonal implied), U^-1 on and above; at least 256
+// threads (the first four waves compute), ends with a barrier.  BOTH = false: U^-1 only (W's lower part is not read, X's
+// is set to zero).  Both go by 16 x 16 blocks, L^-1 as (L^T)^-1 read and
+// stored transposed: the diagonal blocks by back substitution (wave w takes
+// block w of both, one lane per column: lanes 0-15 U, 16-31 L^T), then the
+// others (inverse_merge; Ys is its scratch).
+template <bool BOTH = true>
+__device__ __forceinline__ void lu_inverse(const double (*W)[LDP], double (*X)[LDP], double* rinv,
+                                           double (*Ys)[BLK][BLK + 1]) {
+  const int tid = local_tid(), lane = tid & 63, wave = tid >> 6;
+  // R_m(i, l): m = 1 U, m = 0 L^T (unit diagonal); zero below the diagonal
+  auto Rm = [&](int m, int i, int l) -> double {
+    return m ? ((i <= l) ? W[i][l] : 0.0) : ((i < l) ? W[l][i] : (i == l ? 1.0 : 0.0));
+  };
+  if (tid < KMAX) rinv[tid] = 1.0 / W[tid][tid];
+  if (!BOTH) {
+    for (int e = tid; e < KMAX * KMAX; e += NT1) {
+      const int r = e & 63, c = e >> 6;
+      if (r > c) X[r][c] = 0.0;
+    }
+  }
+  lds_barrier();
+  if (wave < 4 && lane < (BOTH ? 32 : 16)) {
+    const int m = (lane < 16) ? 1 : 0, c = lane & 15, base = BLK * wave;
+    double x[BLK];
+#pragma unroll
+    for (int i = BLK - 1; i >= 0; i--) {
+      double sacc = (i == c) ? 1.0 : 0.0;
+#pragma unroll
+      for (int l = i + 1; l < BLK; l++) sacc = fma(-Rm(m, base + i, base + l), x[l], sacc);
+      x[i] = m ? sacc * rinv[base + i] : sacc;
+    }
+#pragma unroll
+    for (int i = 0; i < BLK; i++) {
+      if (m && i <= c) X[base + i][base + c] = x[i];
+      if (!m && i < c) X[base + c][base + i] = x[i];
+    }
+  }
+  lds_barrier();
+  inverse_merge<BOTH>(W, X, Ys);
 }
 
 // ---------------------------------------------------------------------------

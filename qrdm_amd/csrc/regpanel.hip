@@ -16,14 +16,20 @@
 //
 // Row i leaves the registers when column i is done (R to the right of the
 // diagonal, V to the left), through LDS; the rest is written once, at the end,
-// with the dense V and T = (striu(V^T V) + diag(1 / tau))^-1 of the trailing
-// update.  Panels of more than RP_ROWS rows take one workgroup per RP_ROWS
+// with the dense V of the trailing update.  One wave that holds no rows builds
+// T's diagonal blocks from those entries beside the others' updates.  Panels of more than RP_ROWS rows take one workgroup per RP_ROWS
 // rows: every column's partial sums pass between the workgroups through
 // memory, each a slot of its own that holds a sentinel until it is written.
 //
-// Measured against the memory-based panel: unpivoted QR of 1024 x 1024 15.6 ->
-// 3.6 ms, of 4096 x 2048 129 -> 10.1 ms; 2048 x 1024 DM with 128-column blocks
-// 68.3 -> 9.6 ms; 64 x 48 DM 0.53 -> 0.33 ms.
+// Measured for 64 columns, with V and T (rocprofv3): up to 128 rows 66 us, up
+// to 448 rows 106 us (memory-based: about 180 us for 64 rows, with T another
+// 60), 4096 rows on ten workgroups 189 us (3.8 ms).  A column costs about 2500
+// cycles at 128 rows and 3600 at 448, of which the reflector's scalars take 280;
+// between workgroups the exchange adds 3600.  The loop is unrolled over the
+// four column groups so that every register index is static: with uniform
+// branches in their place the 448-row panel took 163 us.  Unpivoted QR of 1024 x
+// 1024 15.6 -> 2.9 ms, of 4096 x 2048 129 -> 8.5 ms; 2048 x 1024 DM with
+// 128-column blocks 68.4 -> 8.8 ms; 64 x 48 DM 0.53 -> 0.33 ms.
 //
 // Sums of squares are taken plainly: where one leaves [1e-280, 1e280] (or is
 // not a number) the panel is declined before anything is written, and the
@@ -32,9 +38,9 @@
 
 namespace qrdm {
 
-constexpr int RP_ROWS = 512;  // rows per workgroup (eight waves of 64)
+constexpr int RP_ROWS = 448;  // rows per workgroup (seven waves of 64, and the one for T)
 constexpr int RP_SMALL = 128;  // panels up to this many rows: four waves of 32
-constexpr int RP_MID = 384;    // up to this many: eight waves of 48
+constexpr int RP_MID = 336;    // up to this many: seven waves of 48
 constexpr int RP_WGS = 64;     // workgroups of one panel at most
 
 // A slot not yet written: a NaN pattern no published value takes (published
@@ -43,16 +49,20 @@ __device__ constexpr unsigned long long kRpEmpty = 0x7ff4a5a5c3c30f0full;
 // Polls of one slot before a workgroup gives the panel up (about seconds).
 constexpr int RP_POLLS = 1 << 22;
 
+// Two doubles at any multiple of eight bytes.
+typedef double rp_pair __attribute__((ext_vector_type(2), aligned(8)));
+
+// QH: 16-row groups per data wave; NW: data waves.  One more wave builds T.
 template <int QH, int NW>
 struct RegPanelLds {
-  double x[NW][16 * QH];    // column i's rows, per wave
-  double red[2][NW][KMAX];  // the waves' partial sums, by column
-  double row[2][KMAX];      // row i
-  double out[KMAX][LDP];    // the top block: R, V below the diagonal
-  double S[KMAX][LDP];      // V^T V above the diagonal
-  double X[KMAX][LDP];      // T
+  double x[NW][16 * QH];        // column i's rows, per wave
+  double red[2][NW + 1][KMAX];  // partial sums, by column
+  double row[2][KMAX];          // row i
+  double out[KMAX][LDP];        // the top block: R, V below the diagonal
+  double S[KMAX][LDP];          // V^T V above the diagonal, else zero
+  double X[KMAX][LDP];          // T
   double Y[4][BLK][BLK + 1];
-  double rinv[KMAX], tau[KMAX];
+  double tau[KMAX];
 };
 
 // (lane 16 g + li) := the sum over the four lane groups of s[g], column 16 g + li.
@@ -98,18 +108,45 @@ __device__ __forceinline__ double rp_publishable(double v) {
   return v == v ? v : __longlong_as_double(0x7ff8000000000000ll);
 }
 
-// Waits for the slot; false when it stayed empty for RP_POLLS polls.
-__device__ __forceinline__ bool rp_await(const double* slot, double& v) {
-  for (int t = 0; t < RP_POLLS; t++) {
-    const unsigned long long b =
-        __hip_atomic_load(reinterpret_cast<const unsigned long long*>(slot), __ATOMIC_RELAXED,
-                          __HIP_MEMORY_SCOPE_AGENT);
-    if (b != kRpEmpty) {
-      v = __longlong_as_double((long long)b);
-      return true;
+// Whether any of the n values is not zero (a wave).
+__device__ __forceinline__ bool rp_nonzero(const double* v, int n) {
+  bool any = false;
+  for (int e = local_tid() & 63; e < n; e += 64) any |= v[e] != 0.0;
+  return __any(any) != 0;
+}
+
+// v := the sum, in order, of the slots first, first + step, ... < n (each of
+// KMAX values, this lane's); false when one stayed empty for RP_POLLS polls.
+// The slots' loads are in flight together.
+__device__ __forceinline__ bool rp_collect(const double* slots, int first, int step, int n,
+                                           double& v) {
+  constexpr int BATCH = 4;
+  const int lane = local_tid() & 63;
+  v = 0.0;
+  for (int b0 = first; b0 < n; b0 += BATCH * step) {
+    unsigned long long w[BATCH];
+    int polls = 0;
+    for (;;) {
+      bool empty = false;
+#pragma unroll
+      for (int q = 0; q < BATCH; q++) {
+        const int b = b0 + q * step;
+        w[q] = 0ull;
+        if (b < n)
+          w[q] = __hip_atomic_load(
+              reinterpret_cast<const unsigned long long*>(slots) + b * KMAX + lane,
+              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for (int q = 0; q < BATCH; q++) empty |= w[q] == kRpEmpty;
+      if (!__any(empty)) break;
+      if (++polls == RP_POLLS) return false;
     }
+#pragma unroll
+    for (int q = 0; q < BATCH; q++)
+      if (b0 + q * step < n) v += __longlong_as_double((long long)w[q]);
   }
-  return false;
+  return true;
 }
 
 // The panel's columns [0, fjb) at P (leading dimension lda, msub rows) by nwg
@@ -118,174 +155,235 @@ __device__ __forceinline__ bool rp_await(const double* slot, double& v) {
 // column 0 is done), unless truncate is 0; truncate = 2: beta0 is the block's
 // R(0, 0), and every column is tested.  slots (nwg > 1): KMAX columns x
 // (nwg + 1) x KMAX values, empty on entry.  Returns the columns reduced with
-// everything written -- the panel, tau, rows [-KMAX, msub) of the dense V
-// (zero above the panel, where z0 rows exist) and T -- or -1, declined, with
-// nothing written.  Every workgroup returns the same (one that gives up
-// waiting sets flags bit 3, which fails the call).
+// everything written -- the panel, tau, rows [-z0, msub) of the dense V (zero
+// above the panel) and T -- or -1, declined, with nothing written.  Every
+// workgroup returns the same (one that gives up waiting sets flags bit 3,
+// which fails the call).
 template <int QH, int NW, bool GRID>
 __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, double tau_dm,
                                          int truncate, double beta0, double* tau, double* V,
                                          int ldv, int z0, double* T_out, double* slots, int nwg,
                                          int wg, DevState* st, RegPanelLds<QH, NW>& L) {
-  constexpr int WR = 16 * QH, NQ = 4 * QH;
+  constexpr int WR = 16 * QH, NQ = 4 * QH, NT = 64 * (NW + 1);
   const int tid = local_tid(), lane = tid & 63, g = lane >> 4, li = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int row0 = wg * WR * NW + wave * WR;  // this wave's first row
-  const int nu = (fjb + 15) >> 4;
+  const bool data = wave < NW;  // the last wave builds T
+  const int row0 = data ? wg * WR * NW + wave * WR : 0;  // this wave's first row
   // the lane's rows: row0 + 16 (q / 4) + 4 g + q % 4
-  double a[NQ][4];
+  double a[4][NQ];
 #pragma unroll
   for (int u = 0; u < 4; u++)
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int r = row0 + 16 * (q >> 2) + 4 * g + (q & 3), c = 16 * u + li;
-      a[q][u] = (r < msub && c < fjb) ? P[(size_t)c * lda + r] : 0.0;
+    for (int h = 0; h < QH; h++) {
+      const int r = row0 + 16 * h + 4 * g, c = 16 * u + li;
+      const double* p = P + (size_t)c * lda + r;
+      rp_pair lo = {0.0, 0.0}, hi = {0.0, 0.0};
+      if (data && c < fjb) {
+        if (r + 3 < msub) {
+          lo = *reinterpret_cast<const rp_pair*>(p);
+          hi = *reinterpret_cast<const rp_pair*>(p + 2);
+        } else {
+          if (r < msub) lo.x = p[0];
+          if (r + 1 < msub) lo.y = p[1];
+          if (r + 2 < msub) hi.x = p[2];
+        }
+      }
+      a[u][4 * h] = lo.x;
+      a[u][4 * h + 1] = lo.y;
+      a[u][4 * h + 2] = hi.x;
+      a[u][4 * h + 3] = hi.y;
     }
-  const bool cont = truncate == 2;
-  const double thr0 = cont && tau_dm > 0.0 ? tau_dm * beta0 : 5e-14;
-  double thr2 = thr0 * thr0;
-  int k = fjb;
-  bool ok = true;
-  for (int i = 0; i < fjb; i++) {
-    const int buf = i & 1, ui = i >> 4, ii = i & 15;
-    // column i: its owner lanes' rows to every lane of the wave, zero on and
-    // above the diagonal
+  // column 16 u + ii to LDS: its owner lanes' rows, zero on and above the diagonal
+  auto put_column = [&](int u, int ii) {
     if (li == ii) {
 #pragma unroll
-      for (int u = 0; u < 4; u++)
-        if (u == ui) {
-#pragma unroll
-          for (int q = 0; q < NQ; q += 2)
-            *reinterpret_cast<double2*>(&L.x[wave][16 * (q >> 2) + 4 * g + (q & 3)]) =
-                make_double2(a[q][u], a[q + 1][u]);
-        }
+      for (int q = 0; q < NQ; q += 2)
+        *reinterpret_cast<double2*>(&L.x[wave][16 * (q >> 2) + 4 * g + (q & 3)]) =
+            make_double2(a[u][q], a[u][q + 1]);
     }
-    if (row0 <= i) {
-      // row i, before its step: the lanes that hold it
-      const int rr = i - row0;
-      if (rr < WR && g == ((rr >> 2) & 3)) {
-        const int qr = 4 * (rr >> 4) + (rr & 3);
+    if (wg == 0 && wave <= u / QH && lane < WR && lane <= 16 * u + ii - row0)
+      L.x[wave][lane] = 0.0;
+  };
+  // row 16 ur + ii, before its step, from the lanes that hold it
+  auto put_row = [&](int ur, int ii) {
+    if (wg != 0 || wave != ur / QH) return;
+    const int h = 4 * (ur % QH), ql = ii & 3;
 #pragma unroll
-        for (int q = 0; q < NQ; q++)
-          if (q == qr) {
-#pragma unroll
-            for (int u = 0; u < 4; u++) L.row[buf][16 * u + li] = a[q][u];
-          }
-      }
-      if (lane < WR && lane <= rr) L.x[wave][lane] = 0.0;
+    for (int u = 0; u < 4; u++) {
+      const double lo = ql & 1 ? a[u][h + 1] : a[u][h], hi = ql & 1 ? a[u][h + 3] : a[u][h + 2];
+      if (g == ii >> 2) L.row[ii & 1][16 * u + li] = ql & 2 ? hi : lo;
     }
-    wave_lds_sync();
-    double x[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; q += 2) {
-      const double2 t = *reinterpret_cast<const double2*>(&L.x[wave][16 * (q >> 2) + 4 * g + (q & 3)]);
-      x[q] = t.x;
-      x[q + 1] = t.y;
-    }
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-      if (u < nu) {
-        double s1 = 0.0;
-#pragma unroll
-        for (int q = 0; q < NQ; q += 2) {
-          s[u] = fma(x[q], a[q][u], s[u]);
-          s1 = fma(x[q + 1], a[q + 1][u], s1);
-        }
-        s[u] += s1;
-      }
-    double sum = group_sums(s);  // column `lane`
-    if (rdlane(sum, i) == 0.0) {
-      // squares that underflow are not a zero column
-      bool any = false;
-#pragma unroll
-      for (int q = 0; q < NQ; q++) any |= x[q] != 0.0;
-      if (__any(any) && lane == i) sum = 1e-300;
-    }
-    L.red[buf][wave][lane] = sum;
+  };
+  const bool cont = truncate == 2;
+  const double thr0 = cont && tau_dm > 0.0 ? tau_dm * beta0 : 5e-14;
+  double thr2 = truncate && cont ? thr0 * thr0 : -1.0;  // nothing is below -1
+  int k = fjb;
+  bool ok = true;
+  // After the data waves' partial sums of column i: sum := x^T (column lane),
+  // rv := row i's entry there.
+  auto exchange = [&](int i, double& sum, double& rv) {
+    const int buf = i & 1;
     lds_barrier();
-    double rv;
     if constexpr (GRID) {
       // this workgroup's sums (and row i, from the one that holds it) to the
-      // others; wave w then collects workgroups w, w + NW, ... in order
+      // others; wave w then collects workgroups w, w + NW + 1, ... in order
       double* sl = slots + (size_t)i * (nwg + 1) * KMAX;
       if (wave == 0) {
-        double t = 0.0;
+        double t = L.red[buf][0][lane];
 #pragma unroll
-        for (int w = 0; w < NW; w++) t += L.red[buf][w][lane];
+        for (int w = 1; w < NW; w++) t += L.red[buf][w][lane];
+        if (rdlane(t, i) == 0.0 && rp_nonzero(&L.x[0][0], NW * WR) && lane == i) t = 1e-300;
         st_dev(sl + wg * KMAX + lane, rp_publishable(t));
-        if (wg == 0) st_dev(sl + nwg * KMAX + lane, rp_publishable(L.row[buf][lane]));
       }
+      if (wg == 0 && wave == 1) st_dev(sl + nwg * KMAX + lane, rp_publishable(L.row[buf][lane]));
       double t = 0.0, rr = 0.0;
-      bool got = true;
-      for (int b = wave; b < nwg; b += NW) {
-        double v = 0.0;
-        got &= rp_await(sl + b * KMAX + lane, v);
-        t += v;
-      }
-      if (wave == NW - 1) got &= rp_await(sl + nwg * KMAX + lane, rr);
-      if (__any(!got)) {
-        // given up: the call fails
-        if (lane == 0) atomicOr(&st->flags, 8);
+      bool got = rp_collect(sl, wave, NW + 1, nwg, t);
+      if (wave == NW) got &= rp_collect(sl, nwg, 1, nwg + 1, rr);
+      if (!got) {
+        if (lane == 0) atomicOr(&st->flags, 8);  // given up: the call fails
         t = __longlong_as_double(0x7ff8000000000000ll);
       }
       lds_barrier();  // the partial sums of this buffer are read
       L.red[buf][wave][lane] = t;
-      if (wave == NW - 1) L.row[buf][lane] = rr;
+      if (wave == NW) L.row[buf][lane] = rr;
       lds_barrier();
     }
     rv = L.row[buf][lane];
-    sum = 0.0;
+    sum = L.red[buf][0][lane];
 #pragma unroll
-    for (int w = 0; w < NW; w++) sum += L.red[buf][w][lane];
-    // dlarfg: every wave computes the same
+    for (int w = 1; w < (GRID ? NW + 1 : NW); w++) sum += L.red[buf][w][lane];
+  };
+  // dlarfg of column i (every wave computes the same): tau, beta, 1 / (alpha -
+  // beta); false ends the panel before column i.  y = 1 / sqrt(t2) by one
+  // third-order step from the hardware's estimate; the reciprocal of alpha -
+  // beta likewise, its estimate taken beside y's step.
+  auto reflect = [&](int i, double sum, double rv, double& taui, double& beta, double& sc) {
     const double si = rdlane(sum, i), alpha = rdlane(rv, i);
-    const double t2 = fma(alpha, alpha, si);
-    if (si != 0.0 && !(si >= 1e-280 && t2 <= 1e280)) {
-      ok = false;
-      break;
-    }
-    // (a column of one row is not tested: dlarfg_mia returns before the test)
-    if (truncate && (i > 0 || cont) && msub - i > 1 && si < thr2) {
-      k = i;
-      break;
-    }
-    double taui = 0.0, beta = alpha, sc = 1.0;
-    if (si != 0.0) {
-      const double y = rsqrt_nr(t2);
+    const double aa = fabs(alpha), t2 = fma(alpha, alpha, si);
+    if (si >= 1e-280 && t2 <= 1e280 && si >= thr2) {
+      double y = __builtin_amdgcn_rsq(t2);
+      double e = __builtin_amdgcn_rcp(fma(t2, y, aa));
+      const double h = fma(-t2 * y, y, 1.0);
+      y = fma(y * h, fma(0.375, h, 0.5), y);
       double b = t2 * y;
       b = fma(fma(-b, b, t2), 0.5 * y, b);
-      taui = fma(fabs(alpha), y, 1.0);  // (beta - alpha) / beta
-      const double d = fabs(alpha) + b;
-      double e = __builtin_amdgcn_rcp(d);
-      e = fma(e, fma(-d, e, 1.0), e);
-      e = fma(e, fma(-d, e, 1.0), e);
-      sc = alpha >= 0 ? e : -e;  // 1 / (alpha - beta)
+      taui = fma(aa, y, 1.0);  // (beta - alpha) / beta
+      const double r = fma(-(aa + b), e, 1.0);
+      e = fma(fma(r, r, r), e, e);
+      sc = alpha >= 0 ? e : -e;
       beta = alpha >= 0 ? -b : b;
-    }
-    if (i == 0 && tau_dm > 0.0 && fjb > 1 && !cont) thr2 = (tau_dm * beta) * (tau_dm * beta);
-    const double vc = fma(sc, sum, rv);  // c > i: v^T (column c); c < i: (V^T V)(c, i)
-    const double w = taui * vc;
-    if (wg == 0) {
-      if (wave == 0) {
-        L.out[i][lane] = lane < i ? rv : (lane == i ? beta : rv - w);
-        if (lane == 0) L.tau[i] = taui;
-      } else if (wave == 1) {
-        if (lane < i) L.S[lane][i] = vc;
+    } else {
+      // a zero column (tau = 0), the truncation, or out of range
+      bool zero = si == 0.0;
+      if (!GRID && zero) {
+        zero = !rp_nonzero(&L.x[0][0], NW * WR);
+        lds_barrier();  // every wave has looked
       }
+      if (!zero && !(si >= 1e-280 && t2 <= 1e280)) {
+        ok = false;
+        return false;
+      }
+      // (a column of one row is not tested: dlarfg_mia returns before the test)
+      if (msub - i > 1 && si < thr2) {
+        k = i;
+        return false;
+      }
+      taui = 0.0;
+      beta = alpha;
+      sc = 1.0;
     }
-    double f[4];
-    group_values(lane > i ? -w * sc : (lane == i ? sc : 0.0), f);
+    if (truncate && i == 0 && !cont) {
+      const double thr = tau_dm > 0.0 && fjb > 1 ? tau_dm * beta : thr0;
+      thr2 = thr * thr;
+    }
+    return true;
+  };
+  if (data) {
+    put_column(0, 0);
+    put_row(0, 0);
+    bool go = true;
 #pragma unroll
-    for (int u = 0; u < 4; u++)
-      if (u >= ui && u < nu) {
-        if (u == ui && li == ii) {
+    for (int ui = 0; ui < 4; ui++) {
+      for (int ii = 0; go && ii < 16 && 16 * ui + ii < fjb; ii++) {
+        const int i = 16 * ui + ii;
+        wave_lds_sync();
+        double x[NQ];
 #pragma unroll
-          for (int q = 0; q < NQ; q++) a[q][u] = 0.0;  // becomes v = sc x
+        for (int q = 0; q < NQ; q += 2) {
+          const double2 t =
+              *reinterpret_cast<const double2*>(&L.x[wave][16 * (q >> 2) + 4 * g + (q & 3)]);
+          x[q] = t.x;
+          x[q + 1] = t.y;
+        }
+        // eight independent chains
+        double s[4] = {0.0, 0.0, 0.0, 0.0}, s1[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < NQ; q += 2)
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            s[u] = fma(x[q], a[u][q], s[u]);
+            s1[u] = fma(x[q + 1], a[u][q + 1], s1[u]);
+          }
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[u] += s1[u];
+        L.red[i & 1][wave][lane] = group_sums(s);  // column `lane`
+        double sum, rv, taui, beta, sc;
+        exchange(i, sum, rv);
+        go = reflect(i, sum, rv, taui, beta, sc);
+        if (!go) break;
+        // c > i: v^T (column c); c < i: (V^T V)(c, i)
+        const double vc = fma(sc, sum, rv);
+        double f[4];
+        group_values(lane > i ? -(taui * sc) * vc : (lane == i ? sc : 0.0), f);
+        if (li == ii) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) a[ui][q] = 0.0;  // becomes v = sc x
         }
 #pragma unroll
-        for (int q = 0; q < NQ; q++) a[q][u] = fma(x[q], f[u], a[q][u]);
+        for (int u = ui; u < 4; u++) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) a[u][q] = fma(x[q], f[u], a[u][q]);
+          // the next column's way through LDS runs beside the other groups
+          if (u == ui && ii < 15) put_column(ui, ii + 1);
+          if (u == ui + 1 && ii == 15) put_column(ui + 1, 0);
+        }
+        if (ii < 15) put_row(ui, ii + 1);
+        else if (ui < 3) put_row(ui + 1, 0);
+        if (wg == 0 && wave == 0)
+          L.out[i][lane] = lane < i ? rv : (lane == i ? beta : fma(-taui, vc, rv));
       }
+    }
+  } else {
+    if (wg == 0) {
+      for (int r = 0; r < KMAX; r++) L.S[r][lane] = L.X[r][lane] = 0.0;
+    }
+    // T's 16 x 16 diagonal blocks by dlarft's recurrence, lane p its row p
+    // (z = V^T v_i by row broadcasts); the other blocks follow from them
+    double tb[BLK];
+    for (int i = 0; i < fjb; i++) {
+      const int ui = i >> 4, ii = i & 15;
+      double sum, rv, taui, beta, sc;
+      exchange(i, sum, rv);
+      if (!reflect(i, sum, rv, taui, beta, sc)) break;
+      if (wg != 0) continue;
+      const double vc = fma(sc, sum, rv);
+      if (ii == 0) {
+#pragma unroll
+        for (int t = 0; t < BLK; t++) tb[t] = 0.0;
+      }
+      double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+      for (int t = 0; t < BLK; t += 2) {
+        t0 = fma(tb[t], row_bcast(vc, t), t0);
+        t1 = fma(tb[t + 1], row_bcast(vc, t + 1), t1);
+      }
+      const double v = li < ii ? -taui * (t0 + t1) : (li == ii ? taui : 0.0);
+#pragma unroll
+      for (int t = 0; t < BLK; t++) tb[t] = t == ii ? v : tb[t];
+      if (g == ui) L.X[lane][i] = v;
+      if (lane < i) L.S[lane][i] = vc;
+      if (lane == 0) L.tau[i] = taui;
+    }
   }
   lds_barrier();
   if (!ok) return -1;
@@ -293,16 +391,33 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
 #pragma unroll
   for (int u = 0; u < 4; u++)
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int r = row0 + 16 * (q >> 2) + 4 * g + (q & 3), c = 16 * u + li;
-      if (r >= k && r < msub) {
-        if (c < fjb) P[(size_t)c * lda + r] = a[q][u];
-        V[(size_t)c * ldv + r] = c < k ? a[q][u] : 0.0;
+    for (int h = 0; h < QH; h++) {
+      const int r = row0 + 16 * h + 4 * g, c = 16 * u + li;
+      double* p = P + (size_t)c * lda + r;
+      double* pv = V + (size_t)c * ldv + r;
+      const bool in = c < fjb, on = c < k;
+      if (data && r >= k && r + 3 < msub) {
+        const rp_pair lo = {a[u][4 * h], a[u][4 * h + 1]}, hi = {a[u][4 * h + 2], a[u][4 * h + 3]};
+        const rp_pair zero = {0.0, 0.0};
+        if (in) {
+          *reinterpret_cast<rp_pair*>(p) = lo;
+          *reinterpret_cast<rp_pair*>(p + 2) = hi;
+        }
+        *reinterpret_cast<rp_pair*>(pv) = on ? lo : zero;
+        *reinterpret_cast<rp_pair*>(pv + 2) = on ? hi : zero;
+      } else if (data) {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (r + q >= k && r + q < msub) {
+            if (in) p[q] = a[u][4 * h + q];
+            pv[q] = on ? a[u][4 * h + q] : 0.0;
+          }
       }
     }
   if (wg != 0) return k;
+  inverse_merge<false>(L.S, L.X, L.Y);  // T = (striu(V^T V) + diag(1 / tau))^-1
   const int tid2 = local_tid();
-  for (int e = tid2; e < KMAX * KMAX; e += 64 * NW) {
+  for (int e = tid2; e < KMAX * KMAX; e += NT) {
     const int r = e & 63, c = e >> 6;
     if (r < k) {
       const double v = L.out[r][c];
@@ -310,20 +425,9 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
       V[(size_t)c * ldv + r] = c < k ? (r > c ? v : (r == c ? 1.0 : 0.0)) : 0.0;
     }
     if (r < z0) V[(size_t)c * ldv + r - z0] = 0.0;
-    // T^-1 (a column with tau = 0 is no reflector: an identity row and column)
-    const bool on = r < k && c < k && L.tau[r] != 0.0 && L.tau[c] != 0.0;
-    const double sv = on ? (r < c ? L.S[r][c] : (r == c ? 1.0 / L.tau[r] : 0.0))
-                         : (r == c ? 1.0 : 0.0);
-    L.X[r][c] = sv;
+    T_out[r + c * KMAX] = r <= c && c < k ? L.X[r][c] : 0.0;
   }
   if (tid2 < k) tau[tid2] = L.tau[tid2];
-  lds_barrier();  // every S is read
-  lu_inverse<false>(L.X, L.S, L.rinv, L.Y);
-  for (int e = tid2; e < KMAX * KMAX; e += 64 * NW) {
-    const int r = e & 63, c = e >> 6;
-    const bool on = r <= c && c < k && L.tau[r] != 0.0 && L.tau[c] != 0.0;
-    T_out[r + c * KMAX] = on ? L.S[r][c] : 0.0;
-  }
   return k;
 }
 
@@ -334,7 +438,7 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
 // pivot st->pan_beta bounds every column, the first included.  A declined
 // panel sets DevState::flags bit 2 for k_panel_slow, queued behind.
 template <int QH, int NW, bool GRID>
-__global__ __launch_bounds__(64 * NW) void k_panel_reg(double* A, int lda, int j, int m, int fjb,
+__global__ __launch_bounds__(64 * (NW + 1)) void k_panel_reg(double* A, int lda, int j, int m, int fjb,
                                                        double tau_dm, int truncate, double* tau,
                                                        DevState* st, int mode) {
   __shared__ RegPanelLds<QH, NW> L;
@@ -444,26 +548,26 @@ __global__ __launch_bounds__(256) void k_panel_slots(DevState* st, int n, int mo
 }
 
 // The form by the panel's rows (m - j, j the lowest the step can have): up to
-// RP_SMALL rows four waves of 32 rows, up to RP_MID eight of 48, up to RP_ROWS
-// eight of 64 in one workgroup, then RP_ROWS rows per workgroup, all of which
+// RP_SMALL rows four waves of 32 rows, up to RP_MID seven of 48, up to RP_ROWS
+// seven of 64 in one workgroup, then RP_ROWS rows per workgroup, all of which
 // have to be resident together: at most RP_WGS of the 256 CUs.  Larger ones
 // stay in memory.
 void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm,
                         int truncate, double* tau, DevState* st, hipStream_t s, int mode) {
   const int rows = m - j, nwg = (rows + RP_ROWS - 1) / RP_ROWS;
   if (rows <= RP_SMALL) {
-    hipLaunchKernelGGL((k_panel_reg<2, 4, false>), dim3(1), dim3(256), 0, s, A, lda, j, m, fjb,
+    hipLaunchKernelGGL((k_panel_reg<2, 4, false>), dim3(1), dim3(320), 0, s, A, lda, j, m, fjb,
                        tau_dm, truncate, tau, st, mode);
   } else if (rows <= RP_MID) {
-    hipLaunchKernelGGL((k_panel_reg<3, 8, false>), dim3(1), dim3(512), 0, s, A, lda, j, m, fjb,
+    hipLaunchKernelGGL((k_panel_reg<3, 7, false>), dim3(1), dim3(512), 0, s, A, lda, j, m, fjb,
                        tau_dm, truncate, tau, st, mode);
   } else if (nwg == 1) {
-    hipLaunchKernelGGL((k_panel_reg<4, 8, false>), dim3(1), dim3(512), 0, s, A, lda, j, m, fjb,
+    hipLaunchKernelGGL((k_panel_reg<4, 7, false>), dim3(1), dim3(512), 0, s, A, lda, j, m, fjb,
                        tau_dm, truncate, tau, st, mode);
   } else if (nwg <= RP_WGS) {
     hipLaunchKernelGGL(k_panel_slots, dim3(8 * (nwg + 1)), dim3(256), 0, s, st,
                        KMAX * KMAX * (nwg + 1), mode);
-    hipLaunchKernelGGL((k_panel_reg<4, 8, true>), dim3(nwg), dim3(512), 0, s, A, lda, j, m, fjb,
+    hipLaunchKernelGGL((k_panel_reg<4, 7, true>), dim3(nwg), dim3(512), 0, s, A, lda, j, m, fjb,
                        tau_dm, truncate, tau, st, mode);
   }
   hipLaunchKernelGGL(k_panel_slow, dim3(1), dim3(1024), 0, s, A, lda, j, m, fjb, tau_dm,

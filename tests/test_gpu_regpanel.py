@@ -1,7 +1,7 @@
 """The register-held column-by-column panel at the edges of its forms.
 
 The unpivoted QR runs it on every panel: one workgroup of four waves up to
-128 rows, of eight waves up to 384 and 512, several workgroups above; a panel
+128 rows, of seven up to 336 and 448, several workgroups above; a panel
 whose sums of squares leave the safe range is declined and taken by the
 memory-based form.  Reference: LAPACK's dgeqrf (scipy).  Bar: R normwise and
 the reflectors within 64 m eps cond-free for Gaussian input, 1e-12 here.
@@ -53,8 +53,8 @@ def check(got, ref, tol=1e-12):
 
 @pytest.mark.parametrize("m,n,pad", [
     (1, 1, 0), (2, 2, 1), (15, 15, 0), (33, 16, 3), (64, 64, 0), (127, 70, 0), (128, 128, 0),
-    (129, 17, 0), (192, 300, 5), (384, 64, 0), (385, 65, 0), (512, 100, 0), (513, 64, 0),
-    (1024, 40, 0), (1025, 130, 7), (2500, 65, 0), (40, 90, 0)])
+    (129, 17, 0), (192, 300, 5), (336, 64, 0), (337, 65, 0), (448, 100, 0), (449, 64, 0),
+    (896, 40, 0), (897, 130, 7), (4100, 65, 0), (40, 90, 0)])
 def test_sizes(gpu, m, n, pad):
     print("regpanel", m, n, pad, flush=True)
     a = np.random.default_rng(100 * m + n).standard_normal((m, n))
