@@ -514,11 +514,8 @@ int run_dm(const Args& x) {
     // The FP64 trailing update runs deferred and merged into the next step's
     // pass over C (trailing.hip); the reduced-precision products, and
     // QRDM_TRAILING=3pass, apply each step's update in three kernels.
-    // The merged pass moves C in 32-byte vectors: lda % 4 == 0, A 32-byte
-    // aligned, at least four rows.
     const char* pt = getenv("QRDM_TRAILING");
-    bool fused_now = !(pt && strcmp(pt, "3pass") == 0) && lda % 4 == 0 && m >= 4 &&
-                     (reinterpret_cast<uintptr_t>(A) & 31) == 0;
+    bool fused_now = !(pt && strcmp(pt, "3pass") == 0);
     StepBufs bufs{B.V, fused_now ? (size_t)B.ldv * KMAX : 0, B.ldv, B.Wf,
                   fused_now ? (size_t)KMAX * n : 0};
     // Reduced-precision forms (x.trail): the trailing update stays FP64 until

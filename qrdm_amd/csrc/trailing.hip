@@ -32,31 +32,16 @@
 
 namespace qrdm {
 
-constexpr int FU_CH = 16;         // rows per chunk
+constexpr int FU_CH = 32;         // rows per chunk: two interleaved 16-row tiles
 constexpr int FU_NWG = 4;         // waves per workgroup
 constexpr int FU_MAX_SPLIT = 16;  // row slabs of the partial products
-// LDS layouts of the V chunks (64 banks of 4 bytes), measured free of bank
-// conflicts for the accesses below: V_s by rows of 66 doubles (the product-1
-// operand is read as 16-byte pairs of adjacent columns, a lane's rows 33
-// pairs apart), V_{s+1} by columns of 17 doubles (read as pairs of rows).
-constexpr int FU_VP_LD = 66;
-constexpr int FU_VN_LD = FU_CH + 1;
+constexpr int FU_OCC = 2;         // workgroups per CU (64 KB of LDS, 256 registers a lane)
 
-// Launch shapes of the fused pass: U 16-column blocks per wave (a workgroup
-// covers 64 U columns), C prefetched PF chunks ahead, OCC waves per SIMD.
-template <int U>
-struct FuShape;
-template <>
-struct FuShape<1> {
-  static constexpr int PF = 2, OCC = 3;
-};
-template <>
-struct FuShape<2> {
-  static constexpr int PF = 1, OCC = 2;
-};
+// Two doubles at any multiple of eight bytes (a column of any leading dimension).
+typedef double fu_pair __attribute__((ext_vector_type(2), aligned(8)));
 
 // Geometry of one fused pass over rows [r_lo, m) and columns [c0, n):
-// chunks of FU_CH rows from the 16-row boundary at or below r_lo, split into
+// chunks of FU_CH rows from the FU_CH-row boundary at or below r_lo, split into
 // ns slabs of whole chunks, and column groups of gc columns.
 struct FuGeom {
   int base, nchunk, slab_ch, cgroups;
@@ -76,30 +61,52 @@ __host__ __device__ __forceinline__ FuGeom fused_geom(int r_lo, int m, int c0, i
 }
 
 // Workgroups of a fused pass per XCD: column group g goes to XCD g % 8 with
-// all its row slabs, so that the step's end (one workgroup per 64-column
-// tile, dispatched round-robin to the XCDs: tile g on XCD g % 8) reads the
-// slab partials of its columns from its own L2.
+// all its row slabs, so that each XCD holds one round of workgroups.
 __host__ __device__ __forceinline__ int fused_per_xcd(int ns, int cgroups) {
   return ((cgroups + 7) / 8) * ns;
 }
 
+// A 32 x 64 chunk of V in LDS as 16-byte units of two rows: unit (row pair
+// rp, column c) at [c][rp ^ (c % 16)].  The 16 lanes that share a column and
+// the 16 that share a row pair both read 16 different units of a 256-byte
+// line: no bank conflicts in either product.
+typedef double2 FuChunk[KMAX][FU_CH / 2];
+
 // One pass.  APPLY: C -= Vp Wprev (Vp, Wprev of the previous step) before
 // the products; ACCUM: Wp[slab] = Vn^T C.  Rows [r_lo, m) of columns
-// [c0, n) are written (APPLY only).  Wave w of a workgroup owns 16 U
-// columns; lane group g = lane / 16 holds rows 4g..4g+3 of a 16-row chunk,
-// so C moves in 32-byte vectors (lda % 4 == 0, 32-byte aligned A); the V
-// chunks are shared through LDS.  W and the partials have leading dimension
-// n (absolute columns); ns slabs.  With st (the DM loop) r_lo, c0 and the
-// buffers come from st; the grid is sized for the lowest j and surplus
-// workgroups return.
+// [c0, n) are written (APPLY only).
+//
+// What bounds it: the FP64 matrix cores (64 cycles per 16 x 16 x 4 product, 256
+// flops per 16 bytes of C with 64 columns of V), if loads, LDS and barriers
+// stay out of their way.  A wave owns 16 U columns and a chunk of 32 rows is two
+// 16-row tiles, even rows and odd rows: a lane's two consecutive rows are one
+// 16-byte element of C and one 16-byte unit of V, so one LDS read feeds 2 U
+// products and independent accumulators keep the cores busy.  The tile
+// of C in the output layout of product 1 is the B operand of product 2.  The
+// next chunk of V goes from memory straight to the other LDS buffer and the
+// next chunk of C to registers while this one is multiplied (64 U products per
+// wave and barrier), so nothing waits for a load issued in the same chunk.
+// Measured: the first pass at 8192 x 8192 325 us, 53 TF/s, the matrix cores busy
+// in 72 % of the cycles (2.23 GHz under this load); per 8192 x 8192
+// factorisation 17.2 ms against 18.2 with 16-row chunks, V stored to LDS
+// through registers and a barrier every 32 products, 16384 x 1024 1.36 against
+// 1.64.  Odd leading dimensions run here too (3001 x 1777 DM 6.53 -> 6.06 ms
+// against the three-kernel form with 8-byte loads).
+//
+// V is zero above its panel (within 64 rows) and past m, which the callers
+// keep so: no masks in the products, only the stores look at r_lo and m.  W
+// and the partials have leading dimension n (absolute columns); ns slabs.
+// With st (the DM loop) r_lo, c0 and the buffers come from st; the grid is
+// sized for the lowest j and surplus workgroups return.
 template <bool APPLY, bool ACCUM, int U>
-__global__ __launch_bounds__(64 * FU_NWG, FuShape<U>::OCC) void k_fused(
-    double* A, int lda, int r_lo, int m, int c0, int n, StepBufs bufs, double* Wp, int ns,
-    int cur, const DevState* st) {
-  constexpr int PF = FuShape<U>::PF, NSET = PF + 1;
+__global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int lda, int r_lo, int m,
+                                                               int c0, int n, StepBufs bufs,
+                                                               double* Wp, int ns, int cur,
+                                                               const DevState* st) {
   constexpr int WC = 16 * U, GC = FU_NWG * WC;
-  __shared__ __align__(16) double VpS[2][FU_CH][FU_VP_LD];
-  __shared__ __align__(32) double VnS[2][64][FU_VN_LD];
+  // the chunks of V_s and V_{s+1}, two buffers each (arrays of their own, so
+  // that a load on its way into one does not hold up reads of the other)
+  __shared__ FuChunk vp0, vp1, vn0, vn1;
   if (st) {
     if (dm_stopped(st)) return;
     r_lo = st->j;
@@ -112,11 +119,12 @@ __global__ __launch_bounds__(64 * FU_NWG, FuShape<U>::OCC) void k_fused(
   const double* Wprev = bufs.W + (size_t)(cur ^ 1) * bufs.wstride;
   const FuGeom G = fused_geom(r_lo, m, c0, n, ns, GC);
   const int per = fused_per_xcd(ns, G.cgroups);
-  const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
-  if (k >= per) return;
-  const int slab = k % ns, cgrp = xcd + 8 * (k / ns);
+  const int xcd = blockIdx.x & 7, kx = blockIdx.x >> 3;
+  if (kx >= per) return;
+  const int slab = kx % ns, cgrp = xcd + 8 * (kx / ns);
   if (cgrp >= G.cgroups) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, li = lane & 15;
   const int ncol = n - c0;
   const int cbw = cgrp * GC + wave * WC;  // this wave's columns (relative to c0)
@@ -131,140 +139,138 @@ __global__ __launch_bounds__(64 * FU_NWG, FuShape<U>::OCC) void k_fused(
     cok[u] = c < ncol;
     Cc[u] = A + (size_t)(c0 + (cok[u] ? c : (ncol > 0 ? ncol - 1 : 0))) * lda;
   }
-  // the previous step's W tile: wr[s][u] = W(16g + s, column 16u + li) (lane
-  // group g takes the k indices 16g..16g+15 of product 1)
+  // the previous step's W tile, negated: wr[s][u] = -W(4s + g, column 16u + li)
+  // (lane group g takes the k index 4s + g of step s of product 1)
   double wr[16][U];
   if (APPLY) {
 #pragma unroll
-    for (int s = 0; s < 16; s++)
+    for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int u = 0; u < U; u++)
-        wr[s][u] = cok[u] ? Wprev[(size_t)(c0 + cbw + 16 * u + li) * KMAX + 16 * g + s] : 0.0;
+      for (int s = 0; s < 16; s++)
+        wr[s][u] = cok[u] ? -Wprev[(size_t)(c0 + cbw + 16 * u + li) * KMAX + 4 * s + g] : 0.0;
   }
   dbl4 acc[4][U];
 #pragma unroll
   for (int t = 0; t < 4; t++)
 #pragma unroll
     for (int u = 0; u < U; u++) acc[t][u] = (dbl4){0.0, 0.0, 0.0, 0.0};
-  // last 4-row group inside the column (rows up to round_up(m, 4) - 1 exist)
-  const int rclamp = ((m + 3) & ~3) - 4;
-  // V chunk loaders (a thread brings rows vq..vq+3 of column vc).  V_s: wave
-  // w takes rows 8 (w & 1)..+7 of columns 32 (w >> 1)..+31, a lane pair one
-  // column; V_{s+1}: four lanes one column, a wave 16 columns.  Both make the
-  // LDS stores of a wave conflict-free in the layouts above.
-  const int pq = 4 * (2 * (wave & 1) + (lane & 1)), pc = 32 * (wave >> 1) + (lane >> 1);
-  const int nq = 4 * (tid & 3), nc = tid >> 2;
-  auto load_vv = [&](const double* Vb, int c, int vq, int vc) -> dbl4 {
-    const int r = G.base + FU_CH * c + vq;
-    return *reinterpret_cast<const dbl4*>(Vb + (size_t)vc * ldv + r);
-  };
-  // rows outside [r_lo, m) enter the products as zero
-  auto mask4 = [&](int c, int vq, dbl4 v) -> dbl4 {
-    const int r = G.base + FU_CH * c + vq;
+  // chunk c of V into LDS: a wave takes the columns 16 w .. 16 w + 15, four
+  // per load (lane: column lane / 16, unit lane % 16): the lane's byte offsets
+  // from the wave's first column
+  unsigned voff[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) v[q] = (r + q >= r_lo && r + q < m) ? v[q] : 0.0;
-    return v;
-  };
-  auto store_vp = [&](int buf, int c, dbl4 v) {
-    v = mask4(c, pq, v);
+  for (int i = 0; i < 4; i++)
+    voff[i] = 8u * ((unsigned)(4 * i + g) * (unsigned)ldv + 2u * (unsigned)(li ^ (4 * i + g)));
+  auto load_v = [&](const double* V, FuChunk& S, int c) {
+    const char* src =
+        reinterpret_cast<const char*>(V + (size_t)(16 * wave) * ldv + G.base + FU_CH * c);
 #pragma unroll
-    for (int q = 0; q < 4; q++) VpS[buf][pq + q][pc] = -v[q];
+    for (int i = 0; i < 4; i++)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(src + voff[i]),
+          (__attribute__((address_space(3))) void*)&S[16 * wave + 4 * i][0], 16, 0, 0);
   };
-  auto store_vn = [&](int buf, int c, dbl4 v) {
-    v = mask4(c, nq, v);
+  // chunk c of C as it lies in memory: rows base + 32c + 8v + 2g + (0, 1) in
+  // x[u][v] (taken apart into the tiles where they are used: a move here would
+  // wait for the load)
+  auto load_c = [&](int c, fu_pair (&x)[U][4]) {
+    const int r0 = G.base + FU_CH * c;
+    if (r0 + FU_CH <= m) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) VnS[buf][nc][nq + q] = v[q];
-  };
-  auto load_c = [&](int c, dbl4 (&cc)[U]) {
-    const int r = min(G.base + FU_CH * c + 4 * g, rclamp);
+      for (int u = 0; u < U; u++)
 #pragma unroll
-    for (int u = 0; u < U; u++) cc[u] = *reinterpret_cast<const dbl4*>(Cc[u] + r);
+        for (int v = 0; v < 4; v++)
+          x[u][v] = *reinterpret_cast<const fu_pair*>(Cc[u] + r0 + 8 * v + 2 * g);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+          for (int h = 0; h < 2; h++) x[u][v][h] = Cc[u][min(r0 + 8 * v + 2 * g + h, m - 1)];
+    }
   };
-  // product 1's A operand rows: chunk row pi(li) = 4 (li % 4) + li / 4, so
-  // that output row g + 4v of the 16 x 16 tile is chunk row 4g + v
-  const int prow = 4 * (li & 3) + (li >> 2);
-  // One chunk: product 1 on cur (C of chunk c) and the store of its updated
-  // rows, the loads of V for chunk c + 1 and of C for chunk c + PF (into pre,
-  // the set stored a chunk earlier), product 2 on cur, the next V chunk into
-  // LDS, and the barrier.
-  auto step = [&](int c, dbl4 (&cur)[U], dbl4 (&pre)[U]) {
-    const int buf = (c - ch0) & 1;
-    const bool more = c + 1 < ch1;
-    const int cn = more ? c + 1 : c;
-    const int r4 = G.base + FU_CH * c + 4 * g;  // first row of this lane group
-    const bool interior = G.base + FU_CH * c >= r_lo && G.base + FU_CH * (c + 1) <= m;
+  // One chunk: the next one's loads, product 1 and the store of its rows,
+  // product 2.  Tile h of C: rows 8v + 2g + h in cc[h][u][v].
+  auto step = [&](int c, FuChunk& sp, FuChunk& sn, FuChunk& np, FuChunk& nn, fu_pair (&x)[U][4]) {
+    dbl4 cc[2][U];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) cc[h][u][v] = x[u][v][h];
+    if (c + 1 < ch1) {
+      if (APPLY) load_v(Vp, np, c + 1);
+      if (ACCUM) load_v(Vn, nn, c + 1);
+      load_c(c + 1, x);
+    }
     if (APPLY) {
-      // product 1: C -= Vp W on rows 4g + v of columns 16u + li
 #pragma unroll
-      for (int s = 0; s < 16; s += 2) {
-        const double2 a = *reinterpret_cast<const double2*>(&VpS[buf][prow][16 * g + s]);
-#pragma unroll
-        for (int u = 0; u < U; u++)
-          cur[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, wr[s][u], cur[u], 0, 0, 0);
-#pragma unroll
-        for (int u = 0; u < U; u++)
-          cur[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, wr[s + 1][u], cur[u], 0, 0, 0);
-      }
-      if (interior) {
-#pragma unroll
-        for (int u = 0; u < U; u++)
-          if (cok[u]) *reinterpret_cast<dbl4*>(Cc[u] + r4) = cur[u];
-      } else {
+      for (int s = 0; s < 16; s++) {
+        const double2 a = sp[4 * s + g][li ^ (4 * (s & 3) + g)];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-          if (!cok[u]) continue;
-#pragma unroll
-          for (int q = 0; q < 4; q++)
-            if (r4 + q >= r_lo && r4 + q < m) Cc[u][r4 + q] = cur[u][q];
+          cc[0][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, wr[s][u], cc[0][u], 0, 0, 0);
+          cc[1][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, wr[s][u], cc[1][u], 0, 0, 0);
         }
+      }
+      const int r0 = G.base + FU_CH * c;
+      if (r0 >= r_lo && r0 + FU_CH <= m) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (cok[u]) {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+              *reinterpret_cast<fu_pair*>(Cc[u] + r0 + 8 * v + 2 * g) =
+                  (fu_pair){cc[0][u][v], cc[1][u][v]};
+          }
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (cok[u]) {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+#pragma unroll
+              for (int h = 0; h < 2; h++) {
+                const int r = r0 + 8 * v + 2 * g + h;
+                if (r >= r_lo && r < m) Cc[u][r] = cc[h][u][v];
+              }
+          }
       }
     }
-    dbl4 vpn, vnn;
-    if (APPLY) vpn = load_vv(Vp, cn, pq, pc);
-    if (ACCUM) vnn = load_vv(Vn, cn, nq, nc);
-    if (c + PF < ch1) load_c(c + PF, pre);
     if (ACCUM) {
-      if (!interior) {
-        // rows outside [r_lo, m) (R rows above, padding below) enter as zero
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const bool ok = r4 + q >= r_lo && r4 + q < m;
-#pragma unroll
-          for (int u = 0; u < U; u++) cur[u][q] = ok ? cur[u][q] : 0.0;
-        }
-      }
-      // product 2: Wp += Vn^T C, k-step v = rows 4g + v
 #pragma unroll
       for (int v = 0; v < 4; v++) {
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const double a = VnS[buf][16 * t + li][4 * g + v];
+        for (int tp = 0; tp < 4; tp += 2) {
+          double2 a[2];
 #pragma unroll
-          for (int u = 0; u < U; u++)
-            acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, cur[u][v], acc[t][u], 0, 0, 0);
+          for (int t = 0; t < 2; t++) a[t] = sn[16 * (tp + t) + li][(g + 4 * v) ^ li];
+#pragma unroll
+          for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+              for (int u = 0; u < U; u++)
+                acc[tp + t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    h ? a[t].y : a[t].x, cc[h][u][v], acc[tp + t][u], 0, 0, 0);
         }
       }
     }
-    if (more) {
-      if (APPLY) store_vp(buf ^ 1, cn, vpn);
-      if (ACCUM) store_vn(buf ^ 1, cn, vnn);
-    }
-    __syncthreads();
+    __syncthreads();  // the next chunk of V is in LDS (every load has arrived)
   };
-  dbl4 cs[NSET][U];
+  fu_pair x[U][4];
   if (ch1 > ch0) {
-    if (APPLY) store_vp(0, ch0, load_vv(Vp, ch0, pq, pc));
-    if (ACCUM) store_vn(0, ch0, load_vv(Vn, ch0, nq, nc));
-#pragma unroll
-    for (int p = 0; p < PF; p++)
-      if (ch0 + p < ch1) load_c(ch0 + p, cs[p]);
+    if (APPLY) load_v(Vp, vp0, ch0);
+    if (ACCUM) load_v(Vn, vn0, ch0);
+    load_c(ch0, x);
   }
   __syncthreads();
 #pragma clang loop unroll(disable)
-  for (int c = ch0; c < ch1; c += NSET) {
-#pragma unroll
-    for (int q = 0; q < NSET; q++)
-      if (c + q < ch1) step(c + q, cs[q], cs[(q + PF) % NSET]);
+  for (int c = ch0; c < ch1; c += 2) {
+    step(c, vp0, vn0, vp1, vn1, x);
+    if (c + 1 < ch1) step(c + 1, vp1, vn1, vp0, vn0, x);
   }
   if (!ACCUM) return;
   // partial tile: row 16t + g + 4w, column 16u + li of the wave's columns
@@ -280,25 +286,35 @@ __global__ __launch_bounds__(64 * FU_NWG, FuShape<U>::OCC) void k_fused(
   }
 }
 
-// The launch shape (16-column blocks per wave) of the fused passes.
-int g_fused_u = 1;
-
 static int fused_gc(int u) { return FU_NWG * 16 * u; }
-// workgroups in one round: OCC waves per SIMD, four SIMDs per CU, 256 CUs
-static int fused_wgs(int u) { return 256 * (u == 1 ? FuShape<1>::OCC : FuShape<2>::OCC); }
 
-int fused_max_slabs() { return FU_MAX_SPLIT; }
-
-// Row slabs of a fused pass: one round of workgroups on every XCD (its
-// column groups times the slabs within an eighth of the chip's slots) where
-// the column groups allow it.
-int fused_slabs(int r_lo, int m, int c0, int n) {
-  const FuGeom g = fused_geom(r_lo, m, c0, n, 1, fused_gc(g_fused_u));
+// Row slabs of a fused pass with column groups of 64 u columns: one round of
+// workgroups on every XCD (its column groups times the slabs within an eighth
+// of the chip's slots) where the column groups allow it.
+static int fused_slabs_u(int r_lo, int m, int c0, int n, int u) {
+  const FuGeom g = fused_geom(r_lo, m, c0, n, 1, fused_gc(u));
   if (g.cgroups <= 0 || g.nchunk <= 0) return 1;
-  int ns = (fused_wgs(g_fused_u) / 8) / ((g.cgroups + 7) / 8);
+  int ns = (32 * FU_OCC) / ((g.cgroups + 7) / 8);
   if (ns > FU_MAX_SPLIT) ns = FU_MAX_SPLIT;
   if (ns > g.nchunk) ns = g.nchunk;
   return ns < 1 ? 1 : ns;
+}
+
+// 16-column blocks per wave: two, unless one fills more of the chip's slots.
+// A full round of two runs at 53 TF/s (8192 x 8192, 72 % of the matrix cores'
+// cycles), one of one about a tenth slower, so one is taken where two would
+// leave more than a tenth of the slots of one empty (narrow C, or a last
+// column group per XCD that is mostly missing).
+static int fused_u(int r_lo, int m, int c0, int n) {
+  const int w1 = ((n - c0 + 63) / 64) * fused_slabs_u(r_lo, m, c0, n, 1);
+  const int w2 = ((n - c0 + 127) / 128) * fused_slabs_u(r_lo, m, c0, n, 2);
+  return 10 * w2 >= 9 * w1 ? 2 : 1;
+}
+
+int fused_max_slabs() { return FU_MAX_SPLIT; }
+
+int fused_slabs(int r_lo, int m, int c0, int n) {
+  return fused_slabs_u(r_lo, m, c0, n, fused_u(r_lo, m, c0, n));
 }
 
 template <int U>
@@ -322,7 +338,7 @@ void launch_fused(double* A, int lda, int r_lo, int m, int c0, int n, const Step
                   double* Wp, int ns, int apply, int accum, int cur, hipStream_t s,
                   const DevState* st) {
   if (n - c0 <= 0 || m - r_lo <= 0 || !(apply || accum)) return;
-  if (g_fused_u == 2)
+  if (fused_u(r_lo, m, c0, n) == 2)
     launch_fused_u<2>(A, lda, r_lo, m, c0, n, bufs, Wp, ns, apply, accum, cur, s, st);
   else
     launch_fused_u<1>(A, lda, r_lo, m, c0, n, bufs, Wp, ns, apply, accum, cur, s, st);
