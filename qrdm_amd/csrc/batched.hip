@@ -381,7 +381,7 @@ __device__ __forceinline__ int bt_panel_gram(double* a, int lda, int j, int m, i
   }
   lds_barrier();
   if (tid < k) tau[j + tid] = 1.0 / E0[tid][tid];
-  lu_inverse<false>(E0, E1, L.rinv, Yof(L.R1));  // E1 = T (upper)
+  upper_inverse(E0, E1, L.rinv, Yof(L.R1));  // E1 = T (upper)
   for (int e = tid; e < KMAX * KMAX; e += NW * 64) {
     const int r = e & 63, c = e >> 6;
     L.Ts[r + c * KMAX] = (r < k && c < k && r <= c) ? E1[r][c] : 0.0;

@@ -362,102 +362,119 @@ __device__ __forceinline__ int lu_signed_blocked(double (*W)[LDP], int nlim, con
   return nlim;
 }
 
-// The off-diagonal blocks of lu_inverse's X from its diagonal blocks: block
-// distance d = 1, 2, 3 on the matrix cores, one block per wave (the first four
-// waves): X_ij = -X_ii Y with Y = sum_{k = i+1..j} R_ik X_kj (R = U or L^T).
-// Ys: one 16 x 16 scratch tile per wave.  Ends with a barrier.
-template <bool BOTH>
-__device__ __forceinline__ void inverse_merge(const double (*W)[LDP], double (*X)[LDP],
-                                              double (*Ys)[BLK][BLK + 1]) {
-  const int tid = local_tid(), lane = tid & 63, wave = tid >> 6;
-  // R_m(i, l): m = 1 U, m = 0 L^T (unit diagonal); zero below the diagonal
-  auto Rm = [&](int m, int i, int l) -> double {
-    return m ? ((i <= l) ? W[i][l] : 0.0) : ((i < l) ? W[l][i] : (i == l ? 1.0 : 0.0));
-  };
-  // X_m(i, j) of the inverse of R_m, from X's storage
-  auto Xm = [&](int m, int i, int j) -> double {
-    return m ? ((i <= j) ? X[i][j] : 0.0) : ((i < j) ? X[j][i] : (i == j ? 1.0 : 0.0));
-  };
-  const int g = lane >> 4, li = lane & 15;
-  for (int d = 1; d < 4; d++) {
-    const int ntgt = (BOTH ? 2 : 1) * (4 - d);
-    for (int t = wave; wave < 4 && t < ntgt; t += 4) {
-      const int m = BOTH ? (t & 1) : 1, bi = BOTH ? (t >> 1) : t, bj = bi + d;
-      dbl4p acc = {0.0, 0.0, 0.0, 0.0};
-      for (int kb = bi + 1; kb <= bj; kb++) {
+// The inverses of the four 16 x 16 diagonal blocks of the upper triangular W
+// into X (its rows on and above the diagonal), rdiag the reciprocals of W's
+// diagonal; one wave, lane 16 b + c column c of block b.  Back substitution
+// column by column of W: the 15 - l updates after x_l are independent, so a
+// column costs two dependent operations (row by row it costs one per element).
+__device__ __forceinline__ void diag_inverse(const double (*W)[LDP], const double* rdiag,
+                                             double (*X)[LDP]) {
+  const int lane = local_tid() & 63, base = lane & 48, c = lane & 15;
+  double x[BLK];
 #pragma unroll
-        for (int k0 = 0; k0 < BLK; k0 += 4) {
-          const double a = Rm(m, BLK * bi + li, BLK * kb + k0 + g);
-          const double b = Xm(m, BLK * kb + k0 + g, BLK * bj + li);
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-        }
-      }
+  for (int i = 0; i < BLK; i++) x[i] = (i == c) ? 1.0 : 0.0;
 #pragma unroll
-      for (int v = 0; v < 4; v++) Ys[wave][g + 4 * v][li] = acc[v];
-      wave_lds_sync();
-      dbl4p acc2 = {0.0, 0.0, 0.0, 0.0};
+  for (int l = BLK - 1; l >= 0; l--) {
+    x[l] *= rdiag[base + l];
 #pragma unroll
-      for (int k0 = 0; k0 < BLK; k0 += 4) {
-        const double a = Xm(m, BLK * bi + li, BLK * bi + k0 + g);
-        acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, Ys[wave][k0 + g][li], acc2, 0, 0, 0);
-      }
-      wave_lds_sync();  // Ys is reused by the wave's next block
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int r = BLK * bi + g + 4 * v, c = BLK * bj + li;
-        if (m)
-          X[r][c] = -acc2[v];
-        else
-          X[c][r] = -acc2[v];
-      }
-    }
-    lds_barrier();
+    for (int i = 0; i < l; i++) x[i] = fma(-W[base + i][base + l], x[l], x[i]);
   }
+#pragma unroll
+  for (int i = 0; i < BLK; i++)
+    if (i <= c) X[base + i][base + c] = x[i];
 }
 
-// X := L^-1 and U^-1 of the pair held in one 64 x 64 matrix W (L unit lower
-// triangular strictly below the diagonal, U upper triangular on and above
-// it, non-zero diagonal), X in the same layout: L^-1 strictly below the
-// diagonal (its unit diagonal implied), U^-1 on and above; at least 256
-// threads (the first four waves compute), ends with a barrier.  BOTH = false: U^-1 only (W's lower part is not read, X's
-// is set to zero).  Both go by 16 x 16 blocks, L^-1 as (L^T)^-1 read and
-// stored transposed: the diagonal blocks by back substitution (wave w takes
-// block w of both, one lane per column: lanes 0-15 U, 16-31 L^T), then the
-// others (inverse_merge; Ys is its scratch).
-template <bool BOTH = true>
-__device__ __forceinline__ void lu_inverse(const double (*W)[LDP], double (*X)[LDP], double* rinv,
-                                           double (*Ys)[BLK][BLK + 1]) {
-  const int tid = local_tid(), lane = tid & 63, wave = tid >> 6;
-  // R_m(i, l): m = 1 U, m = 0 L^T (unit diagonal); zero below the diagonal
-  auto Rm = [&](int m, int i, int l) -> double {
-    return m ? ((i <= l) ? W[i][l] : 0.0) : ((i < l) ? W[l][i] : (i == l ? 1.0 : 0.0));
-  };
-  if (tid < KMAX) rinv[tid] = 1.0 / W[tid][tid];
-  if (!BOTH) {
-    for (int e = tid; e < KMAX * KMAX; e += NT1) {
+// X(16 ti .., 16 tj ..) := sign * sum over k blocks [k0, k1] of fa(row, q)
+// fb(q, col), 16-deep, on the matrix cores (one wave); the sum is returned in
+// the output layout.
+template <class FA, class FB>
+__device__ __forceinline__ dbl4p block_product(int ti, int tj, int k0, int k1, FA fa, FB fb) {
+  const int lane = local_tid() & 63, g = lane >> 4, li = lane & 15;
+  dbl4p acc = {0.0, 0.0, 0.0, 0.0};
+  for (int kb = k0; kb <= k1; kb++)
+#pragma unroll
+    for (int k4 = 0; k4 < BLK; k4 += 4) {
+      const int q = BLK * kb + k4 + g;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(fa(BLK * ti + li, q), fb(q, BLK * tj + li), acc, 0,
+                                                 0, 0);
+    }
+  return acc;
+}
+
+// The blocks above the diagonal of X = W^-1 (W upper triangular) from its
+// diagonal blocks, by halves: X_12 = -X_11 W_12 X_22 for the two 32 x 32
+// diagonal blocks, then for the whole.  X is zero below its diagonal.  The
+// first four waves compute; Ys: one 16 x 16 tile per wave.  Ends with a barrier.
+__device__ __forceinline__ void inverse_merge(const double (*W)[LDP], double (*X)[LDP],
+                                              double (*Ys)[BLK][BLK + 1]) {
+  const int tid = local_tid(), lane = tid & 63, g = lane >> 4, li = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto fw = [&](int r, int q) { return W[r][q]; };
+  auto fx = [&](int r, int q) { return X[r][q]; };
+  if (wave < 2) {
+    const int b = 2 * wave;
+    const dbl4p y = block_product(b, b + 1, b + 1, b + 1, fw, fx);
+#pragma unroll
+    for (int v = 0; v < 4; v++) Ys[wave][g + 4 * v][li] = y[v];
+    wave_lds_sync();
+    const dbl4p x = block_product(
+        b, 0, b, b, fx, [&](int q, int c) { return Ys[wave][q & 15][c]; });
+#pragma unroll
+    for (int v = 0; v < 4; v++) X[BLK * b + g + 4 * v][BLK * (b + 1) + li] = -x[v];
+  }
+  lds_barrier();
+  const int ti = wave & 1, tj = 2 + ((wave >> 1) & 1);
+  if (wave < 4) {
+    const dbl4p y = block_product(ti, tj, 2, tj, fw, fx);
+#pragma unroll
+    for (int v = 0; v < 4; v++) Ys[wave][g + 4 * v][li] = y[v];
+  }
+  lds_barrier();
+  if (wave < 4) {
+    // Y(kb, tj) is the tile of wave kb + 2 (tj - 2)
+    const dbl4p x = block_product(
+        ti, 0, ti, 1, fx,
+        [&](int q, int c) { return Ys[(q >> 4) + 2 * (tj - 2)][q & 15][c]; });
+#pragma unroll
+    for (int v = 0; v < 4; v++) X[BLK * ti + g + 4 * v][BLK * tj + li] = -x[v];
+  }
+  lds_barrier();
+}
+
+// X := W^-1, W upper triangular (its lower part is not read) with a non-zero
+// diagonal, X zero below the diagonal; at least 256 threads (the first four
+// waves compute), ends with a barrier.  Ys: inverse_merge's scratch.
+__device__ __forceinline__ void upper_inverse(const double (*W)[LDP], double (*X)[LDP], double* rinv,
+                                              double (*Ys)[BLK][BLK + 1]) {
+  const int tid = local_tid(), wave = tid >> 6;
+  if (wave == 0) {
+    rinv[tid] = 1.0 / W[tid][tid];
+    wave_lds_sync();
+    diag_inverse(W, rinv, X);
+  } else {
+    for (int e = tid - 64; e < KMAX * KMAX; e += NT1 - 64) {
       const int r = e & 63, c = e >> 6;
       if (r > c) X[r][c] = 0.0;
     }
   }
   lds_barrier();
-  if (wave < 4 && lane < (BOTH ? 32 : 16)) {
-    const int m = (lane < 16) ? 1 : 0, c = lane & 15, base = BLK * wave;
-    double x[BLK];
+  inverse_merge(W, X, Ys);
+}
+
+// D[r][c] = f(r, c, S[r][c]) over a 64 x 64 matrix; 256 threads, every read
+// before the first write (in one loop the writes hold up the next reads: 600
+// cycles an element instead of 60).
+template <class F>
+__device__ __forceinline__ void map_elements(const double (*S)[LDP], F f, double (*D)[LDP]) {
+  const int tid = local_tid();
+  double v[KMAX * KMAX / NT1];
 #pragma unroll
-    for (int i = BLK - 1; i >= 0; i--) {
-      double sacc = (i == c) ? 1.0 : 0.0;
+  for (int q = 0; q < KMAX * KMAX / NT1; q++) v[q] = S[(tid >> 6) + 4 * q][tid & 63];
 #pragma unroll
-      for (int l = i + 1; l < BLK; l++) sacc = fma(-Rm(m, base + i, base + l), x[l], sacc);
-      x[i] = m ? sacc * rinv[base + i] : sacc;
-    }
-#pragma unroll
-    for (int i = 0; i < BLK; i++) {
-      if (m && i <= c) X[base + i][base + c] = x[i];
-      if (!m && i < c) X[base + c][base + i] = x[i];
-    }
+  for (int q = 0; q < KMAX * KMAX / NT1; q++) {
+    const int r = (tid >> 6) + 4 * q, c = tid & 63;
+    D[r][c] = f(r, c, v[q]);
   }
-  lds_barrier();
-  inverse_merge<BOTH>(W, X, Ys);
 }
 
 // ---------------------------------------------------------------------------
@@ -466,7 +483,7 @@ __device__ __forceinline__ void lu_inverse(const double (*W)[LDP], double (*X)[L
 // fires there, and R1^-1.  Returns k1 >= 0 with S = R1 (on and above the
 // diagonal, zero below) identity-padded beyond k1 and X = R1^-1 (upper,
 // identity beyond k1); or -1 when a pivot does not resolve (the exact panel
-// takes the step over).  Y: lu_inverse's scratch.  The caller's S and diag
+// takes the step over).  Y: upper_inverse's scratch.  The caller's S and diag
 // writes are ordered by a barrier before the call.
 __device__ __forceinline__ int chol1_core(double (*S)[LDP], double (*X)[LDP], double (*Y)[BLK][BLK + 1],
                           double* rinv, const double* diag, int fjb, double tau_dm, int* s_done,
@@ -492,14 +509,12 @@ __device__ __forceinline__ int chol1_core(double (*S)[LDP], double (*X)[LDP], do
       rinv, s_done, s_why, &why);
   if (why == 2) return -1;
   // R1 (zero below the diagonal), identity-padded beyond k1 for the inverse
-  for (int e = tid; e < KMAX * KMAX; e += NT1) {
-    const int r = e >> 6, c = e & 63;
+  map_elements(S, [&](int r, int c, double v) {
     const bool in = r < k1 && c < k1;
-    const double v = (in && c >= r) ? S[r][c] : 0.0;
-    S[r][c] = in ? v : (r == c ? 1.0 : 0.0);
-  }
+    return in ? (c >= r ? v : 0.0) : (r == c ? 1.0 : 0.0);
+  }, S);
   lds_barrier();
-  lu_inverse<false>(S, X, rinv, Y);  // X = R1^-1 (upper part)
+  upper_inverse(S, X, rinv, Y);  // X = R1^-1 (upper part)
   return k1;
 }
 
@@ -649,21 +664,32 @@ __device__ __forceinline__ int tri_jobs(int kind, int wave, TileJob (&jb)[4]) {
 template <class FA, class FB>
 __device__ __forceinline__ int tri_product(int kind, FA fa, FB fb, TileJob (&jb)[4],
                                            dbl4p (&acc)[4]) {
-  const int lane = local_tid() & 63, wave = local_tid() >> 6, g = lane >> 4, li = lane & 15;
+  const int lane = local_tid() & 63, g = lane >> 4, li = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(local_tid() >> 6);
   const int nj = tri_jobs(kind, wave, jb);
 #pragma unroll
   for (int t = 0; t < 4; t++) {
     acc[t] = (dbl4p){0.0, 0.0, 0.0, 0.0};
     if (t < nj) {
-      for (int kb = jb[t].k0; kb <= jb[t].k1; kb++) {
+      // a job's operands are read before its chain of products
+      double a[4][4], b[4][4];
 #pragma unroll
-        for (int k4 = 0; k4 < BLK; k4 += 4) {
-          const int q = BLK * kb + k4 + g;
-          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa(BLK * jb[t].ti + li, q),
-                                                        fb(q, BLK * jb[t].tj + li), acc[t], 0, 0,
-                                                        0);
+      for (int kb = 0; kb < 4; kb++)
+        if (kb >= jb[t].k0 && kb <= jb[t].k1) {
+#pragma unroll
+          for (int k4 = 0; k4 < 4; k4++) {
+            const int q = BLK * kb + 4 * k4 + g;
+            a[kb][k4] = fa(BLK * jb[t].ti + li, q);
+            b[kb][k4] = fb(q, BLK * jb[t].tj + li);
+          }
         }
-      }
+#pragma unroll
+      for (int kb = 0; kb < 4; kb++)
+        if (kb >= jb[t].k0 && kb <= jb[t].k1) {
+#pragma unroll
+          for (int k4 = 0; k4 < 4; k4++)
+            acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[kb][k4], b[kb][k4], acc[t], 0, 0, 0);
+        }
     }
   }
   return nj;
@@ -808,12 +834,11 @@ __device__ __forceinline__ int recon_core(double (*SR)[LDP], double (*SA)[LDP], 
     int npass = 0;
     for (double err = emax * emax; err > 8.7e-19 && npass < 6; err *= emax) npass++;
     // SW = E, SX = F = triu_half(E)
-    for (int e = tid; e < KMAX * KMAX; e += NT1) {
-      const int r = e >> 6, c = e & 63;
-      const double ev = SX[r][c] - (r == c ? 1.0 : 0.0);
+    map_elements(SX, [&](int r, int c, double v) {
+      const double ev = v - (r == c ? 1.0 : 0.0);
       SW[r][c] = ev;
-      SX[r][c] = (r < c) ? ev : (r == c ? 0.5 * ev : 0.0);
-    }
+      return (r < c) ? ev : (r == c ? 0.5 * ev : 0.0);
+    }, SX);
     lds_barrier();
     TileJob jb[4];
     const int lane = tid & 63, g = lane >> 4, li = lane & 15;
@@ -845,10 +870,7 @@ __device__ __forceinline__ int recon_core(double (*SR)[LDP], double (*SA)[LDP], 
         for (int v = 0; v < 4; v++) if (t < nj) SR[BLK * jb[t].ti + g + 4 * v][BLK * jb[t].tj + li] += acc[t][v];
     }
     // R2^-1 = I - F (I - F (...)) into SW (upper)
-    for (int e = tid; e < KMAX * KMAX; e += NT1) {
-      const int r = e >> 6, c = e & 63;
-      SW[r][c] = (r == c ? 1.0 : 0.0) - SX[r][c];
-    }
+    map_elements(SX, [&](int r, int c, double v) { return (r == c ? 1.0 : 0.0) - v; }, SW);
     lds_barrier();
     for (int ps = 0; ps < npass; ps++) {
       const int nj = tri_product(
@@ -897,7 +919,7 @@ __device__ __forceinline__ int recon_core(double (*SR)[LDP], double (*SA)[LDP], 
     lds_barrier();
     if (tid >= k1 && tid < KMAX) SR[tid][tid] = 1.0;
     lds_barrier();
-    lu_inverse<false>(SR, SA, rinv, Y);  // SA = R^-1 (upper part)
+    upper_inverse(SR, SA, rinv, Y);  // SA = R^-1 (upper part)
   }
   // 4. Q11 = P_top R^-1 -> SW
   top_into(SW);
@@ -921,17 +943,30 @@ __device__ __forceinline__ int recon_core(double (*SR)[LDP], double (*SA)[LDP], 
   if (why == 2) return -1;
   // 6. top block (R rows scaled by the signs, V1 below), tau; SX := the
   // signed U (on and above the diagonal) and L (below), identity beyond k
-  for (int e = tid; e < KMAX * KMAX; e += NT1) {
-    const int r = e & 63, c = e >> 6;  // consecutive threads: consecutive rows
-    const bool in = r < k && c < k;
-    const double w = SW[r][c];
-    if (in) A[(size_t)(j + c) * lda + j + r] = (r <= c) ? dsg[r] * SR[r][c] : w;
-    SX[r][c] = in ? (r < c ? dsg[c] * w : (r == c ? -tl[c] : w)) : (r == c ? 1.0 : 0.0);
+  {
+    // consecutive threads: consecutive rows; every read before the writes
+    const int r = tid & 63, c0 = tid >> 6;
+    const double dr = dsg[r];
+    double w[KMAX * KMAX / NT1], sr[KMAX * KMAX / NT1], dc[KMAX * KMAX / NT1];
+#pragma unroll
+    for (int q = 0; q < KMAX * KMAX / NT1; q++) {
+      const int c = c0 + 4 * q;
+      w[q] = SW[r][c];
+      sr[q] = SR[r][c];
+      dc[q] = r == c ? tl[c] : dsg[c];
+    }
+#pragma unroll
+    for (int q = 0; q < KMAX * KMAX / NT1; q++) {
+      const int c = c0 + 4 * q;
+      const bool in = r < k && c < k;
+      if (in) A[(size_t)(j + c) * lda + j + r] = (r <= c) ? dr * sr[q] : w[q];
+      SX[r][c] = in ? (r < c ? dc[q] * w[q] : (r == c ? -dc[q] : w[q])) : (r == c ? 1.0 : 0.0);
+    }
   }
   if (tid < k) tau[tid] = tl[tid];
   lds_barrier();
   // 7. SR := U^-1 (on and above the diagonal; zero below)
-  lu_inverse<false>(SX, SR, rinv, Y);
+  upper_inverse(SX, SR, rinv, Y);
   // 8. M = R^-1 D U^-1, upper triangular, computed transposed (lower) so that
   // consecutive lanes store consecutive rows: the TRI_UU jobs with the tile
   // indices swapped; the tiles below the diagonal blocks are zero.  (T and
@@ -1109,8 +1144,8 @@ __global__ __launch_bounds__(256) void k_reduce_recon(const double* __restrict__
 // rows 16w .. 16w + 15 straight into the A operand (M through LDS), and V^T V
 // accumulates from the product's layout.
 __global__ __launch_bounds__(256) void k_v2(double* A, int lda, int m,
-                                            const double* __restrict__ M, const DevState* st,
-                                            StepBufs bufs, double* gram_part) {
+                                            const double* __restrict__ M, double* tau,
+                                            DevState* st, StepBufs bufs, double* gram_part) {
   __shared__ double Ms[KMAX][LDP];
   __shared__ double Gp[4][10][4][64];
   if (!step_runs(st, RUN_FAST)) return;
@@ -1122,6 +1157,7 @@ __global__ __launch_bounds__(256) void k_v2(double* A, int lda, int m,
   const int rs = j + blockIdx.x * PR_ROWS;
   if (rs >= m) return;
   if (blockIdx.x == 0) {
+    if (tid == 0) st->tau_base = tau;  // for the merged trailing pass
     // V is zero above the panel: the trailing update's slabs start at the
     // 32-row boundary at or below j and rely on it
     const int z0 = j >= KMAX ? j - KMAX : 0;
@@ -1232,7 +1268,7 @@ __global__ __launch_bounds__(256) void k_reduce_t(const double* __restrict__ par
   }
   lds_barrier();
   if (tid < k) tau[j + tid] = 1.0 / SX[tid][tid];  // 2 / S_ii
-  lu_inverse<false>(SX, SY, rinv, Y);  // SY = the upper triangular inverse
+  upper_inverse(SX, SY, rinv, Y);  // SY = the upper triangular inverse
   for (int e2 = tid; e2 < KMAX * KMAX; e2 += NT1) {
     const int r = e2 & 63, c = e2 >> 6;
     T_out[r + c * KMAX] = (r < k && c < k && r <= c) ? SY[r][c] : 0.0;
@@ -1247,9 +1283,11 @@ void launch_panel_fast(double* A, int lda, int j0, int m, double tau_dm, double*
   hipLaunchKernelGGL(k_qgram, dim3(nslab), dim3(256), 0, s, A, lda, m, R1inv, st, gram_part);
   hipLaunchKernelGGL(k_reduce_recon, dim3(KMAX * KMAX / 64), dim3(256), 0, s, gram_part, nslab,
                      G2, R1, R1inv, A, lda, tau_dm, tau, T, M, ticket, st);
-  hipLaunchKernelGGL(k_v2, dim3(nslab), dim3(256), 0, s, A, lda, m, M, st, bufs, gram_part);
-  hipLaunchKernelGGL(k_reduce_t, dim3(KMAX * KMAX / 64), dim3(256), 0, s, gram_part, m, G2, tau,
-                     T, ticket + 1, st);
+  hipLaunchKernelGGL(k_v2, dim3(nslab), dim3(256), 0, s, A, lda, m, M, tau, st, bufs, gram_part);
+  // the merged trailing pass sums V^T V itself (k_fused)
+  if (bufs.vstride == 0)
+    hipLaunchKernelGGL(k_reduce_t, dim3(KMAX * KMAX / 64), dim3(256), 0, s, gram_part, m, G2, tau,
+                       T, ticket + 1, st);
 }
 
 }  // namespace qrdm

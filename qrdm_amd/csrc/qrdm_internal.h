@@ -63,12 +63,21 @@ struct DevState {
                 // update the fused pass applies
   int policy_on;      // 1: the step's tau and delta come from the learned policy
   double pan_beta;    // R(0, 0) of the last column-by-column panel (wide.hip's blocks)
+  double* tau_base;   // tau[0..min(m, n)) (set by the Gram-based panel)
   double tau_step;    // tau and delta of the current step (the defaults, or the
   double delta_step;  // policy's proposal)
   StepRec last;
   StepWork work;
 };
 
+// The block reflector of a step of the merged trailing pass goes from the panel
+// to the step's end as the upper triangular T^-1 = striu(V^T V) + diag(1 / tau)
+// (the compact WY identity; Joffrain, Low, Quintana-Orti, van de Geijn, van
+// Zee, "Accumulating Householder transformations, revisited", ACM TOMS 32(2),
+// 2006), column-major in ws_mat(WS_S) with tau_i, the reciprocal, on the
+// diagonal (0: no reflector, a zero row and column of T) and zero outside
+// fjb_cmp x fjb_cmp.
+//
 // The head of a workspace, the same for every caller: the state, the 64 x 64
 // matrices, the Gram slabs' partial sums and the dense V.  Kernels that are
 // given only the state find the others behind it.

@@ -156,14 +156,16 @@ __device__ __forceinline__ bool rp_collect(const double* slots, int first, int s
 // R(0, 0), and every column is tested.  slots (nwg > 1): KMAX columns x
 // (nwg + 1) x KMAX values, empty on entry.  Returns the columns reduced with
 // everything written -- the panel, tau, rows [-z0, msub) of the dense V (zero
-// above the panel) and T -- or -1, declined, with nothing written.  Every
+// above the panel) and T, or with T_out null T^-1 as the merged trailing pass
+// takes it -- or -1, declined, with nothing written.  Every
 // workgroup returns the same (one that gives up waiting sets flags bit 3,
 // which fails the call).
 template <int QH, int NW, bool GRID>
 __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, double tau_dm,
                                          int truncate, double beta0, double* tau, double* V,
-                                         int ldv, int z0, double* T_out, double* slots, int nwg,
-                                         int wg, DevState* st, RegPanelLds<QH, NW>& L) {
+                                         int ldv, int z0, double* T_out, double* S_out,
+                                         double* slots, int nwg, int wg, DevState* st,
+                                         RegPanelLds<QH, NW>& L) {
   constexpr int WR = 16 * QH, NQ = 4 * QH, NT = 64 * (NW + 1);
   const int tid = local_tid(), lane = tid & 63, g = lane >> 4, li = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -415,7 +417,7 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
       }
     }
   if (wg != 0) return k;
-  inverse_merge<false>(L.S, L.X, L.Y);  // T = (striu(V^T V) + diag(1 / tau))^-1
+  if (T_out) inverse_merge(L.S, L.X, L.Y);  // T = (striu(V^T V) + diag(1 / tau))^-1
   const int tid2 = local_tid();
   for (int e = tid2; e < KMAX * KMAX; e += NT) {
     const int r = e & 63, c = e >> 6;
@@ -425,7 +427,10 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
       V[(size_t)c * ldv + r] = c < k ? (r > c ? v : (r == c ? 1.0 : 0.0)) : 0.0;
     }
     if (r < z0) V[(size_t)c * ldv + r - z0] = 0.0;
-    T_out[r + c * KMAX] = r <= c && c < k ? L.X[r][c] : 0.0;
+    if (T_out)
+      T_out[r + c * KMAX] = r <= c && c < k ? L.X[r][c] : 0.0;
+    else
+      S_out[r + c * KMAX] = c < k ? (r < c ? L.S[r][c] : (r == c ? L.tau[c] : 0.0)) : 0.0;
   }
   if (tid2 < k) tau[tid2] = L.tau[tid2];
   return k;
@@ -457,8 +462,10 @@ __global__ __launch_bounds__(64 * (NW + 1)) void k_panel_reg(double* A, int lda,
   if (wg >= nwg) return;  // the grid is sized for the lowest j
   const double beta0 = truncate == 2 ? st->pan_beta : 0.0;
   const int k = reg_panel<QH, NW, GRID>(A + j + (size_t)j * lda, lda, msub, fjb, tau_dm, truncate,
-                                        beta0, tau, V + j, ldv, min(j, KMAX), ws_mat(st, WS_T),
-                                        ws_slots(st), nwg, wg, st, L);
+                                        beta0, tau, V + j, ldv, min(j, KMAX),
+                                        mode != RUN_ALWAYS && st->fused ? nullptr
+                                                                        : ws_mat(st, WS_T),
+                                        ws_mat(st, WS_S), ws_slots(st), nwg, wg, st, L);
   if (wg == 0 && threadIdx.x == 0) {
     if (k < 0) {
       atomicOr(&st->flags, 4);
@@ -531,7 +538,11 @@ __global__ __launch_bounds__(1024) void k_panel_slow(double* A, int lda, int j, 
     __syncthreads();
   }
   larft_recurrence(Ss, Ts, ts, tmp, k);
-  for (int e = tid; e < KMAX * KMAX; e += 1024) ws_mat(st, WS_T)[e] = Ts[e];
+  for (int e = tid; e < KMAX * KMAX; e += 1024) {
+    const int r = e & 63, c = e >> 6;
+    ws_mat(st, WS_T)[e] = Ts[e];
+    ws_mat(st, WS_S)[e] = c < k ? (r < c ? Ss[e] : (r == c ? ts[c] : 0.0)) : 0.0;
+  }
   if (tid == 0) {
     if (truncate != 2) st->pan_beta = A[(size_t)j * lda + j];
     st->fjb_cmp = k;

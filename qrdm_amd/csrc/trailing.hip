@@ -34,28 +34,28 @@ namespace qrdm {
 
 constexpr int FU_CH = 32;         // rows per chunk: two interleaved 16-row tiles
 constexpr int FU_NWG = 4;         // waves per workgroup
-constexpr int FU_MAX_SPLIT = 16;  // row slabs of the partial products
-constexpr int FU_OCC = 2;         // workgroups per CU (64 KB of LDS, 256 registers a lane)
+constexpr int FU_MAX_SPLIT = 32;  // row slabs of the partial products at most
+constexpr int FU_GC = 16 * FU_NWG;  // columns of a workgroup
+constexpr int FU_OCC = 2;         // workgroups per CU (64 KB of LDS each)
 
 // Two doubles at any multiple of eight bytes (a column of any leading dimension).
 typedef double fu_pair __attribute__((ext_vector_type(2), aligned(8)));
 
 // Geometry of one fused pass over rows [r_lo, m) and columns [c0, n):
 // chunks of FU_CH rows from the FU_CH-row boundary at or below r_lo, split into
-// ns slabs of whole chunks, and column groups of gc columns.
+// ns slabs of whole chunks, and column groups of FU_GC columns.
 struct FuGeom {
   int base, nchunk, slab_ch, cgroups;
 };
 
-__host__ __device__ __forceinline__ FuGeom fused_geom(int r_lo, int m, int c0, int n, int ns,
-                                                      int gc) {
+__host__ __device__ __forceinline__ FuGeom fused_geom(int r_lo, int m, int c0, int n, int ns) {
   FuGeom g;
   g.base = r_lo & ~(FU_CH - 1);
   g.nchunk = (m - g.base + FU_CH - 1) / FU_CH;
   if (g.nchunk < 0) g.nchunk = 0;
   g.slab_ch = (g.nchunk + ns - 1) / ns;
   if (g.slab_ch < 1) g.slab_ch = 1;
-  g.cgroups = (n - c0 + gc - 1) / gc;
+  g.cgroups = (n - c0 + FU_GC - 1) / FU_GC;
   if (g.cgroups < 0) g.cgroups = 0;
   return g;
 }
@@ -72,21 +72,64 @@ __host__ __device__ __forceinline__ int fused_per_xcd(int ns, int cgroups) {
 // line: no bank conflicts in either product.
 typedef double2 FuChunk[KMAX][FU_CH / 2];
 
+// The step's T^-1 (ws_mat WS_S) and tau from k_v2's partial V^T V, after a
+// Gram-based panel: eight entries of the upper triangle at a time per
+// workgroup, the slabs over 32 threads each; every workgroup of the launch
+// takes its share.
+__device__ __forceinline__ void sum_gram(const DevState* st, int m) {
+  __shared__ double part[FU_NWG][8];
+  if (!st->fast || (st->flags & 2)) return;
+  DevState* ws = const_cast<DevState*>(st);  // the workspace's head
+  const double* __restrict__ p = ws_slots(ws);
+  const int j = st->j, k = st->fjb_cmp, nslab = (m - j + PR_ROWS - 1) / PR_ROWS;
+  const int tid = local_tid(), el = tid & 7, sl = tid >> 3;
+  for (int b = blockIdx.x; b < 288; b += gridDim.x) {
+    // unit b: eight rows of one column on or above the diagonal; the columns
+    // 8 q .. 8 q + 7 have q + 1 units each
+    int q = 0;
+    while (b >= 4 * (q + 1) * (q + 2)) q++;
+    const int u = b - 4 * q * (q + 1);
+    const int r = 8 * (u % (q + 1)) + el, c = 8 * q + u / (q + 1), e = r + KMAX * c;
+    double s = 0.0;
+    for (int q0 = sl; q0 < nslab; q0 += 128) {
+      double v[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        v[q] = p[(size_t)(q0 + 32 * q < nslab ? q0 + 32 * q : sl) * KMAX * KMAX + e];
+#pragma unroll
+      for (int q = 0; q < 4; q++) s += q0 + 32 * q < nslab ? v[q] : 0.0;
+    }
+    s += __shfl_xor(s, 8, 64);
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if ((tid & 63) < 8) part[tid >> 6][el] = s;
+    lds_barrier();
+    if (tid < 8) {
+      const double x = (part[0][el] + part[1][el]) + (part[2][el] + part[3][el]);
+      const bool diag = r == c && c < k;
+      const double v = c < k && r < c ? x : (diag ? 2.0 / x : 0.0);
+      ws_mat(ws, WS_S)[e] = v;
+      if (diag) st->tau_base[j + r] = v;
+    }
+    lds_barrier();
+  }
+}
+
 // One pass.  APPLY: C -= Vp Wprev (Vp, Wprev of the previous step) before
 // the products; ACCUM: Wp[slab] = Vn^T C.  Rows [r_lo, m) of columns
 // [c0, n) are written (APPLY only).
 //
 // What bounds it: the FP64 matrix cores (64 cycles per 16 x 16 x 4 product, 256
 // flops per 16 bytes of C with 64 columns of V), if loads, LDS and barriers
-// stay out of their way.  A wave owns 16 U columns and a chunk of 32 rows is two
+// stay out of their way.  A wave owns 16 columns and a chunk of 32 rows is two
 // 16-row tiles, even rows and odd rows: a lane's two consecutive rows are one
-// 16-byte element of C and one 16-byte unit of V, so one LDS read feeds 2 U
+// 16-byte element of C and one 16-byte unit of V, so one LDS read feeds two
 // products and independent accumulators keep the cores busy.  The tile
 // of C in the output layout of product 1 is the B operand of product 2.  The
 // next chunk of V goes from memory straight to the other LDS buffer and the
-// next chunk of C to registers while this one is multiplied (64 U products per
+// next chunk of C to registers while this one is multiplied (64 products per
 // wave and barrier), so nothing waits for a load issued in the same chunk.
-// Measured: the first pass at 8192 x 8192 325 us, 53 TF/s, the matrix cores busy
+// Measured: the first pass at 8192 x 8192 317 us, 54 TF/s, the matrix cores busy
 // in 72 % of the cycles (2.23 GHz under this load); per 8192 x 8192
 // factorisation 17.2 ms against 18.2 with 16-row chunks, V stored to LDS
 // through registers and a barrier every 32 products, 16384 x 1024 1.36 against
@@ -94,19 +137,27 @@ typedef double2 FuChunk[KMAX][FU_CH / 2];
 // against the three-kernel form with 8-byte loads).
 //
 // V is zero above its panel (within 64 rows) and past m, which the callers
-// keep so: no masks in the products, only the stores look at r_lo and m.  W
-// and the partials have leading dimension n (absolute columns); ns slabs.
-// With st (the DM loop) r_lo, c0 and the buffers come from st; the grid is
-// sized for the lowest j and surplus workgroups return.
-template <bool APPLY, bool ACCUM, int U>
+// keep so: no masks in the products, only the stores look at r_lo and m.  W is
+// indexed by absolute columns; the partials, ns slabs, by the columns from the
+// host's c0 on (a narrow C leaves room for more slabs).  With st (the DM loop)
+// r_lo, c0 and the buffers come from st; the grid is sized for the lowest j and
+// surplus workgroups return.
+//
+// On the way, beside the first loads, the workgroups sum V^T V of a Gram-based
+// panel from k_v2's slabs (fixed order) into the step's T^-1, and tau_i =
+// 2 / S_ii from it: the pass needs neither, its end needs both, and a launch of
+// their own with the inverse took 14 us a step.  (The reconstruction's own tau
+// and T agree with these only to about eps times the square of the panel's
+// condition number; the block reflector has to be orthogonal for the V stored.)
+template <bool APPLY, bool ACCUM>
 __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int lda, int r_lo, int m,
                                                                int c0, int n, StepBufs bufs,
                                                                double* Wp, int ns, int cur,
                                                                const DevState* st) {
-  constexpr int WC = 16 * U, GC = FU_NWG * WC;
   // the chunks of V_s and V_{s+1}, two buffers each (arrays of their own, so
   // that a load on its way into one does not hold up reads of the other)
   __shared__ FuChunk vp0, vp1, vn0, vn1;
+  const int cw = c0, ldw = n - c0;  // the partials' columns
   if (st) {
     if (dm_stopped(st)) return;
     r_lo = st->j;
@@ -117,43 +168,36 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   const double* Vn = bufs.V + (size_t)cur * bufs.vstride;
   const double* Vp = bufs.V + (size_t)(cur ^ 1) * bufs.vstride;
   const double* Wprev = bufs.W + (size_t)(cur ^ 1) * bufs.wstride;
-  const FuGeom G = fused_geom(r_lo, m, c0, n, ns, GC);
+  const FuGeom G = fused_geom(r_lo, m, c0, n, ns);
   const int per = fused_per_xcd(ns, G.cgroups);
   const int xcd = blockIdx.x & 7, kx = blockIdx.x >> 3;
-  if (kx >= per) return;
   const int slab = kx % ns, cgrp = xcd + 8 * (kx / ns);
-  if (cgrp >= G.cgroups) return;
+  const bool active = kx < per && cgrp < G.cgroups;
+  if (!active) {
+    if (ACCUM && st) sum_gram(st, m);
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, li = lane & 15;
   const int ncol = n - c0;
-  const int cbw = cgrp * GC + wave * WC;  // this wave's columns (relative to c0)
+  const int cbw = cgrp * FU_GC + wave * 16;  // this wave's columns (relative to c0)
   const int ch0 = slab * G.slab_ch;
   const int ch1 = min(ch0 + G.slab_ch, G.nchunk);
-  // the wave's columns c0 + cbw + 16u + li (past ncol: a valid column, never stored)
-  double* Cc[U];
-  bool cok[U];
-#pragma unroll
-  for (int u = 0; u < U; u++) {
-    const int c = cbw + 16 * u + li;
-    cok[u] = c < ncol;
-    Cc[u] = A + (size_t)(c0 + (cok[u] ? c : (ncol > 0 ? ncol - 1 : 0))) * lda;
-  }
-  // the previous step's W tile, negated: wr[s][u] = -W(4s + g, column 16u + li)
-  // (lane group g takes the k index 4s + g of step s of product 1)
-  double wr[16][U];
+  // the lane's column c0 + cbw + li (past ncol: a valid column, never stored)
+  const bool cok = cbw + li < ncol;
+  double* Cc = A + (size_t)(c0 + min(cbw + li, ncol - 1)) * lda;
+  // the previous step's W tile, negated: wr[s] = -W(4s + g, column li) (lane
+  // group g takes the k index 4s + g of step s of product 1)
+  double wr[16];
   if (APPLY) {
 #pragma unroll
-    for (int u = 0; u < U; u++)
-#pragma unroll
-      for (int s = 0; s < 16; s++)
-        wr[s][u] = cok[u] ? -Wprev[(size_t)(c0 + cbw + 16 * u + li) * KMAX + 4 * s + g] : 0.0;
+    for (int s = 0; s < 16; s++)
+      wr[s] = cok ? -Wprev[(size_t)(c0 + cbw + li) * KMAX + 4 * s + g] : 0.0;
   }
-  dbl4 acc[4][U];
+  dbl4 acc[4];
 #pragma unroll
-  for (int t = 0; t < 4; t++)
-#pragma unroll
-    for (int u = 0; u < U; u++) acc[t][u] = (dbl4){0.0, 0.0, 0.0, 0.0};
+  for (int t = 0; t < 4; t++) acc[t] = (dbl4){0.0, 0.0, 0.0, 0.0};
   // chunk c of V into LDS: a wave takes the columns 16 w .. 16 w + 15, four
   // per load (lane: column lane / 16, unit lane % 16): the lane's byte offsets
   // from the wave's first column
@@ -171,35 +215,29 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
           (__attribute__((address_space(3))) void*)&S[16 * wave + 4 * i][0], 16, 0, 0);
   };
   // chunk c of C as it lies in memory: rows base + 32c + 8v + 2g + (0, 1) in
-  // x[u][v] (taken apart into the tiles where they are used: a move here would
+  // x[v] (taken apart into the tiles where they are used: a move here would
   // wait for the load)
-  auto load_c = [&](int c, fu_pair (&x)[U][4]) {
+  auto load_c = [&](int c, fu_pair (&x)[4]) {
     const int r0 = G.base + FU_CH * c;
     if (r0 + FU_CH <= m) {
 #pragma unroll
-      for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-          x[u][v] = *reinterpret_cast<const fu_pair*>(Cc[u] + r0 + 8 * v + 2 * g);
+      for (int v = 0; v < 4; v++)
+        x[v] = *reinterpret_cast<const fu_pair*>(Cc + r0 + 8 * v + 2 * g);
     } else {
-#pragma unroll
-      for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-#pragma unroll
-          for (int h = 0; h < 2; h++) x[u][v][h] = Cc[u][min(r0 + 8 * v + 2 * g + h, m - 1)];
-    }
-  };
-  // One chunk: the next one's loads, product 1 and the store of its rows,
-  // product 2.  Tile h of C: rows 8v + 2g + h in cc[h][u][v].
-  auto step = [&](int c, FuChunk& sp, FuChunk& sn, FuChunk& np, FuChunk& nn, fu_pair (&x)[U][4]) {
-    dbl4 cc[2][U];
-#pragma unroll
-    for (int u = 0; u < U; u++)
 #pragma unroll
       for (int v = 0; v < 4; v++)
 #pragma unroll
-        for (int h = 0; h < 2; h++) cc[h][u][v] = x[u][v][h];
+        for (int h = 0; h < 2; h++) x[v][h] = Cc[min(r0 + 8 * v + 2 * g + h, m - 1)];
+    }
+  };
+  // One chunk: the next one's loads, product 1 and the store of its rows,
+  // product 2.  Tile h of C: rows 8v + 2g + h in cc[h][v].
+  auto step = [&](int c, FuChunk& sp, FuChunk& sn, FuChunk& np, FuChunk& nn, fu_pair (&x)[4]) {
+    dbl4 cc[2];
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) cc[h][v] = x[v][h];
     if (c + 1 < ch1) {
       if (APPLY) load_v(Vp, np, c + 1);
       if (ACCUM) load_v(Vn, nn, c + 1);
@@ -209,145 +247,116 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
 #pragma unroll
       for (int s = 0; s < 16; s++) {
         const double2 a = sp[4 * s + g][li ^ (4 * (s & 3) + g)];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          cc[0][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, wr[s][u], cc[0][u], 0, 0, 0);
-          cc[1][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, wr[s][u], cc[1][u], 0, 0, 0);
-        }
+        cc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, wr[s], cc[0], 0, 0, 0);
+        cc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, wr[s], cc[1], 0, 0, 0);
       }
       const int r0 = G.base + FU_CH * c;
       if (r0 >= r_lo && r0 + FU_CH <= m) {
+        if (cok) {
 #pragma unroll
-        for (int u = 0; u < U; u++)
-          if (cok[u]) {
+          for (int v = 0; v < 4; v++)
+            *reinterpret_cast<fu_pair*>(Cc + r0 + 8 * v + 2 * g) = (fu_pair){cc[0][v], cc[1][v]};
+        }
+      } else if (cok) {
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-              *reinterpret_cast<fu_pair*>(Cc[u] + r0 + 8 * v + 2 * g) =
-                  (fu_pair){cc[0][u][v], cc[1][u][v]};
-          }
-      } else {
+        for (int v = 0; v < 4; v++)
 #pragma unroll
-        for (int u = 0; u < U; u++)
-          if (cok[u]) {
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-#pragma unroll
-              for (int h = 0; h < 2; h++) {
-                const int r = r0 + 8 * v + 2 * g + h;
-                if (r >= r_lo && r < m) Cc[u][r] = cc[h][u][v];
-              }
+          for (int h = 0; h < 2; h++) {
+            const int r = r0 + 8 * v + 2 * g + h;
+            if (r >= r_lo && r < m) Cc[r] = cc[h][v];
           }
       }
     }
     if (ACCUM) {
 #pragma unroll
       for (int v = 0; v < 4; v++) {
+        double2 a[4];
 #pragma unroll
-        for (int tp = 0; tp < 4; tp += 2) {
-          double2 a[2];
+        for (int t = 0; t < 4; t++) a[t] = sn[16 * t + li][(g + 4 * v) ^ li];
 #pragma unroll
-          for (int t = 0; t < 2; t++) a[t] = sn[16 * (tp + t) + li][(g + 4 * v) ^ li];
+        for (int t = 0; t < 4; t++)
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t].x, cc[0][v], acc[t], 0, 0, 0);
 #pragma unroll
-          for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-              for (int u = 0; u < U; u++)
-                acc[tp + t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                    h ? a[t].y : a[t].x, cc[h][u][v], acc[tp + t][u], 0, 0, 0);
-        }
+        for (int t = 0; t < 4; t++)
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t].y, cc[1][v], acc[t], 0, 0, 0);
       }
     }
     __syncthreads();  // the next chunk of V is in LDS (every load has arrived)
   };
-  fu_pair x[U][4];
+  fu_pair x[4];
   if (ch1 > ch0) {
     if (APPLY) load_v(Vp, vp0, ch0);
     if (ACCUM) load_v(Vn, vn0, ch0);
     load_c(ch0, x);
   }
+  if (ACCUM && st) sum_gram(st, m);
   __syncthreads();
 #pragma clang loop unroll(disable)
   for (int c = ch0; c < ch1; c += 2) {
     step(c, vp0, vn0, vp1, vn1, x);
     if (c + 1 < ch1) step(c + 1, vp1, vn1, vp0, vn0, x);
   }
-  if (!ACCUM) return;
-  // partial tile: row 16t + g + 4w, column 16u + li of the wave's columns
-  double* out = Wp + (size_t)slab * KMAX * n;
+  if (!ACCUM || !cok) return;
+  // partial tile: row 16t + g + 4w of the lane's column
+  double* out = Wp + (size_t)slab * KMAX * ldw + (c0 + cbw + li - cw);
 #pragma unroll
-  for (int u = 0; u < U; u++) {
-    if (!cok[u]) continue;
-    const int col = c0 + cbw + 16 * u + li;
+  for (int t = 0; t < 4; t++)
 #pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int w = 0; w < 4; w++) out[(size_t)(16 * t + g + 4 * w) * n + col] = acc[t][u][w];
-  }
-}
-
-static int fused_gc(int u) { return FU_NWG * 16 * u; }
-
-// Row slabs of a fused pass with column groups of 64 u columns: one round of
-// workgroups on every XCD (its column groups times the slabs within an eighth
-// of the chip's slots) where the column groups allow it.
-static int fused_slabs_u(int r_lo, int m, int c0, int n, int u) {
-  const FuGeom g = fused_geom(r_lo, m, c0, n, 1, fused_gc(u));
-  if (g.cgroups <= 0 || g.nchunk <= 0) return 1;
-  int ns = (32 * FU_OCC) / ((g.cgroups + 7) / 8);
-  if (ns > FU_MAX_SPLIT) ns = FU_MAX_SPLIT;
-  if (ns > g.nchunk) ns = g.nchunk;
-  return ns < 1 ? 1 : ns;
-}
-
-// 16-column blocks per wave: two, unless one fills more of the chip's slots.
-// A full round of two runs at 53 TF/s (8192 x 8192, 72 % of the matrix cores'
-// cycles), one of one about a tenth slower, so one is taken where two would
-// leave more than a tenth of the slots of one empty (narrow C, or a last
-// column group per XCD that is mostly missing).
-static int fused_u(int r_lo, int m, int c0, int n) {
-  const int w1 = ((n - c0 + 63) / 64) * fused_slabs_u(r_lo, m, c0, n, 1);
-  const int w2 = ((n - c0 + 127) / 128) * fused_slabs_u(r_lo, m, c0, n, 2);
-  return 10 * w2 >= 9 * w1 ? 2 : 1;
+    for (int w = 0; w < 4; w++) out[(size_t)(16 * t + g + 4 * w) * ldw] = acc[t][w];
 }
 
 int fused_max_slabs() { return FU_MAX_SPLIT; }
 
+// Row slabs of a fused pass, at most one round of the chip's 64 workgroups per
+// XCD (two per CU), the count with the least cost in chunks: a slab's chunks
+// and two for its start and its partial tile, 1.7 times as long with a second
+// workgroup on the CU, and a twentieth per slab for the step's end.  Measured
+// (us by workgroups per XCD, 4096 x 4096): 32 87, 48 104, 56 92, 64 79;
+// 16384 x 512: 16 87, 32 50, 64 49; 1024 x 1024: 16 16, 32 12, 64 15.  (Waves of
+// 32 columns: 312 against 317 at 8192 x 8192, 169 against 160 at 8192 x 4096;
+// groups of 96 or 128 columns were slower throughout.)
 int fused_slabs(int r_lo, int m, int c0, int n) {
-  return fused_slabs_u(r_lo, m, c0, n, fused_u(r_lo, m, c0, n));
-}
-
-template <int U>
-static void launch_fused_u(double* A, int lda, int r_lo, int m, int c0, int n,
-                           const StepBufs& bufs, double* Wp, int ns, int apply, int accum,
-                           int cur, hipStream_t s, const DevState* st) {
-  const FuGeom g = fused_geom(r_lo, m, c0, n, ns, fused_gc(U));
-  const dim3 grid(8 * fused_per_xcd(ns, g.cgroups)), block(64 * FU_NWG);
-  if (apply && accum)
-    hipLaunchKernelGGL((k_fused<true, true, U>), grid, block, 0, s, A, lda, r_lo, m, c0, n, bufs,
-                       Wp, ns, cur, st);
-  else if (accum)
-    hipLaunchKernelGGL((k_fused<false, true, U>), grid, block, 0, s, A, lda, r_lo, m, c0, n,
-                       bufs, Wp, ns, cur, st);
-  else
-    hipLaunchKernelGGL((k_fused<true, false, U>), grid, block, 0, s, A, lda, r_lo, m, c0, n,
-                       bufs, Wp, ns, cur, st);
+  const FuGeom g = fused_geom(r_lo, m, c0, n, 1);
+  if (g.cgroups <= 0 || g.nchunk <= 0) return 1;
+  const int per = (g.cgroups + 7) / 8;
+  int cap = (int)(16LL * n / (n - c0));  // Wp holds 16 x 64 x n values
+  if (cap > FU_MAX_SPLIT) cap = FU_MAX_SPLIT;
+  if (cap > g.nchunk) cap = g.nchunk;
+  int best = 1;
+  double least = 1e30;
+  for (int ns = 1; ns <= cap; ns++) {
+    if (ns > 1 && per * ns > 32 * FU_OCC) break;
+    const double chunks = (g.nchunk + ns - 1) / ns + 2.0;
+    const double cost = (per * ns > 32 ? 1.7 : 1.0) * chunks + 0.05 * ns;
+    if (cost < least) {
+      least = cost;
+      best = ns;
+    }
+  }
+  return best;
 }
 
 void launch_fused(double* A, int lda, int r_lo, int m, int c0, int n, const StepBufs& bufs,
                   double* Wp, int ns, int apply, int accum, int cur, hipStream_t s,
                   const DevState* st) {
   if (n - c0 <= 0 || m - r_lo <= 0 || !(apply || accum)) return;
-  if (fused_u(r_lo, m, c0, n) == 2)
-    launch_fused_u<2>(A, lda, r_lo, m, c0, n, bufs, Wp, ns, apply, accum, cur, s, st);
+  const FuGeom g = fused_geom(r_lo, m, c0, n, ns);
+  const dim3 grid(8 * fused_per_xcd(ns, g.cgroups)), block(64 * FU_NWG);
+  if (apply && accum)
+    hipLaunchKernelGGL((k_fused<true, true>), grid, block, 0, s, A, lda, r_lo, m, c0, n, bufs, Wp,
+                       ns, cur, st);
+  else if (accum)
+    hipLaunchKernelGGL((k_fused<false, true>), grid, block, 0, s, A, lda, r_lo, m, c0, n, bufs,
+                       Wp, ns, cur, st);
   else
-    launch_fused_u<1>(A, lda, r_lo, m, c0, n, bufs, Wp, ns, apply, accum, cur, s, st);
+    hipLaunchKernelGGL((k_fused<true, false>), grid, block, 0, s, A, lda, r_lo, m, c0, n, bufs,
+                       Wp, ns, cur, st);
 }
 
 // ---------------------------------------------------------------------------
-// The end of a fused step, one 64-column tile of [j + kk, n) per workgroup
+// The end of a fused step, one 16-column tile of [j + kk, n) per workgroup
 // (256 threads): W = T^T sum_slab Wp (the fused pass's partials, summed in
-// slab order; zero for the columns below c0, which the exact panel's dlarf_
+// slab order; zero for the columns below c0, which the column-by-column panel
 // already updated), the step's R12 rows R12 = C_top - V_top W (rows j..j+kk,
 // final, written), then the norm downdate of src/dgeqrdm_work.c:80-109 from
 // them: s = sum of the kk squares (as the reference's loop, :84-86), temp =
@@ -357,118 +366,155 @@ void launch_fused(double* A, int lda, int r_lo, int m, int c0, int n, const Step
 // matrix cores) and its W column is zero, so the next fused pass leaves it --
 // otherwise work *= sqrt(temp).  The running max into st (maxnrm).  W goes to
 // the step's W buffer.
-__global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, int n,
-                                                   const double* __restrict__ T,
+//
+// Latency bounds it: one round of loads, then a chain of products.  Tiles of
+// 16 columns instead of 64 give every CU a workgroup from 4096 columns on and
+// a quarter of the loads in flight per thread; T is not formed: T^-T W = P is
+// solved by blocks of 16 rows with the inverses of T^-1's diagonal blocks, 40
+// products of one wave, whose output layout is the next one's operand layout.
+constexpr int WN_TC = 16;
+
+__global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, int n, int cw,
                                                    const double* __restrict__ Wp, int ns,
                                                    StepBufs bufs, double* work, double* workold,
                                                    DevState* st, double tol3z) {
-  __shared__ double S0[KMAX][LDP];  // T; V's top rows; V chunks of the recompute
-  __shared__ double S1[KMAX][LDP];  // the partials' sum, then W
-  __shared__ double S2[KMAX][LDP];  // C's top rows, then R12; C chunks of the recompute
-  __shared__ double s_ss[4][KMAX];  // per-wave sums of squares of the recomputed columns
-  __shared__ double s_wk[KMAX], s_wo[KMAX];  // work, workold of the tile's columns
+  __shared__ double Us[KMAX][LDP];             // T^-1
+  __shared__ double Di[KMAX][LDP];             // the inverses of its diagonal blocks
+  __shared__ double S1[KMAX][WN_TC + 1];       // the partials' sum, then W
+  __shared__ double s_rd[KMAX];
+  __shared__ double s_ss[4][WN_TC];
+  __shared__ double s_wk[WN_TC], s_wo[WN_TC];  // work, workold of the tile's columns
   __shared__ unsigned long long s_rows[4];
-  __shared__ int s_rec[KMAX];
-  __shared__ int s_any;
+  __shared__ int s_rec[WN_TC];
   if (dm_stopped(st)) return;
   // the step's end is pending from here on (run by the next k_topk or k_step_end)
   if (blockIdx.x == 0 && threadIdx.x == 0) st->pend = 1;
   const int j = st->j, kk = st->fjb_cmp, c0 = st->c0;
   const int jn = j + kk;
-  const int cb = jn + blockIdx.x * KMAX;
+  const int cb = jn + blockIdx.x * WN_TC;
   if (cb >= n) return;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = lane >> 4, li = lane & 15;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, li = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const double* V = v_cur(bufs, st);
   double* W = w_cur(bufs, st);
-  const int ldv = bufs.ldv;
-  // every global read of the prologue in flight together: T, the norms, the
-  // top rows of C and V, and the slab partials (two slabs per round)
-  if (tid < KMAX) {
-    const int col = cb + tid;
-    s_wk[tid] = col < n ? work[col] : 0.0;
-    s_wo[tid] = col < n ? workold[col] : 1.0;
+  const int ldv = bufs.ldv, ldw = n - cw;
+  const int col = cb + li, cl = min(col, n - 1);  // the lane's column
+  // every global read of the prologue in flight together: T^-1, the first
+  // slabs' partials (thread: column li, rows i0 + 16 q), V's and C's top rows
+  double us[KMAX * KMAX / 256];
+#pragma unroll
+  for (int q = 0; q < KMAX * KMAX / 256; q++) us[q] = ws_mat(st, WS_S)[tid + 256 * q];
+  const int i0 = tid >> 4;
+  const double* wp = Wp + (size_t)i0 * ldw + cl - cw;
+  constexpr int YB = 8;  // slabs per round
+  double pv[YB][4];
+  auto load_p = [&](int y0) {
+#pragma unroll
+    for (int y = 0; y < YB; y++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        pv[y][q] = wp[((size_t)min(y0 + y, ns - 1) * KMAX + 16 * q) * ldw];
+  };
+  load_p(0);
+  // V(j + 16 wv + li, 4t + g): product operand; C's rows 16 wv + g + 4v
+  double va[KMAX / 4];
+  const int rt = 16 * wv + li;
+#pragma unroll
+  for (int t = 0; t < KMAX / 4; t++)
+    va[t] = rt < kk ? -V[(size_t)(4 * t + g) * ldv + j + rt] : 0.0;
+  dbl4 r12;
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    const int r = 16 * wv + g + 4 * v;
+    r12[v] = r < kk ? A[(size_t)cl * lda + j + r] : 0.0;
+  }
+  if (tid < WN_TC) {
+    s_wk[tid] = cb + tid < n ? work[cb + tid] : 0.0;
+    s_wo[tid] = cb + tid < n ? workold[cb + tid] : 1.0;
     s_rec[tid] = 0;
   }
-  load_mat(S0, T);
+#pragma unroll
+  for (int q = 0; q < KMAX * KMAX / 256; q++) {
+    const int e = tid + 256 * q, r = e & 63, c = e >> 6;
+    Us[r][c] = us[q];
+    if (r == c) s_rd[r] = us[q];
+  }
+  lds_barrier();
+  // one wave inverts the diagonal blocks while the others wait for their loads
+  if (wv == 3) diag_inverse(Us, s_rd, Di);
   {
-    const int c = tid & 63, i0 = tid >> 6, col = cb + c;
-    const bool in = col >= c0 && col < n;
-    const int cl = col < n ? col : n - 1;
-    double sum[16];
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int y0 = 0; y0 < ns; y0 += YB) {
 #pragma unroll
-    for (int q = 0; q < 16; q++) sum[q] = 0.0;
-    for (int y = 0; y < ns; y += 2) {
-      const int y2 = (y + 1 < ns) ? y + 1 : y;
-      double a0[16], a1[16];
+      for (int y = 0; y < YB; y++)
 #pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const int i = i0 + 4 * q;
-        a0[q] = Wp[((size_t)y * KMAX + i) * n + cl];
-        a1[q] = Wp[((size_t)y2 * KMAX + i) * n + cl];
-      }
+        for (int q = 0; q < 4; q++) sum[q] += y0 + y < ns ? pv[y][q] : 0.0;
+      if (y0 + YB < ns) load_p(y0 + YB);
+    }
+    const int c = tid & 15;
+    const bool in = cb + c >= c0 && cb + c < n;
 #pragma unroll
-      for (int q = 0; q < 16; q++) {
-        sum[q] += a0[q];
-        if (y + 1 < ns) sum[q] += a1[q];
+    for (int q = 0; q < 4; q++) S1[i0 + 16 * q][c] = in ? sum[q] : 0.0;
+  }
+  lds_barrier();
+  if (wv == 0) {
+    // W_i = D_i^T (P_i - sum_{k < i} U_ki^T W_k), D_i the inverse of U_ii;
+    // w[i][v]: row 16 i + g + 4 v
+    dbl4 w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      dbl4 p;
+#pragma unroll
+      for (int v = 0; v < 4; v++) p[v] = S1[16 * i + g + 4 * v][li];
+#pragma unroll
+      for (int k = 0; k < i; k++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          p = __builtin_amdgcn_mfma_f64_16x16x4f64(-Us[16 * k + g + 4 * v][16 * i + li], w[k][v],
+                                                   p, 0, 0, 0);
+      w[i] = (dbl4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int r = g + 4 * v;
+        const double d = r <= li ? Di[16 * i + r][16 * i + li] : 0.0;
+        w[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(d, p[v], w[i], 0, 0, 0);
       }
     }
 #pragma unroll
-    for (int q = 0; q < 16; q++) S1[i0 + 4 * q][c] = in ? sum[q] : 0.0;
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) S1[16 * i + g + 4 * v][li] = w[i][v];
   }
   lds_barrier();
-  dbl4 acc[4];
-  mfma_64(acc, S0, true, S1);  // T^T S1
-  // V's top rows and C's top rows (rows j..j+kk) while the product runs
-  double vt[KMAX * KMAX / 256], ct[KMAX * KMAX / 256];
 #pragma unroll
-  for (int q = 0; q < KMAX * KMAX / 256; q++) {
-    const int e = tid + 256 * q, r = e & 63, cc = e >> 6;
-    vt[q] = (r < kk) ? V[(size_t)cc * ldv + j + r] : 0.0;  // V(j + r, cc)
-    ct[q] = (r < kk && cb + cc < n) ? A[(size_t)(cb + cc) * lda + j + r] : 0.0;
-  }
-  lds_barrier();
-  mfma_store(S1, acc);  // S1 = W
+  for (int t = 0; t < KMAX / 4; t++)
+    r12 = __builtin_amdgcn_mfma_f64_16x16x4f64(va[t], S1[4 * t + g][li], r12, 0, 0, 0);
+  double sq = 0.0;
 #pragma unroll
-  for (int q = 0; q < KMAX * KMAX / 256; q++) {
-    const int e = tid + 256 * q, r = e & 63, cc = e >> 6;
-    S0[r][cc] = vt[q];
-    S2[r][cc] = ct[q];
+  for (int v = 0; v < 4; v++) {
+    const int r = 16 * wv + g + 4 * v;
+    if (r < kk && col < n) A[(size_t)col * lda + j + r] = r12[v];
+    sq = r < kk ? fma(r12[v], r12[v], sq) : sq;
   }
-  lds_barrier();
-  mfma_64(acc, S0, false, S1);  // V_top W
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) S2[16 * wv + g + 4 * v][16 * u + li] -= acc[u][v];
-  lds_barrier();
-  for (int q = 0; q < KMAX * KMAX / 256; q++) {
-    const int e = tid + 256 * q, r = e & 63, cc = e >> 6;
-    if (r < kk && cb + cc < n) A[(size_t)(cb + cc) * lda + j + r] = S2[r][cc];
-  }
-  // norm downdate: the sum of squares of column c's kk R12 entries as four
-  // partial sums (rows p, p + 4, ...; thread p * 64 + c) added in a fixed order
-  {
-    const int c = tid & 63, p = tid >> 6;
-    double sq = 0.0;
-    for (int r = p; r < kk; r += 4) sq = fma(S2[r][c], S2[r][c], sq);
-    s_ss[p][c] = sq;
-  }
-  if (tid == 0) s_any = 0;
+  // norm downdate: the sum of squares of column c's kk R12 entries, four
+  // waves' parts added in a fixed order
+  sq += __shfl_xor(sq, 16, 64);
+  sq += __shfl_xor(sq, 32, 64);
+  if (g == 0) s_ss[wv][li] = sq;
   lds_barrier();
   double mx = 0.0;
-  if (tid < KMAX) {
-    const int c = tid, col = cb + c;
+  if (tid < WN_TC) {
+    const int c = tid;
     const double wk = s_wk[c];
-    if (col < n && wk != 0.0) {
-      const double sq = (s_ss[0][c] + s_ss[1][c]) + (s_ss[2][c] + s_ss[3][c]);
-      double temp = sqrt(fabs(sq)) / wk;
+    if (cb + c < n && wk != 0.0) {
+      const double s2 = (s_ss[0][c] + s_ss[1][c]) + (s_ss[2][c] + s_ss[3][c]);
+      double temp = sqrt(fabs(s2)) / wk;
       const double d2 = (temp + 1.0) * (1.0 - temp);
       temp = (0.0 >= d2) ? 0.0 : d2;
       const double d1 = wk / s_wo[c];
       const double temp2 = temp * (d1 * d1);
       if (temp2 <= tol3z) {
         s_rec[c] = 1;
-        s_any = 1;
       } else {
         const double nw = wk * sqrt(temp);
         s_wk[c] = nw;
@@ -477,74 +523,59 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
     }
   }
   lds_barrier();
+  const bool rec = s_rec[li] != 0;
   unsigned long long rows = 0;
-  if (s_any) {
+  if (__any(rec)) {
     // the recomputed columns take the update on rows [jn, m) now.  Each wave
     // runs its own 16-row blocks (rows jn + 16 wv, then every 64th): D =
     // V_blk W on the matrix cores, V read straight into the A operand, W from
-    // LDS, no workgroup barrier inside the loop.  Lane (g, li) keeps the sums
-    // of squares of columns 16 u + li over its rows g + 4 v of each block.
-    bool fl[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) fl[u] = s_rec[16 * u + li] != 0;
-    double ps[4] = {0.0, 0.0, 0.0, 0.0};
+    // LDS, no workgroup barrier inside the loop.  Lane (g, li) keeps the sum
+    // of squares of its column over its rows g + 4 v of each block.
+    double ps = 0.0;
     for (int rb = jn + 16 * wv; rb < m; rb += 4 * 16) {
       const int ra = rb + li;  // the lane's row of the A operand
-      double va[KMAX / 4];
+      double vb[KMAX / 4];
 #pragma unroll
       for (int t = 0; t < KMAX / 4; t++)
-        va[t] = (ra < m) ? V[(size_t)(4 * t + g) * ldv + ra] : 0.0;  // V(ra, 4t + g)
-      double cv[4][4];
+        vb[t] = (ra < m) ? -V[(size_t)(4 * t + g) * ldv + ra] : 0.0;  // V(ra, 4t + g)
+      dbl4 d;
 #pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int r = rb + g + 4 * v;
-          cv[u][v] = (fl[u] && r < m) ? A[(size_t)(cb + 16 * u + li) * lda + r] : 0.0;
-        }
-      dbl4 d[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) d[u] = (dbl4){0.0, 0.0, 0.0, 0.0};
+      for (int v = 0; v < 4; v++) {
+        const int r = rb + g + 4 * v;
+        d[v] = (rec && r < m) ? A[(size_t)cl * lda + r] : 0.0;
+      }
 #pragma unroll
       for (int t = 0; t < KMAX / 4; t++)
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(vb[t], S1[4 * t + g][li], d, 0, 0, 0);
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-          d[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[t], S1[4 * t + g][16 * u + li], d[u], 0,
-                                                      0, 0);
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int r = rb + g + 4 * v;
-          if (fl[u] && r < m) {
-            const double x = cv[u][v] - d[u][v];
-            A[(size_t)(cb + 16 * u + li) * lda + r] = x;
-            ps[u] = fma(x, x, ps[u]);
-          }
+      for (int v = 0; v < 4; v++) {
+        const int r = rb + g + 4 * v;
+        if (rec && r < m) {
+          A[(size_t)cl * lda + r] = d[v];
+          ps = fma(d[v], d[v], ps);
         }
+      }
     }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      double x = ps[u];
-      x += __shfl_xor(x, 16, 64);
-      x += __shfl_xor(x, 32, 64);
-      if (g == 0) s_ss[wv][16 * u + li] = x;
-    }
-    lds_barrier();
+    ps += __shfl_xor(ps, 16, 64);
+    ps += __shfl_xor(ps, 32, 64);
+    lds_barrier();  // the downdate's sums are read
+    if (g == 0) s_ss[wv][li] = ps;
+    // the columns' updated rows, for a norm taken again below
+    __syncthreads();
     // norms of the recomputed columns (the scaled form where the plain sum
     // of squares leaves the safe range, as dnrm2's scaling does)
     const int mrem = m - jn;
-    for (int q = 0; q < 16; q++) {
-      const int c = 16 * wv + q, col = cb + c;
-      if (!s_rec[c] || col >= n) continue;
-      const double sq = (s_ss[0][c] + s_ss[1][c]) + (s_ss[2][c] + s_ss[3][c]);
+    for (int q = 0; q < WN_TC / 4; q++) {
+      const int c = (WN_TC / 4) * wv + q;
+      if (!s_rec[c] || cb + c >= n) continue;
+      const double s2 = (s_ss[0][c] + s_ss[1][c]) + (s_ss[2][c] + s_ss[3][c]);
       double nr;
       if (mrem <= 0) nr = 0.0;
-      else if (sq >= 1e-280 && sq <= 1e280) nr = sqrt(sq);
-      else nr = wave_nrm2(A + (size_t)col * lda + jn, mrem);
+      else if (s2 >= 1e-280 && s2 <= 1e280) nr = sqrt(s2);
+      else nr = wave_nrm2(A + (size_t)(cb + c) * lda + jn, mrem);
       if (lane == 0) {
         s_wk[c] = nr;
-        workold[col] = nr;
+        workold[cb + c] = nr;
       }
       if (nr == nr) mx = fmax(mx, nr);
       rows += (unsigned long long)(mrem > 0 ? mrem : 0);
@@ -552,10 +583,11 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
   }
   lds_barrier();
   // the tile's norms, and its W (zero for the recomputed columns), column-major
-  if (tid < KMAX && cb + tid < n) work[cb + tid] = s_wk[tid];
-  for (int q = 0; q < KMAX * KMAX / 256; q++) {
-    const int e = tid + 256 * q, i = e & 63, c = e >> 6;
-    if (cb + c < n) W[(size_t)(cb + c) * KMAX + i] = s_rec[c] ? 0.0 : S1[i][c];
+  if (tid < WN_TC && cb + tid < n) work[cb + tid] = s_wk[tid];
+#pragma unroll
+  for (int q = 0; q < WN_TC / 4; q++) {
+    const int c = wv + 4 * q;
+    if (cb + c < n) W[(size_t)(cb + c) * KMAX + lane] = s_rec[c] ? 0.0 : S1[lane][c];
   }
   if (lane == 0) s_rows[wv] = rows;
   // (a lane of wave 0 holds its own column's norm: the wave's maximum goes in)
@@ -569,12 +601,13 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
 void launch_wsum_norm(double* A, int lda, int j0, int m, int n, const double* T,
                       const double* Wp, int ns, const StepBufs& bufs, double* work,
                       double* workold, DevState* st, double tol3z, hipStream_t s) {
+  (void)T;  // the step's T^-1 lies behind the state (ws_mat WS_S)
   // tiles of [j + kk, n), j + kk >= j0 + 1; one workgroup at least (it marks
-  // the step's end pending)
-  int tiles = (n - j0 - 1 + KMAX - 1) / KMAX;
+  // the step's end pending).  The pass's partials start at column j0 + 1.
+  int tiles = (n - j0 - 1 + WN_TC - 1) / WN_TC;
   if (tiles < 1) tiles = 1;
-  hipLaunchKernelGGL(k_wsum_norm, dim3(tiles), dim3(256), 0, s, A, lda, m, n, T, Wp, ns, bufs,
-                     work, workold, st, tol3z);
+  hipLaunchKernelGGL(k_wsum_norm, dim3(tiles), dim3(256), 0, s, A, lda, m, n, j0 + 1, Wp, ns,
+                     bufs, work, workold, st, tol3z);
 }
 
 }  // namespace qrdm
