@@ -545,7 +545,6 @@ int run_dm(const Args& x) {
     }
     HIPCHK(hipMemcpyAsync(B.jp, x.jpvt, sizeof(int) * n, hipMemcpyHostToDevice, s));
     launch_dm_begin(B.st, nfxd, minmn, tau_dm, delta, fused_now ? 1 : 0, s);
-    const int batch = x.trace ? 1 : kBatch;
     int j0 = nfxd, it = 0;
     // the column-by-column panel of the step at column jl, with V and T
     // (RUN_EXACT: it runs when the step's panel is not the Gram-based one, or
@@ -625,6 +624,15 @@ int run_dm(const Args& x) {
       HIPCHK(hipMemcpyAsync(hb[q], B.st, sizeof(DevState), hipMemcpyDeviceToHost, s));
       if (evs) HIPCHK(hipEventRecord(evs[q], s));
     };
+    // Steps of a batch from column jl: as many as blocks of nb columns need to
+    // end the loop, and one more where several do (the truncation shortens
+    // blocks now and then), at most kBatch.  A step queued past the end still
+    // costs its eight launches, 20 us: 64 x 48 takes 1 step, not 8.
+    auto batch_steps = [&](int jl) {
+      if (x.trace) return 1;
+      const int blocks = (minmn - jl + nb - 1) / nb;
+      return std::min(kBatch, blocks > 1 ? blocks + 1 : 1);
+    };
     auto queue_batch = [&](int jl, int q) {
       // Tall panels: Gram-based Householder reconstruction (panel.hip), which
       // also leaves V and T for the trailing update, its first Cholesky beside
@@ -633,8 +641,10 @@ int run_dm(const Args& x) {
       // halts until the host resumes it.  Short panels: the column-by-column
       // exact panel, then dlarft.
       const bool tall = m - jl >= kFastPanelRows && !force_exact;
-      for (int b = 0; b < batch; b++) queue_step(jl, tall);
+      const int steps = batch_steps(jl);
+      for (int b = 0; b < steps; b++) queue_step(jl, tall);
       readback(q);
+      return steps;
     };
     auto wait_slot = [&](int q) {
       if (evs) HIPCHK(hipEventSynchronize(evs[q]));
@@ -646,10 +656,10 @@ int run_dm(const Args& x) {
     // is queued before its state is read back, so the device does not idle
     // through the readback; its grids are sized from the same lower bound.
     int q = 0, jend = j0;
-    queue_batch(j0, q);
+    int steps = queue_batch(j0, q);  // of the batch waited for
     while (true) {
-      const bool ahead = !x.trace && !switch_wanted && j0 + batch * KMAX < minmn;
-      if (ahead) queue_batch(j0, q ^ 1);
+      const bool ahead = !x.trace && !switch_wanted && j0 + steps * KMAX < minmn;
+      const int steps_ahead = ahead ? queue_batch(j0, q ^ 1) : 0;
       DevState* h = wait_slot(q);
       check_panels(h->flags);
       bool in_flight = ahead;
@@ -696,6 +706,7 @@ int run_dm(const Args& x) {
         switch_wanted = true;
       if (in_flight) {
         q ^= 1;  // the batch queued ahead is the one to wait for next
+        steps = steps_ahead;
       } else {
         if (switch_wanted) {
           // the pending merged update reaches rows and columns >= j0 (the
@@ -710,7 +721,7 @@ int run_dm(const Args& x) {
           prec_now = low;
           switch_wanted = false;
         }
-        queue_batch(j0, q);
+        steps = queue_batch(j0, q);
       }
     }
     if (fused_now && it > 0) {
