@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <climits>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -821,26 +822,80 @@ int guarded(const Args& x) {
 }  // namespace
 
 namespace {
-// Copies a column-major host block into a fresh device block (ld rounded up).
+// A column-major block on the device, packed (leading dimension = rows), and
+// its copies from and to host memory.  Packed host blocks move in one copy.
+// Others go through a buffer of the call's own, kStage bytes at a time, so
+// that the rows between the block's columns are neither read into the device
+// nor written: hipMemcpy2D moves pageable memory row by row (1024 x 512: 4.7 ms
+// in and 3.7 ms out, packed or not, against 0.13 and 0.24 ms for one copy).
 struct DevBlock {
+  static constexpr size_t kStage = (size_t)8 << 20;
   double* p = nullptr;
-  int ld = 0;
+  int rows = 0, cols = 0;
+  DevBlock() = default;
+  DevBlock(const DevBlock&) = delete;
+  DevBlock& operator=(const DevBlock&) = delete;
   ~DevBlock() {
     if (p) (void)hipFree(p);
   }
+  void alloc(int r, int c) {
+    rows = r;
+    cols = c;
+    HIPCHK(hipMalloc(&p, sizeof(double) * (size_t)(r > 0 ? r : 1) * (c > 0 ? c : 1)));
+  }
+  void from_host(const double* h, int ld) {
+    if (rows <= 0 || cols <= 0) return;
+    if (ld == rows || cols == 1) {
+      HIPCHK(hipMemcpy(p, h, sizeof(double) * (size_t)rows * cols, hipMemcpyHostToDevice));
+      return;
+    }
+    const int step = stage_cols();
+    std::vector<double> buf((size_t)step * rows);
+    for (int c = 0; c < cols; c += step) {
+      const int nc = std::min(step, cols - c);
+      for (int i = 0; i < nc; i++)
+        memcpy(&buf[(size_t)i * rows], h + (size_t)(c + i) * ld, sizeof(double) * rows);
+      HIPCHK(hipMemcpy(p + (size_t)c * rows, buf.data(), sizeof(double) * (size_t)rows * nc,
+                       hipMemcpyHostToDevice));
+    }
+  }
+  void to_host(double* h, int ld) const {
+    if (rows <= 0 || cols <= 0) return;
+    if (ld == rows || cols == 1) {
+      HIPCHK(hipMemcpy(h, p, sizeof(double) * (size_t)rows * cols, hipMemcpyDeviceToHost));
+      return;
+    }
+    const int step = stage_cols();
+    std::vector<double> buf((size_t)step * rows);
+    for (int c = 0; c < cols; c += step) {
+      const int nc = std::min(step, cols - c);
+      HIPCHK(hipMemcpy(buf.data(), p + (size_t)c * rows, sizeof(double) * (size_t)rows * nc,
+                       hipMemcpyDeviceToHost));
+      for (int i = 0; i < nc; i++)
+        memcpy(h + (size_t)(c + i) * ld, &buf[(size_t)i * rows], sizeof(double) * rows);
+    }
+  }
+
+ private:
+  int stage_cols() const {
+    const size_t c = kStage / (sizeof(double) * (size_t)rows);
+    return c < 1 ? 1 : (c < (size_t)cols ? (int)c : cols);
+  }
 };
-void to_device(DevBlock& b, const double* h, int ldh, int rows, int cols) {
-  b.ld = ((rows + 31) / 32) * 32;
-  if (b.ld < 32) b.ld = 32;
-  HIPCHK(hipMalloc(&b.p, sizeof(double) * (size_t)b.ld * (cols > 0 ? cols : 1)));
-  if (rows > 0 && cols > 0)
-    HIPCHK(hipMemcpy2D(b.p, sizeof(double) * b.ld, h, sizeof(double) * ldh,
-                       sizeof(double) * rows, cols, hipMemcpyHostToDevice));
-}
-void to_host(double* h, int ldh, const DevBlock& b, int rows, int cols) {
-  if (rows > 0 && cols > 0)
-    HIPCHK(hipMemcpy2D(h, sizeof(double) * ldh, b.p, sizeof(double) * b.ld,
-                       sizeof(double) * rows, cols, hipMemcpyDeviceToHost));
+
+// Runs a host-pointer entry point: a device error or a failed host allocation
+// becomes a return code and its text (no exception leaves the C ABI).
+template <typename F>
+int host_call(F f) {
+  try {
+    return f();
+  } catch (const HipError& e) {
+    g_err = std::string(e.what) + ": " + hipGetErrorString(e.e);
+    return -1000 - (int)e.e;
+  } catch (const std::bad_alloc&) {
+    g_err = "host memory for the copies";
+    return -1000 - (int)hipErrorOutOfMemory;
+  }
 }
 }  // namespace
 
@@ -1069,19 +1124,18 @@ int qrdm_dgeqrf(int m, int n, double* a, int lda, double* tau) {
   if (m < 0 || n < 0 || lda < (m > 1 ? m : 1)) return -1;
   if (m == 0 || n == 0) return 0;
   const int k = m < n ? m : n;
-  try {
+  return host_call([&] {
     DevBlock da, dt;
-    to_device(da, a, lda, m, n);
-    to_device(dt, tau, k, k, 1);
-    int info = qrdm_dgeqrf_dev(m, n, da.p, da.ld, dt.p, nullptr);
+    da.alloc(m, n);
+    dt.alloc(k, 1);
+    da.from_host(a, lda);
+    dt.from_host(tau, k);
+    int info = qrdm_dgeqrf_dev(m, n, da.p, m, dt.p, nullptr);
     if (info != 0) return info;
-    to_host(a, lda, da, m, n);
-    to_host(tau, k, dt, k, 1);
+    da.to_host(a, lda);
+    dt.to_host(tau, k);
     return 0;
-  } catch (const HipError& e) {
-    g_err = std::string(e.what) + ": " + hipGetErrorString(e.e);
-    return -1000 - (int)e.e;
-  }
+  });
 }
 
 int qrdm_dormqr(int trans, int m, int n, int k, const double* a, int lda, const double* tau,
@@ -1089,19 +1143,19 @@ int qrdm_dormqr(int trans, int m, int n, int k, const double* a, int lda, const 
   if (m < 0 || n < 0 || k < 0 || k > m || lda < (m > 1 ? m : 1) || ldc < (m > 1 ? m : 1))
     return -1;
   if (m == 0 || n == 0 || k == 0) return 0;
-  try {
+  return host_call([&] {
     DevBlock da, dt, dc;
-    to_device(da, a, lda, m, k);
-    to_device(dt, tau, k, k, 1);
-    to_device(dc, c, ldc, m, n);
-    int info = qrdm_dormqr_dev(trans, m, n, k, da.p, da.ld, dt.p, dc.p, dc.ld, nullptr);
+    da.alloc(m, k);
+    dt.alloc(k, 1);
+    dc.alloc(m, n);
+    da.from_host(a, lda);
+    dt.from_host(tau, k);
+    dc.from_host(c, ldc);
+    int info = qrdm_dormqr_dev(trans, m, n, k, da.p, m, dt.p, dc.p, m, nullptr);
     if (info != 0) return info;
-    to_host(c, ldc, dc, m, n);
+    dc.to_host(c, ldc);
     return 0;
-  } catch (const HipError& e) {
-    g_err = std::string(e.what) + ": " + hipGetErrorString(e.e);
-    return -1000 - (int)e.e;
-  }
+  });
 }
 
 int dgeqrdm(int matrix_layout, int m, int n, double* a, int lda, int* jpvt, double* tau,
@@ -1110,38 +1164,23 @@ int dgeqrdm(int matrix_layout, int m, int n, double* a, int lda, int* jpvt, doub
   int bad = check_args(x);
   if (bad) return bad;
   const int minmn = m < n ? m : n;
-  double *d_a = nullptr, *d_tau = nullptr;
-  int ldd = ((m + 31) / 32) * 32;
-  try {
-    HIPCHK(hipMalloc(&d_a, sizeof(double) * (size_t)ldd * n));
-    HIPCHK(hipMalloc(&d_tau, sizeof(double) * (size_t)minmn));
-    HIPCHK(hipMemcpy2D(d_a, sizeof(double) * ldd, a, sizeof(double) * lda, sizeof(double) * m, n,
-                       hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(d_tau, tau, sizeof(double) * minmn, hipMemcpyHostToDevice));
-  } catch (const HipError& e) {
-    g_err = std::string(e.what) + ": " + hipGetErrorString(e.e);
-    if (d_a) (void)hipFree(d_a);
-    if (d_tau) (void)hipFree(d_tau);
-    return -1000 - (int)e.e;
-  }
-  x.a = d_a;
-  x.lda = ldd;
-  x.tau = d_tau;
-  int info = guarded(x);
-  if (info > -1000) {
-    hipError_t e1 = hipMemcpy2D(a, sizeof(double) * lda, d_a, sizeof(double) * ldd,
-                                sizeof(double) * m, n, hipMemcpyDeviceToHost);
-    hipError_t e2 = hipMemcpy(tau, d_tau, sizeof(double) * minmn, hipMemcpyDeviceToHost);
-    if (e1 != hipSuccess || e2 != hipSuccess) {
-      g_err = std::string("copy back: ") + hipGetErrorString(e1 != hipSuccess ? e1 : e2);
-      info = -1000 - (int)(e1 != hipSuccess ? e1 : e2);
+  return host_call([&] {
+    DevBlock da, dt;
+    da.alloc(m, n);
+    dt.alloc(minmn, 1);
+    da.from_host(a, lda);
+    dt.from_host(tau, minmn);
+    x.a = da.p;
+    x.lda = m;
+    x.tau = dt.p;
+    const int info = guarded(x);
+    if (info > -1000) {
+      da.to_host(a, lda);
+      dt.to_host(tau, minmn);
     }
-  }
-  (void)hipFree(d_a);
-  (void)hipFree(d_tau);
-  return info;
+    return info;
+  });
 }
-
 
 qrdm_batch_plan* qrdm_batch_plan_create(int count, const qrdm_batch_item* items, int nb) {
   std::lock_guard<std::mutex> lk(g_mu);
