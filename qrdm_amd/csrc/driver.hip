@@ -362,6 +362,7 @@ int run_wide(const Args& x, Buffers& B, int nfxd, double eta, int enable_stop, d
     // column right of it (the block's own later ones included) before the
     // next; the part that the truncation ends is the last
     int kk = 0;
+    if (it == 0) launch_zero(B.V, sizeof(double) * (size_t)B.ldv * KMAX, s);  // rows from m on
     for (int i0 = 0; i0 < fjb; i0 += KMAX) {
       const int kb = std::min(KMAX, fjb - i0), jp = j + i0;
       launch_panel_exact(A, lda, jp, m, kb, tau_dm, i0 == 0 ? 1 : 2, x.tau + jp,
@@ -756,6 +757,8 @@ int run_dm(const Args& x) {
 // KMAX columns, each followed by its block update of the columns to the right.
 void blocked_qr(double* A, int lda, int m, int n, int ncols_qr, double* tau, Buffers& B,
                 hipStream_t s) {
+  // the panels write V's rows below m only; the merged passes read whole chunks
+  launch_zero(B.V, sizeof(double) * (size_t)B.ldv * KMAX, s);
   for (int j = 0; j < ncols_qr; j += KMAX) {
     const int kb = (ncols_qr - j) < KMAX ? (ncols_qr - j) : KMAX;
     launch_panel_exact(A, lda, j, m, kb, 0.0, 0, tau + j, B.st, s);  // V and T too
@@ -782,16 +785,23 @@ int run_ormqr(int trans, int m, int n, int k, const double* A, int lda, const do
   workspace_for(m, n, &B);
   HIPCHK(hipMemsetAsync(B.st, 0, sizeof(DevState), s));
   const int nblk = (k + KMAX - 1) / KMAX;
+  // Each block's update is merged with the next block's product, as the DM
+  // loop's steps are (trailing.hip): one pass over C per block.
+  const StepBufs bufs{B.V, (size_t)B.ldv * KMAX, B.ldv, B.Wf, (size_t)KMAX * n};
+  int jp = 0;
   for (int q = 0; q < nblk; q++) {
     const int b = trans ? q : nblk - 1 - q;  // Q^T: H(0) first; Q: H(k-1) first
-    const int j = b * KMAX;
+    const int j = b * KMAX, cur = b & 1;
     const int kb = (k - j) < KMAX ? (k - j) : KMAX;
-    launch_set_kk(B.st, kb, s);
-    launch_build_v(A, lda, j, m, B.ldv, B.st, B.V, B.ldv, s);
-    launch_gram(B.V, B.ldv, j, m, nullptr, KMAX, nullptr, B.gram_part, B.S, s);
-    launch_larft(B.S, tau + j, B.st, B.T, s);
-    launch_larfb(C, ldc, j, m, 0, n, B.V, B.ldv, B.T, trans, B.Wp, B.W, B.nsplit, s);
+    launch_panel_exact(const_cast<double*>(A), lda, j, m, kb, 0.0, PANEL_GIVEN,
+                       const_cast<double*>(tau) + j, B.st, s);
+    const int r = q > 0 ? std::min(j, jp) : j, ns = fused_slabs(r, m, 0, n);
+    launch_fused(C, ldc, r, m, 0, n, bufs, B.Wp, ns, q > 0, 1, cur, s, B.st);
+    launch_wsum(j, m, 0, n, nullptr, trans, B.Wp, B.Wf + cur * bufs.wstride, ns, s, B.st);
+    jp = j;
   }
+  launch_fused(C, ldc, jp, m, 0, n, bufs, B.Wp, fused_slabs(jp, m, 0, n), 1, 0,
+               ((jp / KMAX) & 1) ^ 1, s, nullptr);
   HIPCHK(hipStreamSynchronize(s));
   return 0;
 }

@@ -521,95 +521,6 @@ __device__ __forceinline__ void gram_tiles(const dbl4 (&xb)[4], dbl4 (&gt)[10]) 
     }
 }
 
-__device__ __forceinline__ void gram_slab_mfma(const double* X, double* out) {
-  dbl4 acc[4];
-#pragma unroll
-  for (int u = 0; u < 4; u++) acc[u] = (dbl4){0.0, 0.0, 0.0, 0.0};
-  gram_slab_acc(X, acc);
-  gram_store(acc, out);
-}
-
-// ---------------------------------------------------------------------------
-// Gram matrix of up to 64 columns over a row range: partial sums per
-// GRAM_ROWS-row slab, then a fixed-order reduction.  Used for the candidate
-// cosines (cblas_dsyrk, src/dgeqrdm_work.c:376-379) and for V^T V (dlarft).
-__global__ __launch_bounds__(256) void k_gram_partial(const double* __restrict__ base, int ld,
-                                                      int r0, int r1,
-                                                      const int* __restrict__ cols,
-                                                      int ncols_max,
-                                                      const int* __restrict__ ncols_dev,
-                                                      double* partial, const DevState* st,
-                                                      int mode) {
-  __shared__ double X[KMAX * (GRAM_ROWS + 1)];
-  if (!step_runs(st, mode)) return;
-  if (mode == RUN_DM) {  // the step's candidates: columns and rows from j
-    base += (size_t)st->j * ld;
-    r0 = st->j;
-  } else if (mode != RUN_ALWAYS) {
-    r0 = st->j;
-  }
-  const int nc = ncols_dev ? *ncols_dev : ncols_max;
-  // slabs past r1 (the grid is sized for the lowest j) write zero partials
-  const int rs = r0 + blockIdx.x * GRAM_ROWS;
-  // 256 threads: 16 elements each, all loads issued before the LDS writes
-  double xv[KMAX * GRAM_ROWS / 256];
-#pragma unroll
-  for (int q = 0; q < KMAX * GRAM_ROWS / 256; q++) {
-    const int t = threadIdx.x + 256 * q;
-    const int c = t / GRAM_ROWS, r = t % GRAM_ROWS;
-    const bool ok = c < nc && rs + r < r1;
-    const int cc = ok ? (cols ? cols[c] : c) : 0;
-    xv[q] = ok ? base[(size_t)cc * ld + rs + r] : 0.0;
-  }
-#pragma unroll
-  for (int q = 0; q < KMAX * GRAM_ROWS / 256; q++) {
-    const int t = threadIdx.x + 256 * q;
-    X[(t / GRAM_ROWS) * (GRAM_ROWS + 1) + t % GRAM_ROWS] = xv[q];
-  }
-  __syncthreads();
-  gram_slab_mfma(X, partial + (size_t)blockIdx.x * KMAX * KMAX);
-}
-
-__global__ __launch_bounds__(256) void k_gram_reduce(const double* __restrict__ partial,
-                                                     int nslab, double* G,
-                                                     const DevState* st, int mode) {
-  __shared__ double part[4][64];
-  if (!step_runs(st, mode)) return;
-  const int e = blockIdx.x * 64 + (threadIdx.x & 63);
-  // entries below the diagonal take the value of their mirror: G is exactly
-  // symmetric, the upper triangle as dsyrk('U') forms it
-  const int pr = e & 63, pc = e >> 6;
-  const int es = (pr > pc) ? pc + pr * KMAX : e;
-  const int q = threadIdx.x >> 6;
-  // slabs q, q+4, ... summed eight loads at a time (index clamped, surplus masked)
-  double s = 0.0;
-  for (int b0 = q; b0 < nslab; b0 += 32) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int b = b0 + 4 * u;
-      v[u] = partial[(size_t)(b < nslab ? b : q) * KMAX * KMAX + es];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; u++) s += (b0 + 4 * u < nslab) ? v[u] : 0.0;
-  }
-  part[q][threadIdx.x & 63] = s;
-  __syncthreads();
-  if (q == 0) G[e] = (part[0][threadIdx.x] + part[1][threadIdx.x]) +
-                     (part[2][threadIdx.x] + part[3][threadIdx.x]);
-}
-
-void launch_gram(const double* base, int ld, int r0, int r1, const int* cols, int ncols_max,
-                 const int* ncols_dev, double* partial, double* G, hipStream_t s,
-                 const DevState* st, int mode) {
-  int nslab = (r1 - r0 + GRAM_ROWS - 1) / GRAM_ROWS;
-  if (nslab < 1) nslab = 1;
-  hipLaunchKernelGGL(k_gram_partial, dim3(nslab), dim3(256), 0, s, base, ld, r0, r1, cols,
-                     ncols_max, ncols_dev, partial, st, mode);
-  hipLaunchKernelGGL(k_gram_reduce, dim3(KMAX * KMAX / 64), dim3(256), 0, s, partial, nslab, G,
-                     st, mode);
-}
-
 // ---------------------------------------------------------------------------
 // The end of DM_perm (src/dgeqrdm_work.c:354-418), one wave:
 // 1. greedy acceptance: the max-norm column first, then, in sorted order,
@@ -872,7 +783,7 @@ __global__ __launch_bounds__(256) void k_gram_cand(double* A, int lda, int m, do
   }
 }
 
-// The DM step's candidate Gram reduce (as k_gram_reduce, RUN_DM), then the
+// The sum of the step's candidate Grams in slab order, then the
 // last workgroup to finish (atomic ticket, reset for the next launch) runs
 // the greedy acceptance and the step's plan on it (select_wave).
 __global__ __launch_bounds__(256) void k_reduce_select(const double* __restrict__ partial,
@@ -1136,35 +1047,8 @@ __device__ __forceinline__ int panel_exact_body(double* A, int lda, int j, int m
 }
 
 // ---------------------------------------------------------------------------
-// Dense copy of the block reflector V (unit lower trapezoidal, zero padded to
-// KMAX columns and to mpad rows, zero above row j) into V[r + c*ldv].
-__global__ __launch_bounds__(256) void k_build_v(const double* __restrict__ A, int lda, int j,
-                                                 int m, int mpad, const DevState* st,
-                                                 double* V, int ldv, int mode) {
-  if (!step_runs(st, mode)) return;
-  if (mode != RUN_ALWAYS) j = st->j;
-  const int kk = st->fjb_cmp;
-  const int r = blockIdx.x * 256 + threadIdx.x;
-  if (r >= mpad) return;
-  for (int c = 0; c < KMAX; c++) {
-    double v = 0.0;
-    int rr = r - j;  // row within the panel
-    if (c < kk && r < m && rr >= c) v = (rr == c) ? 1.0 : A[(size_t)(j + c) * lda + r];
-    V[(size_t)c * ldv + r] = v;
-  }
-}
-
-void launch_build_v(const double* A, int lda, int j, int m, int mpad, const DevState* st,
-                    double* V, int ldv, hipStream_t s, int mode) {
-  hipLaunchKernelGGL(k_build_v, dim3((mpad + 255) / 256), dim3(256), 0, s, A, lda, j, m, mpad,
-                     st, V, ldv, mode);
-}
-
-// ---------------------------------------------------------------------------
 // dlarft, DIRECT='F', STOREV='C' (call site src/dgeqrdm_work.c:751-754):
 // T(0:i,i) = -tau_i T(0:i,0:i) (V^T v_i)(0:i), T(i,i) = tau_i, from S = V^T V.
-// With nslab > 0, S is first summed from nslab partial Grams (the exact
-// panel's V slabs); 256 threads, the recurrence on the first 64.
 // The recurrence for the whole workgroup (at least 64 threads): Ss = V^T V
 // and Ts (zero on entry) column-major with leading dimension KMAX, ts the
 // kk scalars tau, tmp KMAX doubles; all in LDS.
@@ -1185,45 +1069,6 @@ __device__ __forceinline__ void larft_recurrence(const double* Ss, double* Ts, c
     }
     __syncthreads();
   }
-}
-
-__global__ __launch_bounds__(256) void k_larft(const double* __restrict__ S,
-                                               const double* __restrict__ tau,
-                                               const DevState* st, double* T, int mode,
-                                               int nslab) {
-  __shared__ double Ss[KMAX * KMAX];
-  __shared__ double Ts[KMAX * KMAX];
-  __shared__ double tmp[KMAX], ts[KMAX];
-  if (!step_runs(st, mode)) return;
-  if (mode != RUN_ALWAYS) tau += st->j;
-  const int tid = threadIdx.x;
-  const int kk = st->fjb_cmp;
-  for (int e = tid; e < KMAX * KMAX; e += 256) {
-    double v = 0.0;
-    if (nslab > 0) {
-      for (int b0 = 0; b0 < nslab; b0 += 8) {  // eight loads in flight
-        double pv[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-          pv[u] = S[(size_t)(b0 + u < nslab ? b0 + u : 0) * KMAX * KMAX + e];
-#pragma unroll
-        for (int u = 0; u < 8; u++) v += (b0 + u < nslab) ? pv[u] : 0.0;
-      }
-    } else {
-      v = S[e];
-    }
-    Ss[e] = v;
-    Ts[e] = 0.0;
-  }
-  if (tid < KMAX) ts[tid] = tid < kk ? tau[tid] : 0.0;
-  __syncthreads();
-  larft_recurrence(Ss, Ts, ts, tmp, kk);
-  for (int e = tid; e < KMAX * KMAX; e += 256) T[e] = Ts[e];
-}
-
-void launch_larft(const double* S, const double* tau, const DevState* st, double* T,
-                  hipStream_t s, int mode, int nslab) {
-  hipLaunchKernelGGL(k_larft, dim3(1), dim3(256), 0, s, S, tau, st, T, mode, nslab);
 }
 
 // ---------------------------------------------------------------------------
@@ -1665,6 +1510,10 @@ void launch_wsum(int j, int m, int c0, int n, const double* T, int trans, const 
                  double* W, int nsplit, hipStream_t s, const DevState* st) {
   const int ncol = n - c0, mrow = m - j;
   if (ncol <= 0 || mrow <= 0) return;
+  if (!T) {
+    launch_wsum_fused(c0, n, nullptr, trans, Wp, W, nsplit, s, st);
+    return;
+  }
   const G1Geom g = gemm1_geom(j, m, c0, n, nsplit);
   const dim3 grid((ncol + 63) / 64);
   static_assert(G1_MAX_SPLIT == 16, "k_wsum instances cover 16 slabs");
@@ -1672,13 +1521,6 @@ void launch_wsum(int j, int m, int c0, int n, const double* T, int trans, const 
     hipLaunchKernelGGL(k_wsum<8>, grid, dim3(256), 0, s, Wp, g.ns, n, c0, ncol, T, trans, W, st);
   else
     hipLaunchKernelGGL(k_wsum<16>, grid, dim3(256), 0, s, Wp, g.ns, n, c0, ncol, T, trans, W, st);
-}
-
-void launch_larfb_w(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
-                    const double* T, int trans, double* Wp, double* W, int nsplit, hipStream_t s,
-                    const DevState* st) {
-  launch_gemm1(A, lda, j, m, c0, n, V, ldv, Wp, nsplit, s, st);
-  launch_wsum(j, m, c0, n, T, trans, Wp, W, nsplit, s, st);
 }
 
 void launch_larfb_apply(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
@@ -1693,12 +1535,6 @@ void launch_larfb_apply(double* A, int lda, int j, int m, int c0, int n, const d
   else
     hipLaunchKernelGGL(k_gemm2, dim3((mrow + 63) / 64, ctiles), dim3(256), 0, s, A, lda, j, m,
                        c0, ncol, V, ldv, W, n, st);
-}
-
-void launch_larfb(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
-                  const double* T, int trans, double* Wp, double* W, int nsplit, hipStream_t s) {
-  launch_larfb_w(A, lda, j, m, c0, n, V, ldv, T, trans, Wp, W, nsplit, s, nullptr);
-  launch_larfb_apply(A, lda, j, m, c0, n, V, ldv, W, s, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1803,12 +1639,6 @@ void launch_dm_begin(DevState* st, int j, int minmn, double tau, double delta, i
 
 // ---------------------------------------------------------------------------
 // Small helpers.
-__global__ void k_set_kk(DevState* st, int kk) { st->fjb_cmp = kk; }
-
-void launch_set_kk(DevState* st, int kk, hipStream_t s) {
-  hipLaunchKernelGGL(k_set_kk, dim3(1), dim3(1), 0, s, st, kk);
-}
-
 __global__ void k_resume(DevState* st) { st->halt = 0; }
 
 void launch_resume(DevState* st, hipStream_t s) {

@@ -1096,7 +1096,7 @@ __device__ __forceinline__ void recon_body(const double* __restrict__ G2, const 
   }
 }
 
-// G2 = the sum of pass 2's partial Grams (as k_gram_reduce), then the last
+// G2 = the sum of pass 2's partial Grams in slab order, then the last
 // workgroup to finish (atomic ticket, reset for the next launch) runs the
 // reconstruction on it.
 __global__ __launch_bounds__(256) void k_reduce_recon(const double* __restrict__ partial,
@@ -1203,6 +1203,62 @@ __global__ __launch_bounds__(256) void k_v2(double* A, int lda, int m,
   for (int p = 0; p < 10; p++) gt[p] = (dbl4p){0.0, 0.0, 0.0, 0.0};
   gram_tiles(vb, gt);
   gram_sum_store(gt, Gp, gram_part + (size_t)blockIdx.x * KMAX * KMAX);
+}
+
+// The block reflector of a factored panel (A below the diagonal, tau): the dense
+// V of columns [j, j + k) into buffer (j / KMAX) & 1 -- zero on the 64 rows above
+// the panel and from m to ws_ldv(m) -- and each 64-row slab's part of V^T V into
+// the slots, for the merged pass (trailing.hip) to sum beside its first loads.
+// One launch of up to a workgroup per 64 rows, 8 us at 4096 rows, in place of
+// four (the copy of V one row per thread over all 64 columns, the Gram from it,
+// its sum, and dlarft's recurrence in one workgroup: 147 us).
+__global__ __launch_bounds__(256) void k_given_panel(const double* __restrict__ A, int lda, int j,
+                                                     int m, int k, const double* tau,
+                                                     DevState* st) {
+  __shared__ double Gp[4][10][4][64];
+  const int tid = local_tid(), lane = tid & 63, wv = tid >> 6, g = lane >> 4, li = lane & 15;
+  const int ldv = ws_ldv(m), cur = (j / KMAX) & 1;
+  double* V = ws_v(st, m) + (size_t)cur * ldv * KMAX;
+  if (blockIdx.x == 0) {
+    if (tid == 0) {
+      st->j = j;
+      st->fjb_cmp = k;
+      st->fast = 1;
+      st->given = 1;
+      st->tau_base = const_cast<double*>(tau) - j;
+    }
+    for (int e = tid; e < KMAX * KMAX; e += 256) {
+      const int r = j - KMAX + (e & 63), c = e >> 6;
+      if (r >= 0) V[(size_t)c * ldv + r] = 0.0;
+    }
+  }
+  const int rb = j + blockIdx.x * PR_ROWS + 16 * wv;
+  dbl4p vb[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int r = rb + g + 4 * v, c = 16 * u + li;
+      const bool below = c < k && r < m && r - j > c;
+      const double x = A[(size_t)(j + (below ? c : 0)) * lda + (below ? r : j)];
+      vb[u][v] = below ? x : (c < k && r < m && r - j == c ? 1.0 : 0.0);
+    }
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      if (rb + g + 4 * v < ldv) V[(size_t)(16 * u + li) * ldv + rb + g + 4 * v] = vb[u][v];
+  dbl4p gt[10];
+#pragma unroll
+  for (int p = 0; p < 10; p++) gt[p] = (dbl4p){0.0, 0.0, 0.0, 0.0};
+  gram_tiles(vb, gt);
+  gram_sum_store(gt, Gp, ws_slots(st) + (size_t)blockIdx.x * KMAX * KMAX);
+}
+
+void launch_given_panel(const double* A, int lda, int j, int m, int k, const double* tau,
+                        DevState* st, hipStream_t s) {
+  hipLaunchKernelGGL(k_given_panel, dim3((m - j + PR_ROWS - 1) / PR_ROWS), dim3(256), 0, s, A, lda,
+                     j, m, k, tau, st);
 }
 
 // The block reflector of the Gram-based panel from the V it stored: S = V^T V

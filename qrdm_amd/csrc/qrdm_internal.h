@@ -64,6 +64,8 @@ struct DevState {
   int policy_on;      // 1: the step's tau and delta come from the learned policy
   double pan_beta;    // R(0, 0) of the last column-by-column panel (wide.hip's blocks)
   double* tau_base;   // tau[0..min(m, n)) (set by the Gram-based panel)
+  int given;          // 1: V and tau are a factored panel's (ormqr); the merged pass leaves
+                      // tau as it is and takes its geometry from the host
   double tau_step;    // tau and delta of the current step (the defaults, or the
   double delta_step;  // policy's proposal)
   StepRec last;
@@ -237,15 +239,6 @@ int topk_blocks(int n);
 void launch_topk(const double* work, int j0, int m, int n, int nb, double tau, double* tmp_val,
                  int* tmp_idx, unsigned* ticket, DevState* st, int* ncols_dev, int enable_stop,
                  double eta, hipStream_t s);
-// Gram of ncols (<= 64) columns over rows [r0, r1): columns are
-// base[(cols ? cols[c] : c) * ld + r].  partial needs ceil((r1-r0)/GRAM_ROWS)
-// * 64 * 64 doubles.  G is 64 x 64 column-major; entries beyond ncols are 0.
-// mode RUN_DM: base and r0 move by st->j columns and rows (the candidates of
-// the step); RUN_EXACT: r0 = st->j (the step's V), run only with the exact
-// panel.  r0 is then the lower bound j0.
-void launch_gram(const double* base, int ld, int r0, int r1, const int* cols, int ncols_max,
-                 const int* ncols_dev, double* partial, double* G, hipStream_t s,
-                 const DevState* st = nullptr, int mode = RUN_ALWAYS);
 // The step's candidate Gram over rows j..m (RUN_DM geometry; j0 <= j sizes
 // the grid), then, in the last workgroup of the reduce (*ticket is 0 between
 // launches), the greedy cosine acceptance and the step's plan: permute_marked's
@@ -270,24 +263,24 @@ void launch_apply_perm(double* A, int lda, int m, double* work, int* jp, const i
 // the dense V (rows max(j - KMAX, 0) .. m of ws_v, of the step's parity with
 // st->fused) and T (ws_mat), and uses the Gram partials' space.  truncate: 0
 // none, 1 the DM test, 2 the DM test of a panel that continues a wider block.
+// PANEL_GIVEN: the columns are factored already; A and tau are only read, and V
+// (of buffer j / KMAX & 1, rows up to ws_ldv(m), j a multiple of KMAX) and the
+// partial V^T V (slots) are written, from which the merged pass forms T^-1.
+constexpr int PANEL_GIVEN = 3;
 void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm,
                         int truncate, double* tau, DevState* st, hipStream_t s,
                         int mode = RUN_ALWAYS);
-void launch_build_v(const double* A, int lda, int j, int m, int mpad, const DevState* st,
-                    double* V, int ldv, hipStream_t s, int mode = RUN_ALWAYS);
-// T from S = V^T V.
-void launch_larft(const double* S, const double* tau, const DevState* st, double* T,
-                  hipStream_t s, int mode = RUN_ALWAYS, int nslab = 0);
+void launch_given_panel(const double* A, int lda, int j, int m, int k, const double* tau,
+                        DevState* st, hipStream_t s);
 // Block reflector from the left on rows [j, m), columns [c0, n):
 // trans = 1: C := (I - V T V^T)^T C (dgeqrdm's trailing update);
-// trans = 0: C := (I - V T V^T) C.
+// trans = 0: C := (I - V T V^T) C.  V is zero on the 32 rows above j and on
+// the rows from m to ldv; W holds 64 x n values.
 void launch_larfb(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
                   const double* T, int trans, double* Wp, double* W, int nsplit, hipStream_t s);
-// The two halves of launch_larfb: W = op(T) V^T C, then C -= V W.  With st
-// (the DM loop) j and c0 come from st and the host values are lower bounds.
-void launch_larfb_w(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
-                    const double* T, int trans, double* Wp, double* W, int nsplit, hipStream_t s,
-                    const DevState* st = nullptr);
+// Second half of the three-kernel trailing update (launch_gemm1 and launch_wsum
+// before it): C -= V W.  With st (the DM loop) j and c0 come from st and the host
+// values are lower bounds.
 void launch_larfb_apply(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
                         const double* W, hipStream_t s, const DevState* st = nullptr);
 // Precision of the trailing update's two products (mixed.hip): FP64 runs
@@ -334,12 +327,18 @@ void launch_policy_update(float* theta, float* m1, float* m2, const float* parti
 void launch_policy_pack(const float* theta, void* net, float tau_lo, float tau_hi,
                         float delta_lo, float delta_hi, hipStream_t s);
 void launch_policy_predict(const void* net, const float* x, int ns, float* out, hipStream_t s);
-// launch_larfb_w's two launches: the partial products Wp = V^T C per row
-// slab, then W = op(T) sum Wp.
+// The three-kernel update's first two launches: the partial products Wp = V^T C per row
+// slab, then W = op(T) sum Wp.  launch_wsum with T = nullptr: the partials
+// of a merged pass (launch_fused) over columns [c0, n), nsplit its slabs; W by
+// absolute column (KMAX x n), from the T^-1 behind st.
 void launch_gemm1(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
                   double* Wp, int nsplit, hipStream_t s, const DevState* st);
 void launch_wsum(int j, int m, int c0, int n, const double* T, int trans, const double* Wp,
                  double* W, int nsplit, hipStream_t s, const DevState* st);
+// W = op(T) sum Wp (64 x n by absolute column) from a merged pass's ns slabs over
+// columns [c0, n); T = nullptr: from the T^-1 behind st.
+void launch_wsum_fused(int c0, int n, const double* T, int trans, const double* Wp, double* W,
+                       int ns, hipStream_t s, const DevState* st);
 // Norm downdate of columns [j + fjb_cmp, n) (j, fjb_cmp from st; j0 <= j
 // sizes the grid).
 void launch_norm_update(const double* A, int lda, int j0, int m, int n, double* work,
@@ -354,7 +353,6 @@ void launch_step_end(DevState* st, int* ncols_dev, int m, int n, int enable_stop
 void launch_dm_begin(DevState* st, int j, int minmn, double tau, double delta, int fused,
                      hipStream_t s);
 
-void launch_set_kk(DevState* st, int kk, hipStream_t s);
 // ---- wide DM steps, 64 < nb <= KW (wide.hip): host-driven, one sync per step.
 // The top kmax (<= KW) of work[0..nsub) (value descending, index ascending)
 // by sort passes through the two key buffers (wide_sort_keys(n) entries

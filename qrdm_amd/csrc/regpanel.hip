@@ -565,6 +565,10 @@ __global__ __launch_bounds__(256) void k_panel_slots(DevState* st, int n, int mo
 // stay in memory.
 void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm,
                         int truncate, double* tau, DevState* st, hipStream_t s, int mode) {
+  if (truncate == PANEL_GIVEN) {
+    launch_given_panel(A, lda, j, m, fjb, tau, st, s);
+    return;
+  }
   const int rows = m - j, nwg = (rows + RP_ROWS - 1) / RP_ROWS;
   if (rows <= RP_SMALL) {
     hipLaunchKernelGGL((k_panel_reg<2, 4, false>), dim3(1), dim3(320), 0, s, A, lda, j, m, fjb,

@@ -107,9 +107,9 @@ __device__ __forceinline__ void sum_gram(const DevState* st, int m) {
     if (tid < 8) {
       const double x = (part[0][el] + part[1][el]) + (part[2][el] + part[3][el]);
       const bool diag = r == c && c < k;
-      const double v = c < k && r < c ? x : (diag ? 2.0 / x : 0.0);
-      ws_mat(ws, WS_S)[e] = v;
-      if (diag) st->tau_base[j + r] = v;
+      const double t = !diag ? 0.0 : (st->given ? st->tau_base[j + r] : 2.0 / x);
+      ws_mat(ws, WS_S)[e] = c < k && r < c ? x : t;
+      if (diag && !st->given) st->tau_base[j + r] = t;
     }
     lds_barrier();
   }
@@ -160,9 +160,11 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   const int cw = c0, ldw = n - c0;  // the partials' columns
   if (st) {
     if (dm_stopped(st)) return;
-    r_lo = st->j;
-    c0 = st->c0;
-    cur = st->it & 1;
+    if (!st->given) {
+      r_lo = st->j;
+      c0 = st->c0;
+      cur = st->it & 1;
+    }
   }
   const int ldv = bufs.ldv;
   const double* Vn = bufs.V + (size_t)cur * bufs.vstride;
@@ -374,6 +376,45 @@ void launch_fused(double* A, int lda, int r_lo, int m, int c0, int n, const Step
 // products of one wave, whose output layout is the next one's operand layout.
 constexpr int WN_TC = 16;
 
+// S1 (64 x 16): P in, W out; U = T^-1 and D the inverses of U's 16 x 16 diagonal
+// blocks; one wave.  TRANS: U^T W = P, W_i = D_i^T (P_i - sum_{k < i} U_ki^T W_k);
+// otherwise U W = P, W_i = D_i (P_i - sum_{k > i} U_ik W_k).
+template <bool TRANS>
+__device__ __forceinline__ void wy_solve(const double (*Us)[LDP], const double (*Di)[LDP],
+                                         double (*S1)[WN_TC + 1]) {
+  const int lane = local_tid() & 63, g = lane >> 4, li = lane & 15;
+  dbl4 w[4];  // w[i][v]: row 16 i + g + 4 v
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int i = TRANS ? q : 3 - q;
+    dbl4 p;
+#pragma unroll
+    for (int v = 0; v < 4; v++) p[v] = S1[16 * i + g + 4 * v][li];
+#pragma unroll
+    for (int h = 0; h < q; h++) {
+      const int k = TRANS ? h : 3 - h;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const double u = TRANS ? Us[16 * k + g + 4 * v][16 * i + li]
+                               : Us[16 * i + li][16 * k + g + 4 * v];
+        p = __builtin_amdgcn_mfma_f64_16x16x4f64(-u, w[k][v], p, 0, 0, 0);
+      }
+    }
+    w[i] = (dbl4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int r = g + 4 * v;
+      const double d = TRANS ? (r <= li ? Di[16 * i + r][16 * i + li] : 0.0)
+                             : (li <= r ? Di[16 * i + li][16 * i + r] : 0.0);
+      w[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(d, p[v], w[i], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) S1[16 * i + g + 4 * v][li] = w[i][v];
+}
+
 __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, int n, int cw,
                                                    const double* __restrict__ Wp, int ns,
                                                    StepBufs bufs, double* work, double* workold,
@@ -457,34 +498,7 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
     for (int q = 0; q < 4; q++) S1[i0 + 16 * q][c] = in ? sum[q] : 0.0;
   }
   lds_barrier();
-  if (wv == 0) {
-    // W_i = D_i^T (P_i - sum_{k < i} U_ki^T W_k), D_i the inverse of U_ii;
-    // w[i][v]: row 16 i + g + 4 v
-    dbl4 w[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      dbl4 p;
-#pragma unroll
-      for (int v = 0; v < 4; v++) p[v] = S1[16 * i + g + 4 * v][li];
-#pragma unroll
-      for (int k = 0; k < i; k++)
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-          p = __builtin_amdgcn_mfma_f64_16x16x4f64(-Us[16 * k + g + 4 * v][16 * i + li], w[k][v],
-                                                   p, 0, 0, 0);
-      w[i] = (dbl4){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int r = g + 4 * v;
-        const double d = r <= li ? Di[16 * i + r][16 * i + li] : 0.0;
-        w[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(d, p[v], w[i], 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) S1[16 * i + g + 4 * v][li] = w[i][v];
-  }
+  if (wv == 0) wy_solve<true>(Us, Di, S1);
   lds_barrier();
 #pragma unroll
   for (int t = 0; t < KMAX / 4; t++)
@@ -608,6 +622,107 @@ void launch_wsum_norm(double* A, int lda, int j0, int m, int n, const double* T,
   if (tiles < 1) tiles = 1;
   hipLaunchKernelGGL(k_wsum_norm, dim3(tiles), dim3(256), 0, s, A, lda, m, n, j0 + 1, Wp, ns,
                      bufs, work, workold, st, tol3z);
+}
+
+// W = op(T) sum_slab Wp from a merged pass, without the norm downdate: ormqr's
+// blocks (GIVEN: from T^-1 behind st, as above) and the blocks of the unpivoted
+// QR and of the wide steps (from T).  One 16-column tile per workgroup, latency
+// bound as the step's end; W by absolute column.
+template <bool GIVEN>
+__global__ __launch_bounds__(256) void k_wsum_fused(int c0, int n, const double* __restrict__ T,
+                                                    int trans, const double* __restrict__ Wp,
+                                                    int ns, double* W, const DevState* st) {
+  __shared__ double Us[KMAX][LDP];  // T^-1, or T
+  __shared__ double Di[KMAX][LDP];
+  __shared__ double S1[KMAX][WN_TC + 1];
+  __shared__ double s_rd[KMAX];
+  const int cb = c0 + blockIdx.x * WN_TC;
+  if (cb >= n) return;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, li = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ldw = n - c0;
+  const double* U = GIVEN ? ws_mat(const_cast<DevState*>(st), WS_S) : T;
+  double us[KMAX * KMAX / 256];
+#pragma unroll
+  for (int q = 0; q < KMAX * KMAX / 256; q++) us[q] = U[tid + 256 * q];
+  const int i0 = tid >> 4;
+  const double* wp = Wp + (size_t)i0 * ldw + min(cb + li, n - 1) - c0;
+  constexpr int YB = 8;  // slabs per round
+  double pv[YB][4];
+  auto load_p = [&](int y0) {
+#pragma unroll
+    for (int y = 0; y < YB; y++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        pv[y][q] = wp[((size_t)min(y0 + y, ns - 1) * KMAX + 16 * q) * ldw];
+  };
+  load_p(0);
+#pragma unroll
+  for (int q = 0; q < KMAX * KMAX / 256; q++) {
+    const int e = tid + 256 * q, r = e & 63, c = e >> 6;
+    Us[r][c] = us[q];
+    if (r == c) s_rd[r] = us[q];
+  }
+  lds_barrier();
+  if (GIVEN && wv == 3) diag_inverse(Us, s_rd, Di);
+  {
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int y0 = 0; y0 < ns; y0 += YB) {
+#pragma unroll
+      for (int y = 0; y < YB; y++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) sum[q] += y0 + y < ns ? pv[y][q] : 0.0;
+      if (y0 + YB < ns) load_p(y0 + YB);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) S1[i0 + 16 * q][li] = sum[q];
+  }
+  lds_barrier();
+  if (GIVEN) {
+    if (wv == 0) {
+      if (trans) wy_solve<true>(Us, Di, S1);
+      else wy_solve<false>(Us, Di, S1);
+    }
+  } else {
+    // rows 16 wv .. of op(T) S1
+    dbl4 w = (dbl4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < KMAX / 4; t++) {
+      const int k = 4 * t + g, r = 16 * wv + li;
+      w = __builtin_amdgcn_mfma_f64_16x16x4f64(trans ? Us[k][r] : Us[r][k], S1[k][li], w, 0, 0, 0);
+    }
+    lds_barrier();
+#pragma unroll
+    for (int v = 0; v < 4; v++) S1[16 * wv + g + 4 * v][li] = w[v];
+  }
+  lds_barrier();
+#pragma unroll
+  for (int q = 0; q < WN_TC / 4; q++) {
+    const int c = wv + 4 * q;
+    if (cb + c < n) W[(size_t)(cb + c) * KMAX + lane] = S1[lane][c];
+  }
+}
+
+void launch_wsum_fused(int c0, int n, const double* T, int trans, const double* Wp, double* W,
+                       int ns, hipStream_t s, const DevState* st) {
+  if (n - c0 <= 0) return;
+  const dim3 grid((n - c0 + WN_TC - 1) / WN_TC);
+  if (T)
+    hipLaunchKernelGGL(k_wsum_fused<false>, grid, dim3(256), 0, s, c0, n, T, trans, Wp, ns, W, st);
+  else
+    hipLaunchKernelGGL(k_wsum_fused<true>, grid, dim3(256), 0, s, c0, n, T, trans, Wp, ns, W, st);
+}
+
+// A block reflector on its own: V^T C, W = op(T) V^T C, C -= V W.
+void launch_larfb(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
+                  const double* T, int trans, double* Wp, double* W, int nsplit, hipStream_t s) {
+  (void)nsplit;  // Wp holds the slabs that fused_slabs chooses
+  if (n - c0 <= 0 || m - j <= 0) return;
+  const StepBufs bufs{const_cast<double*>(V), 0, ldv, W, 0};
+  const int ns = fused_slabs(j, m, c0, n);
+  launch_fused(A, lda, j, m, c0, n, bufs, Wp, ns, 0, 1, 0, s, nullptr);
+  launch_wsum_fused(c0, n, T, trans, Wp, W, ns, s, nullptr);
+  launch_fused(A, lda, j, m, c0, n, bufs, Wp, ns, 1, 0, 0, s, nullptr);
 }
 
 }  // namespace qrdm
