@@ -145,7 +145,8 @@ struct Buffers {
   double* M;          // 64 * 64
   double* V;          // 2 * mpad * 64: the dense V of two consecutive steps
   int ldv;
-  double* Wp;  // nsplit * 64 * n: partial products of the trailing update
+  double* Wp;  // nsplit * 64 * n: partial products of the trailing update, the wide
+               // steps' candidate Gram
   double* W;   // 64 * n: W of the three-kernel trailing update (relative to c0)
   double* Wf;  // 2 * 64 * n: W of two consecutive steps, by absolute column (fused form)
   int* perm;   // kPermInts: (dst, src) pairs, then the panel's candidate ranks
@@ -154,11 +155,10 @@ struct Buffers {
   unsigned* tickets;  // launch tickets (zero between uses): [0] top-k, [1] selection,
                       // [2] reconstruction, [3] T of the Gram-based panel
   int nsplit;
-  // wide steps (nb > KMAX) only: sort keys, the candidate Gram, the
-  // selection's output, the swap pairs
+  // wide steps (nb > KMAX) only: sort keys, the selection's output, the swap
+  // pairs
   double* wval[2] = {nullptr, nullptr};
   int* widx[2] = {nullptr, nullptr};
-  double* wG = nullptr;  // KW x KW
   int* wsel = nullptr;   // 2 + KW
   int* wpairs = nullptr;  // 4 KW
 };
@@ -197,7 +197,6 @@ size_t layout_buffers(int m, int n, char* base, Buffers* b, int nb = KMAX) {
       t.wval[q] = carve<double>(p, (size_t)wide_sort_keys(n));
       t.widx[q] = carve<int>(p, (size_t)wide_sort_keys(n));
     }
-    t.wG = carve<double>(p, (size_t)KW * KW);
     t.wsel = carve<int>(p, 2 + KW);
     t.wpairs = carve<int>(p, 4 * KW);
   }
@@ -337,8 +336,9 @@ int run_wide(const Args& x, Buffers& B, int nfxd, double eta, int enable_stop, d
     const double* val = nullptr;
     launch_topk_wide(B.work + j, nsub, kmax, B.wval, B.widx, &val, s);
     const int* idx = wide_topk_idx(B.wval, B.widx, val);
-    launch_gram_wide(A, lda, j, m, idx, kmax, B.wG, KW, s);
-    launch_select_wide(B.wG, KW, val, kmax, tau_dm, delta, B.wsel, s);
+    // (the Gram and its partial sums in Wp, free until the block's update)
+    launch_gram_wide(A, lda, j, m, idx, kmax, B.Wp, n, s);
+    launch_select_wide(B.Wp, n, val, kmax, tau_dm, delta, B.wsel, s);
     HIPCHK(hipMemcpyAsync(hout.data(), B.wsel, sizeof(int) * (2 + KW), hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(hidx.data(), idx, sizeof(int) * kmax, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));

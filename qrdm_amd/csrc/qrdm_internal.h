@@ -362,7 +362,8 @@ void launch_topk_wide(const double* work, int nsub, int kmax, double* val[2], in
                       const double** out_val, hipStream_t s);
 const int* wide_topk_idx(double* val[2], int* idx[2], const double* out_val);
 // Gram of the nc candidate columns j + idx[c] over rows [j, m) (tile pairs
-// on or above the diagonal of 64 x 64 tiles; G column-major, ld ldg).
+// on or above the diagonal of 64 x 64 tiles; G column-major, ld ldg >= nc).  G
+// holds 1024 x ldg values, those past the first KW columns scratch.
 void launch_gram_wide(const double* A, int lda, int j, int m, const int* idx, int nc, double* G,
                       int ldg, hipStream_t s);
 // out[0] = nc, out[1] = fjb, out[2 + s] = rank of the s-th accepted candidate.
