@@ -17,19 +17,20 @@
 // Row i leaves the registers when column i is done (R to the right of the
 // diagonal, V to the left), through LDS; the rest is written once, at the end,
 // with the dense V of the trailing update.  One wave that holds no rows builds
-// T's diagonal blocks from those entries beside the others' updates.  Panels of more than RP_ROWS rows take one workgroup per RP_ROWS
-// rows: every column's partial sums pass between the workgroups through
+// T's diagonal blocks from those entries beside the others' updates.  Panels of
+// more than RP_ROWS rows take a workgroup per RP_HALF (or RP_ROWS) rows: every column's partial sums pass between the workgroups through
 // memory, each a slot of its own that holds a sentinel until it is written.
 //
-// Measured for 64 columns, with V and T (rocprofv3): up to 128 rows 66 us, up
-// to 448 rows 106 us (memory-based: about 180 us for 64 rows, with T another
-// 60), 4096 rows on ten workgroups 189 us (3.8 ms).  A column costs about 2500
-// cycles at 128 rows and 3600 at 448, of which the reflector's scalars take 280;
-// between workgroups the exchange adds 3600.  The loop is unrolled over the
-// four column groups so that every register index is static: with uniform
-// branches in their place the 448-row panel took 163 us.  Unpivoted QR of 1024 x
-// 1024 15.6 -> 2.9 ms, of 4096 x 2048 129 -> 8.5 ms; 2048 x 1024 DM with
-// 128-column blocks 68.4 -> 8.8 ms; 64 x 48 DM 0.53 -> 0.33 ms.
+// Measured for 64 columns, with V and T (rocprofv3): up to 128 rows 65 us, up
+// to 448 rows 104 us (memory-based: about 180 us for 64 rows, with T another
+// 60), 1024 rows on five workgroups 136 us, 4096 rows on nineteen 160 us
+// (memory-based 3.8 ms; on ten workgroups over all XCDs 189).  A column costs
+// about 2500 cycles at 128 rows and 3600 at 448, of which the reflector's scalars
+// take 280; between workgroups the exchange adds 2000 to 2500.  The loop is
+// unrolled over the four column groups so that every register index is static:
+// with uniform branches in their place the 448-row panel took 163 us.  Unpivoted
+// QR of 1024 x 1024 15.6 -> 2.2 ms, of 4096 x 2048 129 -> 6.7 ms; 2048 x 1024 DM
+// with 128-column blocks 68.4 -> 4.2 ms; 64 x 48 DM 0.53 -> 0.21 ms.
 //
 // Sums of squares are taken plainly: where one leaves [1e-280, 1e280] (or is
 // not a number) the panel is declined before anything is written, and the
@@ -42,6 +43,12 @@ constexpr int RP_ROWS = 448;  // rows per workgroup (seven waves of 64, and the 
 constexpr int RP_SMALL = 128;  // panels up to this many rows: four waves of 32
 constexpr int RP_MID = 336;    // up to this many: seven waves of 48
 constexpr int RP_WGS = 64;     // workgroups of one panel at most
+constexpr int RP_HALF = 224;   // rows per workgroup while that leaves RP_XCD of them at most
+// Up to this many workgroups (one per CU: an XCD has 32) every eighth of the grid
+// works, which puts them on one XCD, whose L2 then carries the exchange: a round
+// among ten took 1900 cycles against 2700 over all XCDs (3000 with a fresh slot for
+// every column, which is read from memory first).  Only speed depends on it.
+constexpr int RP_XCD = 28;
 
 // A slot not yet written: a NaN pattern no published value takes (published
 // NaNs are made the canonical one).
@@ -56,7 +63,8 @@ typedef double rp_pair __attribute__((ext_vector_type(2), aligned(8)));
 template <int QH, int NW>
 struct RegPanelLds {
   double x[NW][16 * QH];        // column i's rows, per wave
-  double red[2][NW + 1][KMAX];  // partial sums, by column
+  double red[2][NW][KMAX];      // partial sums, by column
+  double all[2][NW + 2][KMAX];  // their sums over shares of the workgroups, and row i
   double row[2][KMAX];          // row i
   double out[KMAX][LDP];        // the top block: R, V below the diagonal
   double S[KMAX][LDP];          // V^T V above the diagonal, else zero
@@ -153,8 +161,10 @@ __device__ __forceinline__ bool rp_collect(const double* slots, int first, int s
 // workgroups, this one the rows from wg * 16 QH NW.  Truncation: 5e-14 is the
 // bound of the columns after the first (tau_dm > 0: tau_dm |R(0, 0)| once
 // column 0 is done), unless truncate is 0; truncate = 2: beta0 is the block's
-// R(0, 0), and every column is tested.  slots (nwg > 1): KMAX columns x
-// (nwg + 1) x KMAX values, empty on entry.  Returns the columns reduced with
+// R(0, 0), and every column is tested.  slots (nwg > 1): four columns' sets
+// of (nwg + 1) x KMAX values, empty on entry; column i uses set i mod 4 and
+// empties its own slot of column i + 2, whose values (of column i - 2) every
+// workgroup has read before any publishes column i - 1.  Returns the columns reduced with
 // everything written -- the panel, tau, rows [-z0, msub) of the dense V (zero
 // above the panel) and T, or with T_out null T^-1 as the merged trailing pass
 // takes it -- or -1, declined, with nothing written.  Every
@@ -229,15 +239,22 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
     if constexpr (GRID) {
       // this workgroup's sums (and row i, from the one that holds it) to the
       // others; wave w then collects workgroups w, w + NW + 1, ... in order
-      double* sl = slots + (size_t)i * (nwg + 1) * KMAX;
+      double* sl = slots + (size_t)(i & 3) * (nwg + 1) * KMAX;
+      double* s2 = slots + (size_t)((i + 2) & 3) * (nwg + 1) * KMAX;
+      const double none = __longlong_as_double((long long)kRpEmpty);
+      handoff_wait();  // the slot emptied a column ago is empty for everyone
       if (wave == 0) {
         double t = L.red[buf][0][lane];
 #pragma unroll
         for (int w = 1; w < NW; w++) t += L.red[buf][w][lane];
         if (rdlane(t, i) == 0.0 && rp_nonzero(&L.x[0][0], NW * WR) && lane == i) t = 1e-300;
         st_dev(sl + wg * KMAX + lane, rp_publishable(t));
+        st_dev(s2 + wg * KMAX + lane, none);
       }
-      if (wg == 0 && wave == 1) st_dev(sl + nwg * KMAX + lane, rp_publishable(L.row[buf][lane]));
+      if (wg == 0 && wave == 1) {
+        st_dev(sl + nwg * KMAX + lane, rp_publishable(L.row[buf][lane]));
+        st_dev(s2 + nwg * KMAX + lane, none);
+      }
       double t = 0.0, rr = 0.0;
       bool got = rp_collect(sl, wave, NW + 1, nwg, t);
       if (wave == NW) got &= rp_collect(sl, nwg, 1, nwg + 1, rr);
@@ -245,15 +262,19 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
         if (lane == 0) atomicOr(&st->flags, 8);  // given up: the call fails
         t = __longlong_as_double(0x7ff8000000000000ll);
       }
-      lds_barrier();  // the partial sums of this buffer are read
-      L.red[buf][wave][lane] = t;
-      if (wave == NW) L.row[buf][lane] = rr;
+      L.all[buf][wave][lane] = t;
+      if (wave == NW) L.all[buf][NW + 1][lane] = rr;
       lds_barrier();
-    }
-    rv = L.row[buf][lane];
-    sum = L.red[buf][0][lane];
+      rv = L.all[buf][NW + 1][lane];
+      sum = L.all[buf][0][lane];
 #pragma unroll
-    for (int w = 1; w < (GRID ? NW + 1 : NW); w++) sum += L.red[buf][w][lane];
+      for (int w = 1; w < NW + 1; w++) sum += L.all[buf][w][lane];
+    } else {
+      rv = L.row[buf][lane];
+      sum = L.red[buf][0][lane];
+#pragma unroll
+      for (int w = 1; w < NW; w++) sum += L.red[buf][w][lane];
+    }
   };
   // dlarfg of column i (every wave computes the same): tau, beta, 1 / (alpha -
   // beta); false ends the panel before column i.  y = 1 / sqrt(t2) by one
@@ -445,7 +466,7 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
 template <int QH, int NW, bool GRID>
 __global__ __launch_bounds__(64 * (NW + 1)) void k_panel_reg(double* A, int lda, int j, int m, int fjb,
                                                        double tau_dm, int truncate, double* tau,
-                                                       DevState* st, int mode) {
+                                                       DevState* st, int mode, int stride) {
   __shared__ RegPanelLds<QH, NW> L;
   if (!step_runs(st, mode)) return;
   const int ldv = ws_ldv(m);
@@ -458,8 +479,9 @@ __global__ __launch_bounds__(64 * (NW + 1)) void k_panel_reg(double* A, int lda,
   }
   const int msub = m - j;
   const int nwg = GRID ? (msub + 16 * QH * NW - 1) / (16 * QH * NW) : 1;
-  const int wg = blockIdx.x;
-  if (wg >= nwg) return;  // the grid is sized for the lowest j
+  const int wg = blockIdx.x / stride;
+  // one workgroup in stride works; the grid is sized for the lowest j
+  if (wg * stride != (int)blockIdx.x || wg >= nwg) return;
   const double beta0 = truncate == 2 ? st->pan_beta : 0.0;
   const int k = reg_panel<QH, NW, GRID>(A + j + (size_t)j * lda, lda, msub, fjb, tau_dm, truncate,
                                         beta0, tau, V + j, ldv, min(j, KMAX),
@@ -570,21 +592,26 @@ void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm
     return;
   }
   const int rows = m - j, nwg = (rows + RP_ROWS - 1) / RP_ROWS;
-  if (rows <= RP_SMALL) {
+  const int half = (rows + RP_HALF - 1) / RP_HALF;
+  auto grid = [&](auto kernel, int n) {
+    const int stride = n <= RP_XCD ? 8 : 1;
+    hipLaunchKernelGGL(k_panel_slots, dim3(n + 1), dim3(256), 0, s, st, 4 * KMAX * (n + 1), mode);
+    hipLaunchKernelGGL(kernel, dim3(n * stride), dim3(512), 0, s, A, lda, j, m, fjb, tau_dm,
+                       truncate, tau, st, mode, stride);
+  };
+  if (rows <= RP_SMALL)
     hipLaunchKernelGGL((k_panel_reg<2, 4, false>), dim3(1), dim3(320), 0, s, A, lda, j, m, fjb,
-                       tau_dm, truncate, tau, st, mode);
-  } else if (rows <= RP_MID) {
+                       tau_dm, truncate, tau, st, mode, 1);
+  else if (rows <= RP_MID)
     hipLaunchKernelGGL((k_panel_reg<3, 7, false>), dim3(1), dim3(512), 0, s, A, lda, j, m, fjb,
-                       tau_dm, truncate, tau, st, mode);
-  } else if (nwg == 1) {
+                       tau_dm, truncate, tau, st, mode, 1);
+  else if (nwg == 1)
     hipLaunchKernelGGL((k_panel_reg<4, 7, false>), dim3(1), dim3(512), 0, s, A, lda, j, m, fjb,
-                       tau_dm, truncate, tau, st, mode);
-  } else if (nwg <= RP_WGS) {
-    hipLaunchKernelGGL(k_panel_slots, dim3(8 * (nwg + 1)), dim3(256), 0, s, st,
-                       KMAX * KMAX * (nwg + 1), mode);
-    hipLaunchKernelGGL((k_panel_reg<4, 7, true>), dim3(nwg), dim3(512), 0, s, A, lda, j, m, fjb,
-                       tau_dm, truncate, tau, st, mode);
-  }
+                       tau_dm, truncate, tau, st, mode, 1);
+  else if (half <= RP_XCD)
+    grid(k_panel_reg<2, 7, true>, half);
+  else if (nwg <= RP_WGS)
+    grid(k_panel_reg<4, 7, true>, nwg);
   hipLaunchKernelGGL(k_panel_slow, dim3(1), dim3(1024), 0, s, A, lda, j, m, fjb, tau_dm,
                      truncate, tau, st, mode, nwg > RP_WGS ? 1 : 0);
 }
