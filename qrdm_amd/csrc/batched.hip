@@ -69,132 +69,206 @@ __device__ __forceinline__ double bt_v(const double* a, int lda, int j, int kk, 
   return rr == c ? 1.0 : a[(size_t)(j + c) * lda + row];
 }
 
-// C := C - V T^T V^T C on rows [j, m), columns [c0, n), in 64-column tiles.
-// P = V^T C: wave w takes the 16-row chunks w % 4, w % 4 + 4, ... and the
-// 16-column groups u of its share (all four with 4 waves; two, by w / 4, with
-// 8), accumulating its partial on the matrix cores (lane group g holds rows
-// 4g..4g+3 of a chunk, as k_gemm1); the partials are summed in wave order in
-// LDS.  W = T^T P (waves 0..3, rows 16w..), then C -= V W as C^T -= W^T V^T,
-// wave w taking the 16-row blocks w, w + NW, ...
+// C := C - V T^T V^T C on rows [j, m), columns [c0, n), 128 columns at a time, a
+// wave two groups of 16: P = V^T C down the rows, W = T^T P, C -= V W back up the
+// rows (the last rows of C are still in the L2).  V goes through LDS in 32-row
+// chunks (E's space, two buffers) as the merged pass of trailing.hip keeps it; a
+// wave holds its whole columns' P, so W follows in registers (the layout of one
+// product's result is the next one's operand).
+//
+// Memory bounds it, through the loads in flight: the matrices of a launch exceed
+// the caches, and one wave per SIMD (LDS holds one workgroup per CU) hides
+// nothing.  So two chunks of V and C are on their way to registers beside the
+// one in LDS, and 128 columns share a reading of V.  Per CU of a launch over 1024
+// matrices up to 1024 x 512 (8.87 -> 7.08 ms): 2.2 ms, about 11 GB in all, against
+// 2.95 with V read per wave and no loads in flight across chunks, and 4.7 with one
+// chunk in flight and 64 columns.
 template <int NW>
 __device__ __forceinline__ void bt_trailing(double* a, int lda, int j, int m, int kk, int c0, int n,
                             BatchLds<NW>& L) {
-  constexpr int UPW = 16 / NW;  // 16-column groups per wave in P
-  const int tid = local_tid(), lane = tid & 63, wave = tid >> 6;
+  static_assert(NW == 4, "a chunk of V is staged by four waves");
+  FuChunk* S = reinterpret_cast<FuChunk*>(&L.u.E[0][0][0]);
+  static_assert(sizeof(L.u.E) >= 2 * sizeof(FuChunk), "V's chunks lie in E");
+  constexpr int U = 2;  // column groups per wave
+  const int tid = local_tid(), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, li = lane & 15;
-  const int wr = wave & 3, u0 = UPW * (wave >> 2);
-  double* Wl = L.R1;  // [k][c], leading dimension KMAX + 1
-  // V columns of this lane (16t + li), clamped to a valid column
-  const double* vcol[4];
+  const int nch = (m - j + FU_CH - 1) / FU_CH;
+  // rows r, r + 1 of a column, rows from m on read as the last one
+  auto pair_at = [&](const double* col, int r) -> fu_pair {
+    if (r + 1 < m) return *reinterpret_cast<const fu_pair*>(col + r);
+    return (fu_pair){col[min(r, m - 1)], col[m - 1]};
+  };
+  struct Regs {
+    fu_pair v[4], c[U][4];
+  };
+  for (int cb = c0; cb < n; cb += 64 * U) {
+    double* Cc[U];
+    bool on[U], cok[U];  // the wave has columns of the group; the lane's one exists
 #pragma unroll
-  for (int t = 0; t < 4; t++) vcol[t] = a + (size_t)(j + min(16 * t + li, kk - 1)) * lda;
-  for (int cb = c0; cb < n; cb += 64) {
-    const int ncl = min(64, n - cb);
-    const double* ccol[UPW];
+    for (int u = 0; u < U; u++) {
+      const int col = cb + 64 * u + 16 * wave + li;
+      on[u] = cb + 64 * u + 16 * wave < n;
+      cok[u] = col < n;
+      Cc[u] = a + (size_t)min(col, n - 1) * lda;
+    }
+    // chunk ch: V's columns 16 wave + 4 i + g, rows 2 li, 2 li + 1; C's rows
+    // j + 32 ch + 8 v + 2 g + (0, 1) of the lane's columns
+    auto load = [&](int ch, Regs& x) {
+      if (ch < 0 || ch >= nch) return;
+      const int r0 = j + FU_CH * ch;
+      if (r0 + FU_CH <= m) {  // whole: plain loads, back to back
 #pragma unroll
-    for (int u = 0; u < UPW; u++) ccol[u] = a + (size_t)(cb + min(16 * (u0 + u) + li, ncl - 1)) * lda;
-    dbl4 acc[4][UPW];
+        for (int i = 0; i < 4; i++)
+          x.v[i] = *reinterpret_cast<const fu_pair*>(
+              a + (size_t)(j + min(16 * wave + 4 * i + g, kk - 1)) * lda + r0 + 2 * li);
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+        for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int u = 0; u < UPW; u++) acc[t][u] = (dbl4){0.0, 0.0, 0.0, 0.0};
-    for (int rs = j + 16 * wr; rs < m; rs += 64) {
-      double vr[4][4], cr[UPW][4];
+          for (int v = 0; v < 4; v++)
+            x.c[u][v] = *reinterpret_cast<const fu_pair*>(Cc[u] + r0 + 8 * v + 2 * g);
+        return;
+      }
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int row = rs + 4 * g + q, rr = row - j;
-        const bool rok = row < m;
+      for (int i = 0; i < 4; i++)
+        x.v[i] = pair_at(a + (size_t)(j + min(16 * wave + 4 * i + g, kk - 1)) * lda,
+                         j + FU_CH * ch + 2 * li);
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const int c = 16 * t + li;
-          const double x = (rok && c < kk && rr > c) ? vcol[t][row] : 0.0;
-          vr[t][q] = (rr == c && c < kk) ? 1.0 : x;
+      for (int u = 0; u < U; u++)
+        if (on[u]) {
+#pragma unroll
+          for (int v = 0; v < 4; v++) x.c[u][v] = pair_at(Cc[u], j + FU_CH * ch + 8 * v + 2 * g);
         }
+    };
+    auto store_v = [&](int ch, const fu_pair (&x)[4]) {
+      if (ch < 0 || ch >= nch) return;
+      if (ch > 1 && kk == KMAX && j + FU_CH * (ch + 1) <= m) {  // below the top block, whole
 #pragma unroll
-        for (int u = 0; u < UPW; u++)
-          cr[u][q] = (rok && 16 * (u0 + u) + li < ncl) ? ccol[u][row] : 0.0;
+        for (int i = 0; i < 4; i++) {
+          const int c = 16 * wave + 4 * i + g;
+          S[ch & 1][c][li ^ (c & 15)] = make_double2(x[i].x, x[i].y);
+        }
+        return;
       }
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-          for (int u = 0; u < UPW; u++)
-            acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(vr[t][q], cr[u][q], acc[t][u], 0, 0,
-                                                             0);
-    }
-    // sum of the wave partials, in wave order: P(16t + g + 4v, 16u + li)
-    __syncthreads();  // the previous tile is done with Wl
-    for (int w = 0; w < NW; w++) {
-      if (wave == w) {
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-          for (int u = 0; u < UPW; u++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-              double* p = &Wl[(16 * t + g + 4 * v) * (KMAX + 1) + 16 * (u0 + u) + li];
-              *p = (wr == 0) ? acc[t][u][v] : *p + acc[t][u][v];
-            }
+      for (int i = 0; i < 4; i++) {
+        const int c = 16 * wave + 4 * i + g, pr = FU_CH * ch + 2 * li;
+        double2 v;
+        v.x = (c < kk && j + pr < m) ? (pr > c ? x[i].x : (pr == c ? 1.0 : 0.0)) : 0.0;
+        v.y = (c < kk && j + pr + 1 < m) ? (pr + 1 > c ? x[i].y : (pr + 1 == c ? 1.0 : 0.0)) : 0.0;
+        S[ch & 1][c][li ^ (c & 15)] = v;
       }
-      __syncthreads();
-    }
-    // W = T^T P: T(i, r) = Ts[i + r * KMAX]
-    dbl4 wacc[4];
-    if (wave < 4) {
+    };
+    dbl4 acc[U][4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) wacc[u] = (dbl4){0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-      for (int k0 = 0; k0 < KMAX; k0 += 4) {
-        const double av = L.Ts[(k0 + g) + (16 * wave + li) * KMAX];
+    for (int u = 0; u < U; u++)
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-          wacc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-              av, Wl[(k0 + g) * (KMAX + 1) + 16 * u + li], wacc[u], 0, 0, 0);
+      for (int t = 0; t < 4; t++) acc[u][t] = (dbl4){0.0, 0.0, 0.0, 0.0};
+    // chunk ch's products; x0: chunk ch (V stored already), x1: ch + 1, which
+    // follows into LDS; ch + 2 is fetched over x0
+    auto down = [&](int ch, Regs& x0, Regs& x1) {
+      lds_barrier();  // chunk ch is in LDS; the other buffer is read
+      fu_pair c[U][4];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) c[u][v] = x0.c[u][v];
+      load(ch + 2, x0);
+      const FuChunk& V = S[ch & 1];
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        double2 x[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) x[t] = V[16 * t + li][(g + 4 * v) ^ li];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (on[u]) {
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+              acc[u][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t].x, c[u][v].x, acc[u][t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+              acc[u][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t].y, c[u][v].y, acc[u][t], 0, 0, 0);
+          }
       }
+      store_v(ch + 1, x1.v);
+    };
+    Regs xa, xb;
+    load(0, xa);
+    load(1, xb);
+    store_v(0, xa.v);
+    for (int ch = 0; ch < nch; ch += 2) {
+      down(ch, xa, xb);
+      if (ch + 1 < nch) down(ch + 1, xb, xa);
     }
-    __syncthreads();
-    if (wave < 4) {
+    // back from the last chunk, in LDS still
+    load(nch - 1, xa);
+    load(nch - 2, xb);
+    // P's rows 16 t + g + 4 v in acc[u][t][v], -W's in w[u][t][v]: W_t = sum over
+    // the blocks k <= t of T_kt^T P_k
+    dbl4 w[U][4];
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+    for (int t = 0; t < 4; t++) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) Wl[(16 * wave + g + 4 * v) * (KMAX + 1) + 16 * u + li] = wacc[u][v];
-    }
-    __syncthreads();
-    // C -= V W on 16-row blocks: D_u(c, r) = sum_k W(k, 16u + c) V(r, k)
-    const double* cbase = a + (size_t)cb * lda;
-    for (int rb = j + 16 * wave; rb < m; rb += 16 * NW) {
-      // W is read from LDS in every row block: kept out of the loop (64
-      // doubles per lane), it pushed the kernel past 512 VGPRs into scratch
-      __asm__ volatile("" ::: "memory");
-      const int row = rb + li;
-      double vk[KMAX / 4];
+      for (int u = 0; u < U; u++) w[u][t] = (dbl4){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int s = 0; s < KMAX / 4; s++) vk[s] = bt_v(a, lda, j, kk, row, 4 * s + g, m);
-      double cval[4][4];
-#pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int k = 0; k <= t; k++)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-          const int c = 16 * u + g + 4 * v;
-          cval[u][v] = (c < ncl && row < m) ? cbase[(size_t)c * lda + row] : 0.0;
+          const double x = -L.Ts[(16 * k + g + 4 * v) + (16 * t + li) * KMAX];
+#pragma unroll
+          for (int u = 0; u < U; u++)
+            w[u][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, acc[u][k][v], w[u][t], 0, 0, 0);
         }
-      dbl4 d[4];
+    }
+    auto up = [&](int ch, Regs& x0, Regs& x1) {
+      fu_pair c[U][4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) d[u] = (dbl4){0.0, 0.0, 0.0, 0.0};
+      for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int s = 0; s < KMAX / 4; s++)
+        for (int v = 0; v < 4; v++) c[u][v] = x0.c[u][v];
+      load(ch - 2, x0);
+      const FuChunk& V = S[ch & 1];
+      dbl4 d[U][2];
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-          d[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(Wl[(4 * s + g) * (KMAX + 1) + 16 * u + li],
-                                                     vk[s], d[u], 0, 0, 0);
+      for (int u = 0; u < U; u++) d[u][0] = d[u][1] = (dbl4){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int s = 0; s < 16; s++) {
+        const double2 x = V[4 * s + g][li ^ (4 * (s & 3) + g)];
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int c = 16 * u + g + 4 * v;
-          if (c < ncl && row < m) a[(size_t)(cb + c) * lda + row] = cval[u][v] - d[u][v];
+        for (int u = 0; u < U; u++)
+          if (on[u]) {
+            d[u][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, w[u][s >> 2][s & 3], d[u][0], 0, 0, 0);
+            d[u][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, w[u][s >> 2][s & 3], d[u][1], 0, 0, 0);
+          }
+      }
+      if (j + FU_CH * (ch + 1) <= m) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (cok[u]) {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+              *reinterpret_cast<fu_pair*>(Cc[u] + j + FU_CH * ch + 8 * v + 2 * g) =
+                  (fu_pair){c[u][v].x + d[u][0][v], c[u][v].y + d[u][1][v]};
+          }
+      } else
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (cok[u]) {
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            const int r = j + FU_CH * ch + 8 * v + 2 * g;
+            const fu_pair o = {c[u][v].x + d[u][0][v], c[u][v].y + d[u][1][v]};
+            if (r + 1 < m) *reinterpret_cast<fu_pair*>(Cc[u] + r) = o;
+            else if (r < m) Cc[u][r] = o.x;
+          }
         }
+      store_v(ch - 1, x1.v);
+      lds_barrier();
+    };
+    for (int ch = nch - 1; ch >= 0; ch -= 2) {
+      up(ch, xa, xb);
+      if (ch > 0) up(ch - 1, xb, xa);
     }
   }
 }
@@ -240,15 +314,22 @@ __device__ __forceinline__ void bt_gram(int r0, int m, int ncols, ColFn colval, 
   dbl4p gt[10];
 #pragma unroll
   for (int p = 0; p < 10; p++) gt[p] = (dbl4p){0.0, 0.0, 0.0, 0.0};
-  for (int rb = r0 + 16 * wv; rb < m; rb += NW * 16) {
-    dbl4p xb[4];
+  dbl4p xn[4];  // the next block, on its way while this one is multiplied
+  auto load = [&](int rb) {
 #pragma unroll
     for (int u = 0; u < 4; u++)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int c = 16 * u + li, r = rb + g + 4 * v;
-        xb[u][v] = (c < ncols && r < m) ? colval(c, r) : 0.0;
+        xn[u][v] = (c < ncols && r < m) ? colval(c, r) : 0.0;
       }
+  };
+  load(r0 + 16 * wv);
+  for (int rb = r0 + 16 * wv; rb < m; rb += NW * 16) {
+    dbl4p xb[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) xb[u] = xn[u];
+    if (rb + NW * 16 < m) load(rb + NW * 16);
     gram_tiles(xb, gt);
   }
   bt_gram_store(reinterpret_cast<double (*)[LDP]>(L.R1), gt);
@@ -302,19 +383,26 @@ __device__ __forceinline__ int bt_panel_gram(double* a, int lda, int j, int m, i
   dbl4p gt[10];
 #pragma unroll
   for (int p = 0; p < 10; p++) gt[p] = (dbl4p){0.0, 0.0, 0.0, 0.0};
-  for (int rb = j + 16 * wv; rb < m; rb += NW * 16) {
+  double pn[KMAX / 4];  // the next block's P
+  auto load_p = [&](int rb, int kc) {
     const int ra = rb + li;
-    double pa[KMAX / 4];
 #pragma unroll
     for (int t = 0; t < KMAX / 4; t++)
-      pa[t] = (ra < m && 4 * t + g < k1) ? a[(size_t)(j + 4 * t + g) * lda + ra] : 0.0;
+      pn[t] = (ra < m && 4 * t + g < kc) ? a[(size_t)(j + 4 * t + g) * lda + ra] : 0.0;
+  };
+  load_p(j + 16 * wv, k1);
+  for (int rb = j + 16 * wv; rb < m; rb += NW * 16) {
+    double pa[KMAX / 4];
+#pragma unroll
+    for (int t = 0; t < KMAX / 4; t++) pa[t] = pn[t];
+    if (rb + NW * 16 < m) load_p(rb + NW * 16, k1);
     dbl4p qb[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) qb[u] = (dbl4p){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int t = 0; t < KMAX / 4; t++)
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int u = t / 4; u < 4; u++)
         qb[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[t], E1[4 * t + g][16 * u + li], qb[u], 0, 0,
                                                      0);
     gram_tiles(qb, gt);
@@ -344,19 +432,19 @@ __device__ __forceinline__ int bt_panel_gram(double* a, int lda, int j, int m, i
   // (summed into E1 in wave order).
 #pragma unroll
   for (int p = 0; p < 10; p++) gt[p] = (dbl4p){0.0, 0.0, 0.0, 0.0};
+  load_p(j + 16 * wv, k);
   for (int rb = j + 16 * wv; rb < m; rb += NW * 16) {
-    const int ra = rb + li;
     double pa[KMAX / 4];
 #pragma unroll
-    for (int t = 0; t < KMAX / 4; t++)
-      pa[t] = (ra < m && 4 * t + g < k) ? a[(size_t)(j + 4 * t + g) * lda + ra] : 0.0;
+    for (int t = 0; t < KMAX / 4; t++) pa[t] = pn[t];
+    if (rb + NW * 16 < m) load_p(rb + NW * 16, k);
     dbl4p vb[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) vb[u] = (dbl4p){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int t = 0; t < KMAX / 4; t++)
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int u = t / 4; u < 4; u++)
         vb[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[t], E0[4 * t + g][16 * u + li], vb[u], 0, 0,
                                                      0);
 #pragma unroll
@@ -390,6 +478,48 @@ __device__ __forceinline__ int bt_panel_gram(double* a, int lda, int j, int m, i
   return k;
 }
 
+// The norms of columns c, c + step, c + 2 step, c + 3 step (below n), each
+// summed as wave_nrm2 does, the four columns' loads in flight together (one
+// column at a time waits for memory 1.5 us per column and wave).
+__device__ __forceinline__ void bt_nrm2x4(const double* a, int lda, int c, int step, int n, int m,
+                                          double (&nr)[4]) {
+  const int lane = local_tid() & 63;
+  const double* x[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) x[q] = a + (size_t)min(c + q * step, n - 1) * lda;
+  double s[4][4];
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+#pragma unroll
+    for (int u = 0; u < 4; u++) s[q][u] = 0.0;
+  int i = lane;
+  for (; i + 192 < m; i += 256) {
+    double v[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int u = 0; u < 4; u++) v[q][u] = x[q][i + 64 * u];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int u = 0; u < 4; u++) s[q][u] = fma(v[q][u], v[q][u], s[q][u]);
+  }
+  for (; i < m; i += 64) {
+    double v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = x[q][i];
+#pragma unroll
+    for (int q = 0; q < 4; q++) s[q][0] = fma(v[q], v[q], s[q][0]);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) nr[q] = wave_sum((s[q][0] + s[q][1]) + (s[q][2] + s[q][3]));
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    if (nr[q] >= 1e-280 && nr[q] <= 1e280) nr[q] = sqrt(nr[q]);
+    else if (c + q * step < n) nr[q] = wave_nrm2(x[q], m);
+  }
+}
+
 // One DM-QR (dgeqrdm semantics, free columns) of the matrix it by the whole
 // workgroup.  Returns info (0, or -13 for a non-finite entry, A untouched).
 template <int NW>
@@ -403,14 +533,20 @@ __device__ __forceinline__ int bt_factor(const BatchItem& it, double* A, double*
   const int minmn = m < n ? m : n;
   // initial norms (src/dgeqrdm_work.c:670-682), as k_init_norms
   double mx = 0.0, bad = 0.0;
-  for (int c = wave; c < n; c += NW) {
-    const double nr = wave_nrm2(a + (size_t)c * lda, m);
-    if (lane == 0) {
-      L.work[c] = nr;
-      L.wold[c] = nr;
+  for (int c = wave; c < n; c += 4 * NW) {
+    double nr4[4];
+    bt_nrm2x4(a, lda, c, NW, n, m, nr4);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if (c + NW * q >= n) break;
+      const double nr = nr4[q];
+      if (lane == 0) {
+        L.work[c + NW * q] = nr;
+        L.wold[c + NW * q] = nr;
+      }
+      if (!(nr <= DBL_MAX)) bad = 1.0;
+      else mx = fmax(mx, nr);
     }
-    if (!(nr <= DBL_MAX)) bad = 1.0;
-    else mx = fmax(mx, nr);
   }
   for (int c = tid; c < n; c += NT) L.jp[c] = c + 1;
   const double maxnrm0 = block_max(mx, L.red);
@@ -512,21 +648,30 @@ __device__ __forceinline__ int bt_factor(const BatchItem& it, double* A, double*
     const int fjb = L.st.fjb, npair = L.st.npair;
     // --- column moves (whole columns; work and jpvt with them, not workold)
     if (npair > 0) {
-      const int rb_rows = max(1, min(m, (8 * NT) / npair));
-      for (int r0 = 0; r0 < m; r0 += rb_rows) {
-        const int rows = min(rb_rows, m - r0), tot = npair * rows;
-        double v[8];
+      // a wave takes 32-row blocks: lane (h, r) row r of the pairs 2 p + h, every
+      // pair read before any is written, no barrier (with 8 elements a thread and
+      // two barriers per round over all rows 0.90 ms per CU of the launch above; 0.50)
+      constexpr int MV = 2 * KMAX / 2;  // pairs per lane at most
+      const int h = lane >> 5;
+      for (int r0 = 32 * wave; r0 < m; r0 += 32 * NW) {
+        const int r = r0 + (lane & 31);
+        double v[MV];
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-          const int e = tid + NT * q;
-          v[q] = (e < tot) ? a[(size_t)L.perm[2 * (e / rows) + 1] * lda + r0 + e % rows] : 0.0;
-        }
-        __syncthreads();
+        for (int p0 = 0; p0 < MV; p0 += 8)
+          if (2 * p0 < npair) {
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-          const int e = tid + NT * q;
-          if (e < tot) a[(size_t)L.perm[2 * (e / rows)] * lda + r0 + e % rows] = v[q];
-        }
+            for (int p = p0; p < p0 + 8; p++) {
+              const int pp = min(2 * p + h, npair - 1);
+              v[p] = a[(size_t)L.perm[2 * pp + 1] * lda + min(r, m - 1)];
+            }
+          }
+#pragma unroll
+        for (int p0 = 0; p0 < MV; p0 += 8)
+          if (2 * p0 < npair) {
+#pragma unroll
+            for (int p = p0; p < p0 + 8; p++)
+              if (2 * p + h < npair && r < m) a[(size_t)L.perm[2 * (2 * p + h)] * lda + r] = v[p];
+          }
       }
       double wv = 0.0;
       int jv = 0;
@@ -585,25 +730,48 @@ __device__ __forceinline__ int bt_factor(const BatchItem& it, double* A, double*
     // --- norm_update (src/dgeqrdm_work.c:80-109), as k_norm_update
     double nmx = 0.0;
     const int mrem = m - j - kk;
-    for (int col = j + kk + wave; col < n; col += NW) {
-      double wk = L.work[col];
-      if (wk == 0.0) continue;
-      const double* ac = a + (size_t)col * lda + j;
-      const double x = (lane < kk) ? ac[lane] : 0.0;
-      const double s = wave_sum(x * x);
-      double temp = sqrt(fabs(s)) / wk;
-      const double d2 = (temp + 1.0) * (1.0 - temp);
-      temp = (0.0 >= d2) ? 0.0 : d2;
-      const double d1 = wk / L.wold[col];
-      const double temp2 = temp * (d1 * d1);
-      if (temp2 <= P.tol3z) {
-        wk = (mrem > 0) ? wave_nrm2(ac + kk, mrem) : 0.0;
-        if (lane == 0) L.wold[col] = wk;
-      } else {
-        wk *= sqrt(temp);
+    // a wave's columns j + kk + wave + NW i, i < 64: their sums by the wave, eight
+    // columns' loads in flight, then lane i does column i's arithmetic
+    for (int cb = j + kk + wave; cb < n; cb += 64 * NW) {
+      const int nc64 = min(64, (n - cb + NW - 1) / NW);
+      double s2 = 0.0;
+      for (int i0 = 0; i0 < nc64; i0 += 8) {
+        double x[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+          x[q] = (lane < kk) ? a[(size_t)min(cb + NW * (i0 + q), n - 1) * lda + j + lane] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) x[q] = wave_sum(x[q] * x[q]);
+#pragma unroll
+        for (int q = 0; q < 8; q++) s2 = lane == i0 + q ? x[q] : s2;
       }
-      if (lane == 0) L.work[col] = wk;
-      if (wk == wk) nmx = fmax(nmx, wk);
+      const int col = cb + NW * lane;
+      const bool mine = lane < nc64;
+      double wk = mine ? L.work[col] : 0.0;
+      const bool live = wk != 0.0;  // (also not for a lane without a column)
+      bool again = false;
+      if (live) {
+        double temp = sqrt(fabs(s2)) / wk;
+        const double d2 = (temp + 1.0) * (1.0 - temp);
+        temp = (0.0 >= d2) ? 0.0 : d2;
+        const double d1 = wk / L.wold[col];
+        const double temp2 = temp * (d1 * d1);
+        again = temp2 <= P.tol3z;
+        if (!again) wk *= sqrt(temp);
+      }
+      for (unsigned long long left = __ballot(again); left; left &= left - 1) {
+        const int i = __builtin_ctzll(left);
+        const double nr =
+            (mrem > 0) ? wave_nrm2(a + (size_t)(cb + NW * i) * lda + j + kk, mrem) : 0.0;
+        if (lane == i) {
+          wk = nr;
+          L.wold[col] = nr;
+        }
+      }
+      if (live) {
+        L.work[col] = wk;
+        if (wk == wk) nmx = fmax(nmx, wk);
+      }
     }
     const double maxnrm = block_max(nmx, L.red);
     // --- step end (src/dgeqrdm_work.c:740, :780-785)

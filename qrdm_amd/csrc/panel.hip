@@ -775,7 +775,7 @@ __global__ __launch_bounds__(256) void k_qgram(const double* __restrict__ A, int
 #pragma unroll
   for (int t = 0; t < KMAX / 4; t++)
 #pragma unroll
-    for (int u = 0; u < 4; u++)
+    for (int u = t / 4; u < 4; u++)
       qb[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[t], Ri[4 * t + g][16 * u + li], qb[u], 0, 0, 0);
   dbl4p gt[10];
 #pragma unroll
@@ -1179,7 +1179,7 @@ __global__ __launch_bounds__(256) void k_v2(double* A, int lda, int m,
 #pragma unroll
   for (int t = 0; t < KMAX / 4; t++)
 #pragma unroll
-    for (int u = 0; u < 4; u++)
+    for (int u = t / 4; u < 4; u++)
       vb[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[t], Ms[4 * t + g][16 * u + li], vb[u], 0, 0, 0);
   // rows of the top block keep V1 (unit lower, written by the
   // reconstruction): overlay; then V and the panel's V2 rows out
