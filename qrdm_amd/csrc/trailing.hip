@@ -30,11 +30,13 @@
 // of its norm instead of 1.7e-15, at the same speed).
 #include "qrdm_internal.h"
 
+#include <algorithm>
+
 namespace qrdm {
 
 constexpr int FU_CH = 32;         // rows per chunk: two interleaved 16-row tiles
 constexpr int FU_NWG = 4;         // waves per workgroup
-constexpr int FU_MAX_SPLIT = 32;  // row slabs of the partial products at most
+constexpr int FU_MAX_SPLIT = 64;  // row slabs of the partial products at most
 constexpr int FU_GC = 16 * FU_NWG;  // columns of a workgroup
 constexpr int FU_OCC = 2;         // workgroups per CU (64 KB of LDS each)
 
@@ -60,10 +62,56 @@ __host__ __device__ __forceinline__ FuGeom fused_geom(int r_lo, int m, int c0, i
   return g;
 }
 
-// Workgroups of a fused pass per XCD: column group g goes to XCD g % 8 with
-// all its row slabs, so that each XCD holds one round of workgroups.
+// Workgroups of a fused pass per XCD: the (slab, column group) pairs, slab by slab,
+// in eight equal runs, so that every XCD has work however few column groups there
+// are and reads only its slabs' part of V.  (With a column group's slabs all on one
+// XCD every XCD read the whole V, and narrow C left some idle: 16384 x 1024 took
+// 86 us a pass.)
 __host__ __device__ __forceinline__ int fused_per_xcd(int ns, int cgroups) {
-  return ((cgroups + 7) / 8) * ns;
+  return (ns * cgroups + 7) / 8;
+}
+
+// Row slabs of a fused pass, at most one round of the chip's 64 workgroups per
+// XCD (two per CU): the cost of a count in chunks -- a slab's chunks and two for its
+// start and its partial tile, 1.7 times as long with a second workgroup on the CU,
+// and a twentieth per slab for the step's end -- or a large value where Wp (16 x 64
+// x n values) does not hold the partials.  Measured (us by workgroups per XCD, 4096
+// x 4096): 32 87, 48 104, 56 92, 64 79; 16384 x 512: 16 87, 32 50, 64 49; 1024 x
+// 1024: 16 16, 32 12, 64 15.  (Waves of 32 columns: 312 against 317 at 8192 x 8192,
+// 169 against 160 at 8192 x 4096; groups of 96 or 128 columns were slower
+// throughout.)
+__host__ __device__ __forceinline__ float fused_cost(int ns, int nchunk, int cgroups, int ncol,
+                                                     int n) {
+  const int per = fused_per_xcd(ns, cgroups);
+  if (ns > 1 && (per > 32 * FU_OCC || ns > nchunk || (long long)ns * ncol > 16LL * n)) return 1e9f;
+  const float chunks = (float)((nchunk + ns - 1) / ns) + 2.0f;
+  return (per > 32 ? 1.7f : 1.0f) * chunks + 0.05f * (float)ns;
+}
+
+// The count with the least cost, by a wave (lane: count lane + 1): the DM loop's
+// steps choose theirs on the device, from their own j and c0.  Chosen by the host
+// from the column reached at the last readback, up to sixteen steps before, the
+// last passes over 16384 x 1024 took as long as the first, 84 us.
+__device__ __forceinline__ int fused_slabs_wave(int r_lo, int m, int c0, int n) {
+  static_assert(FU_MAX_SPLIT == 64, "a lane per count");
+  const FuGeom g = fused_geom(r_lo, m, c0, n, 1);
+  if (g.cgroups <= 0 || g.nchunk <= 0) return 1;
+  const int ns = (local_tid() & 63) + 1;
+  const float cost = fused_cost(ns, g.nchunk, g.cgroups, n - c0, n);
+  // costs are positive: their bits are ordered as they are; equal ones, fewer slabs
+  int best = __float_as_int(cost), arg = ns;
+  auto take = [&](int ob, int oa) {
+    const bool t = ob < best || (ob == best && oa < arg);
+    best = t ? ob : best;
+    arg = t ? oa : arg;
+  };
+  take(xor_lane<1>(best), xor_lane<1>(arg));
+  take(xor_lane<2>(best), xor_lane<2>(arg));
+  take(xor_lane<4>(best), xor_lane<4>(arg));
+  take(xor_lane<8>(best), xor_lane<8>(arg));
+  take(xor_lane<16>(best), xor_lane<16>(arg));
+  take(xor_lane<32>(best), xor_lane<32>(arg));
+  return __builtin_amdgcn_readfirstlane(arg);
 }
 
 // A 32 x 64 chunk of V in LDS as 16-byte units of two rows: unit (row pair
@@ -138,10 +186,9 @@ __device__ __forceinline__ void sum_gram(const DevState* st, int m) {
 //
 // V is zero above its panel (within 64 rows) and past m, which the callers
 // keep so: no masks in the products, only the stores look at r_lo and m.  W is
-// indexed by absolute columns; the partials, ns slabs, by the columns from the
-// host's c0 on (a narrow C leaves room for more slabs).  With st (the DM loop)
-// r_lo, c0 and the buffers come from st; the grid is sized for the lowest j and
-// surplus workgroups return.
+// indexed by absolute columns; the partials, ns slabs, by the columns from c0 on (a
+// narrow C leaves room for more slabs).  With st (the DM loop) r_lo, c0, ns and the
+// buffers come from st; surplus workgroups of the grid return.
 //
 // On the way, beside the first loads, the workgroups sum V^T V of a Gram-based
 // panel from k_v2's slabs (fixed order) into the step's T^-1, and tau_i =
@@ -157,15 +204,16 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   // the chunks of V_s and V_{s+1}, two buffers each (arrays of their own, so
   // that a load on its way into one does not hold up reads of the other)
   __shared__ FuChunk vp0, vp1, vn0, vn1;
-  const int cw = c0, ldw = n - c0;  // the partials' columns
   if (st) {
     if (dm_stopped(st)) return;
     if (!st->given) {
       r_lo = st->j;
       c0 = st->c0;
       cur = st->it & 1;
+      ns = fused_slabs_wave(r_lo, m, c0, n);
     }
   }
+  const int ldw = n - c0;
   const int ldv = bufs.ldv;
   const double* Vn = bufs.V + (size_t)cur * bufs.vstride;
   const double* Vp = bufs.V + (size_t)(cur ^ 1) * bufs.vstride;
@@ -173,8 +221,9 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   const FuGeom G = fused_geom(r_lo, m, c0, n, ns);
   const int per = fused_per_xcd(ns, G.cgroups);
   const int xcd = blockIdx.x & 7, kx = blockIdx.x >> 3;
-  const int slab = kx % ns, cgrp = xcd + 8 * (kx / ns);
-  const bool active = kx < per && cgrp < G.cgroups;
+  const int pair = xcd * per + kx;
+  const int slab = G.cgroups > 0 ? pair / G.cgroups : ns, cgrp = pair - slab * G.cgroups;
+  const bool active = kx < per && slab < ns;
   if (!active) {
     if (ACCUM && st) sum_gram(st, m);
     return;
@@ -305,7 +354,7 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   }
   if (!ACCUM || !cok) return;
   // partial tile: row 16t + g + 4w of the lane's column
-  double* out = Wp + (size_t)slab * KMAX * ldw + (c0 + cbw + li - cw);
+  double* out = Wp + (size_t)slab * KMAX * ldw + (cbw + li);
 #pragma unroll
   for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -314,32 +363,14 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
 
 int fused_max_slabs() { return FU_MAX_SPLIT; }
 
-// Row slabs of a fused pass, at most one round of the chip's 64 workgroups per
-// XCD (two per CU), the count with the least cost in chunks: a slab's chunks
-// and two for its start and its partial tile, 1.7 times as long with a second
-// workgroup on the CU, and a twentieth per slab for the step's end.  Measured
-// (us by workgroups per XCD, 4096 x 4096): 32 87, 48 104, 56 92, 64 79;
-// 16384 x 512: 16 87, 32 50, 64 49; 1024 x 1024: 16 16, 32 12, 64 15.  (Waves of
-// 32 columns: 312 against 317 at 8192 x 8192, 169 against 160 at 8192 x 4096;
-// groups of 96 or 128 columns were slower throughout.)
 int fused_slabs(int r_lo, int m, int c0, int n) {
   const FuGeom g = fused_geom(r_lo, m, c0, n, 1);
   if (g.cgroups <= 0 || g.nchunk <= 0) return 1;
-  const int per = (g.cgroups + 7) / 8;
-  int cap = (int)(16LL * n / (n - c0));  // Wp holds 16 x 64 x n values
-  if (cap > FU_MAX_SPLIT) cap = FU_MAX_SPLIT;
-  if (cap > g.nchunk) cap = g.nchunk;
   int best = 1;
-  double least = 1e30;
-  for (int ns = 1; ns <= cap; ns++) {
-    if (ns > 1 && per * ns > 32 * FU_OCC) break;
-    const double chunks = (g.nchunk + ns - 1) / ns + 2.0;
-    const double cost = (per * ns > 32 ? 1.7 : 1.0) * chunks + 0.05 * ns;
-    if (cost < least) {
-      least = cost;
+  for (int ns = 2; ns <= FU_MAX_SPLIT; ns++)
+    if (fused_cost(ns, g.nchunk, g.cgroups, n - c0, n) <
+        fused_cost(best, g.nchunk, g.cgroups, n - c0, n))
       best = ns;
-    }
-  }
   return best;
 }
 
@@ -348,7 +379,13 @@ void launch_fused(double* A, int lda, int r_lo, int m, int c0, int n, const Step
                   const DevState* st) {
   if (n - c0 <= 0 || m - r_lo <= 0 || !(apply || accum)) return;
   const FuGeom g = fused_geom(r_lo, m, c0, n, ns);
-  const dim3 grid(8 * fused_per_xcd(ns, g.cgroups)), block(64 * FU_NWG);
+  // with st the device chooses the slabs, at most one round (or a pair per chunk)
+  int per = fused_per_xcd(ns, g.cgroups);
+  if (st) {
+    const long long most = ((long long)g.nchunk * g.cgroups + 7) / 8;
+    per = std::max(per, (int)std::min(most, (long long)std::max(32 * FU_OCC, (g.cgroups + 7) / 8)));
+  }
+  const dim3 grid(8 * per), block(64 * FU_NWG);
   if (apply && accum)
     hipLaunchKernelGGL((k_fused<true, true>), grid, block, 0, s, A, lda, r_lo, m, c0, n, bufs, Wp,
                        ns, cur, st);
@@ -420,8 +457,8 @@ __device__ __forceinline__ void wy_solve(const double (*Us)[LDP], const double (
     for (int v = 0; v < 4; v++) S1[16 * i + g + 4 * v][li] = w[i][v];
 }
 
-__global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, int n, int cw,
-                                                   const double* __restrict__ Wp, int ns,
+__global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, int n,
+                                                   const double* __restrict__ Wp,
                                                    StepBufs bufs, double* work, double* workold,
                                                    DevState* st, double tol3z) {
   __shared__ double Us[KMAX][LDP];             // T^-1
@@ -443,7 +480,7 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const double* V = v_cur(bufs, st);
   double* W = w_cur(bufs, st);
-  const int ldv = bufs.ldv, ldw = n - cw;
+  const int ldv = bufs.ldv, ldw = n - c0, ns = fused_slabs_wave(j, m, c0, n);
   const int col = cb + li, cl = min(col, n - 1);  // the lane's column
   // every global read of the prologue in flight together: T^-1, the first
   // slabs' partials (thread: column li, rows i0 + 16 q), V's and C's top rows
@@ -451,7 +488,7 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
 #pragma unroll
   for (int q = 0; q < KMAX * KMAX / 256; q++) us[q] = ws_mat(st, WS_S)[tid + 256 * q];
   const int i0 = tid >> 4;
-  const double* wp = Wp + (size_t)i0 * ldw + cl - cw;
+  const double* wp = Wp + (size_t)i0 * ldw + max(cl - c0, 0);
   constexpr int YB = 8;  // slabs per round
   double pv[YB][4];
   auto load_p = [&](int y0) {
@@ -620,12 +657,13 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
 void launch_wsum_norm(double* A, int lda, int j0, int m, int n, const double* T,
                       const double* Wp, int ns, const StepBufs& bufs, double* work,
                       double* workold, DevState* st, double tol3z, hipStream_t s) {
-  (void)T;  // the step's T^-1 lies behind the state (ws_mat WS_S)
+  (void)T;   // the step's T^-1 lies behind the state (ws_mat WS_S)
+  (void)ns;  // the slabs as the pass chose them
   // tiles of [j + kk, n), j + kk >= j0 + 1; one workgroup at least (it marks
-  // the step's end pending).  The pass's partials start at column j0 + 1.
+  // the step's end pending).
   int tiles = (n - j0 - 1 + WN_TC - 1) / WN_TC;
   if (tiles < 1) tiles = 1;
-  hipLaunchKernelGGL(k_wsum_norm, dim3(tiles), dim3(256), 0, s, A, lda, m, n, j0 + 1, Wp, ns,
+  hipLaunchKernelGGL(k_wsum_norm, dim3(tiles), dim3(256), 0, s, A, lda, m, n, Wp,
                      bufs, work, workold, st, tol3z);
 }
 
