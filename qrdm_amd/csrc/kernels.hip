@@ -67,6 +67,30 @@ __device__ __forceinline__ double wave_nrm2(const double* __restrict__ x, int n)
   return amax * sqrt(wave_sum(s2));
 }
 
+// wave_nrm2 with sixteen loads in flight per lane (the same sums in the same order).
+__device__ __forceinline__ double wave_nrm2_deep(const double* __restrict__ x, int n) {
+  const int lane = local_tid() & 63;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  int i = lane;
+  for (; i + 960 < n; i += 1024) {
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = x[i + 64 * u];
+#pragma unroll
+    for (int u = 0; u < 16; u++) s[u & 3] = fma(v[u], v[u], s[u & 3]);
+  }
+  for (; i + 192 < n; i += 256) {
+    double v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[u] = x[i + 64 * u];
+#pragma unroll
+    for (int u = 0; u < 4; u++) s[u] = fma(v[u], v[u], s[u]);
+  }
+  for (; i < n; i += 64) s[0] = fma(x[i], x[i], s[0]);
+  const double t = wave_sum((s[0] + s[1]) + (s[2] + s[3]));
+  return t >= 1e-280 && t <= 1e280 ? sqrt(t) : wave_nrm2(x, n);
+}
+
 // Block-wide sum; red must hold blockDim.x/64 doubles.  All threads return it.
 __device__ double block_sum(double v, double* red) {
   const int lane = local_tid() & 63, wave = local_tid() >> 6, nw = blockDim.x >> 6;
@@ -136,10 +160,10 @@ __device__ __forceinline__ double dsign(double a, double b) {
 
 // ---------------------------------------------------------------------------
 // Initial partial norms: work[c] = workold[c] = ||A(r0:m, c)||, max over all
-// columns (src/dgeqrdm_work.c:670-682).  One wave per column.
-// One wave per column, NORM_COLS columns per wave; the maximum is reduced in
-// the workgroup first so that only one atomic per workgroup reaches the
-// single maxnrm word (same-address atomics serialise).
+// columns (src/dgeqrdm_work.c:670-682), a wave per column; the maximum is reduced
+// in the workgroup first so that only one atomic per workgroup reaches the
+// single maxnrm word (same-address atomics serialise).  (NORM_COLS: columns per
+// wave of the norm update.)
 constexpr int NORM_COLS = 4;
 
 __device__ __forceinline__ void block_max_atomic(double v, int bad, DevState* st) {
@@ -161,14 +185,14 @@ __device__ __forceinline__ void block_max_atomic(double v, int bad, DevState* st
 
 __global__ __launch_bounds__(256) void k_init_norms(const double* __restrict__ A, int lda,
                                                      int r0, int m, int n, double* work,
-                                                     double* workold, DevState* st) {
+                                                     double* workold, DevState* st, int cols) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   double mx = 0.0;
   int bad = 0;
-  for (int q = 0; q < NORM_COLS; q++) {
-    const int col = (blockIdx.x * 4 + wave) * NORM_COLS + q;
+  for (int q = 0; q < cols; q++) {
+    const int col = (blockIdx.x * 4 + wave) * cols + q;
     if (col >= n) break;
-    const double nr = wave_nrm2(A + (size_t)col * lda + r0, m - r0);
+    const double nr = wave_nrm2_deep(A + (size_t)col * lda + r0, m - r0);
     if (lane == 0) {
       work[col] = nr;
       workold[col] = nr;
@@ -181,9 +205,11 @@ __global__ __launch_bounds__(256) void k_init_norms(const double* __restrict__ A
 
 void launch_init_norms(const double* A, int lda, int r0, int m, int n, double* work,
                        double* workold, DevState* st, hipStream_t s) {
-  const int waves = (n + NORM_COLS - 1) / NORM_COLS;
+  // a column per wave up to 16384 (4096 atomics at most): 16384 x 1024 with four
+  // left three CUs in four idle, 117 us; 25 us so, with sixteen loads in flight
+  const int cols = (n + 16383) / 16384, waves = (n + cols - 1) / cols;
   hipLaunchKernelGGL(k_init_norms, dim3((waves + 3) / 4), dim3(256), 0, s, A, lda, r0, m, n,
-                     work, workold, st);
+                     work, workold, st, cols);
 }
 
 // ---------------------------------------------------------------------------
