@@ -809,6 +809,34 @@ __global__ __launch_bounds__(256) void k_gram_cand(double* A, int lda, int m, do
   }
 }
 
+// Column blockIdx.x of the slabs' sum (KMAX x KMAX partials, upper triangles, summed
+// in slab order by the four waves' shares) into G, with its mirror: 64 workgroups.
+// The lanes below the diagonal load nothing: taking their values from the mirrored
+// entries, a line each, made the sum three times as long (the candidate Grams'
+// kernel 25.7 us at 16384 rows and 15.5 at 8192 x 8192; 14.0 and 12.5 so).
+__device__ __forceinline__ void reduce_column(const double* __restrict__ partial, int nslab,
+                                              double* G, double (*part)[64]) {
+  const int r = threadIdx.x & 63, c = blockIdx.x, q = threadIdx.x >> 6;
+  double s = 0.0;
+  if (r <= c) {
+    const double* p = partial + r + c * KMAX;
+    for (int b0 = q; b0 < nslab; b0 += 64) {
+      double v[16];
+#pragma unroll
+      for (int u = 0; u < 16; u++) v[u] = p[(size_t)min(b0 + 4 * u, nslab - 1) * KMAX * KMAX];
+#pragma unroll
+      for (int u = 0; u < 16; u++) s += (b0 + 4 * u < nslab) ? v[u] : 0.0;
+    }
+  }
+  part[q][r] = s;
+  __syncthreads();
+  if (q == 0 && r <= c) {
+    const double x = (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
+    st_dev(G + r + c * KMAX, x);
+    if (r < c) st_dev(G + c + r * KMAX, x);
+  }
+}
+
 // The sum of the step's candidate Grams in slab order, then the
 // last workgroup to finish (atomic ticket, reset for the next launch) runs
 // the greedy acceptance and the step's plan on it (select_wave).
@@ -830,26 +858,8 @@ __global__ __launch_bounds__(256) void k_reduce_select(const double* __restrict_
   double* Wq = w_prev(bufs, st);
   const int jw = st->j, ncw = max(st->nc, 1);
   const int cid_lane = st->cand_idx[threadIdx.x & 63];
-  const int e = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int pr = e & 63, pc = e >> 6;
-  const int es = (pr > pc) ? pc + pr * KMAX : e;  // symmetric: the upper triangle's value
   const int q = threadIdx.x >> 6;
-  double sacc = 0.0;
-  for (int b0 = q; b0 < nslab; b0 += 32) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int b = b0 + 4 * u;
-      v[u] = partial[(size_t)(b < nslab ? b : q) * KMAX * KMAX + es];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; u++) sacc += (b0 + 4 * u < nslab) ? v[u] : 0.0;
-  }
-  part[q][threadIdx.x & 63] = sacc;
-  __syncthreads();
-  if (q == 0)
-    st_dev(G + e, (part[0][threadIdx.x] + part[1][threadIdx.x]) +
-                      (part[2][threadIdx.x] + part[3][threadIdx.x]));
+  reduce_column(partial, nslab, G, part);
   handoff_wait();
   __syncthreads();
   if (threadIdx.x == 0) s_last = last_to_arrive(ticket, gridDim.x) ? 1 : 0;

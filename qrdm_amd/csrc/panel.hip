@@ -727,8 +727,8 @@ __device__ __forceinline__ void load_mat(double (*S)[LDP], const double* __restr
 }
 
 // The sum over the four waves (in wave order) of their upper-tile Grams gt,
-// both triangles, column-major into out (64 x 64).  Gp: LDS for the waves'
-// tiles.  Ends after the writes (no barrier).
+// column-major into out (64 x 64; nothing below the diagonal tiles).  Gp: LDS for
+// the waves' tiles.  Ends after the writes (no barrier).
 __device__ __forceinline__ void gram_sum_store(const dbl4p (&gt)[10], double (*Gp)[10][4][64],
                                                double* out) {
   const int tid = local_tid(), lane = tid & 63, wv = tid >> 6;
@@ -744,7 +744,6 @@ __device__ __forceinline__ void gram_sum_store(const dbl4p (&gt)[10], double (*G
     const double x = ((Gp[0][p][v][ln] + Gp[1][p][v][ln]) + Gp[2][p][v][ln]) + Gp[3][p][v][ln];
     const int r = 16 * u + (ln >> 4) + 4 * v, c = 16 * u2 + (ln & 15);
     out[r + (size_t)c * KMAX] = x;
-    if (u != u2) out[c + (size_t)r * KMAX] = x;
   }
 }
 
@@ -1111,24 +1110,7 @@ __global__ __launch_bounds__(256) void k_reduce_recon(const double* __restrict__
   if (!step_runs(st, RUN_FAST)) return;
   ReconIn rin;
   recon_inputs(rin, st, R1, R1inv, A, lda);
-  const int e = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int q = threadIdx.x >> 6;
-  double sacc = 0.0;
-  for (int b0 = q; b0 < nslab; b0 += 32) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int b = b0 + 4 * u;
-      v[u] = partial[(size_t)(b < nslab ? b : q) * KMAX * KMAX + e];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; u++) sacc += (b0 + 4 * u < nslab) ? v[u] : 0.0;
-  }
-  part[q][threadIdx.x & 63] = sacc;
-  __syncthreads();
-  if (q == 0)
-    st_dev(G2 + e, (part[0][threadIdx.x] + part[1][threadIdx.x]) +
-                       (part[2][threadIdx.x] + part[3][threadIdx.x]));
+  reduce_column(partial, nslab, G2, part);
   handoff_wait();
   __syncthreads();
   if (threadIdx.x == 0) s_last = last_to_arrive(ticket, gridDim.x) ? 1 : 0;
