@@ -94,11 +94,6 @@ __device__ __forceinline__ void bt_trailing(double* a, int lda, int j, int m, in
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, li = lane & 15;
   const int nch = (m - j + FU_CH - 1) / FU_CH;
-  // rows r, r + 1 of a column, rows from m on read as the last one
-  auto pair_at = [&](const double* col, int r) -> fu_pair {
-    if (r + 1 < m) return *reinterpret_cast<const fu_pair*>(col + r);
-    return (fu_pair){col[min(r, m - 1)], col[m - 1]};
-  };
   struct Regs {
     fu_pair v[4], c[U][4];
   };
@@ -129,16 +124,30 @@ __device__ __forceinline__ void bt_trailing(double* a, int lda, int j, int m, in
             x.c[u][v] = *reinterpret_cast<const fu_pair*>(Cc[u] + r0 + 8 * v + 2 * g);
         return;
       }
+      // the last one: rows from m on read as the last row (every load in flight
+      // before any is used)
+      double lo[4 + 4 * U], hi[4 + 4 * U];
 #pragma unroll
-      for (int i = 0; i < 4; i++)
-        x.v[i] = pair_at(a + (size_t)(j + min(16 * wave + 4 * i + g, kk - 1)) * lda,
-                         j + FU_CH * ch + 2 * li);
+      for (int i = 0; i < 4; i++) {
+        const double* col = a + (size_t)(j + min(16 * wave + 4 * i + g, kk - 1)) * lda;
+        lo[i] = col[min(r0 + 2 * li, m - 1)];
+        hi[i] = col[min(r0 + 2 * li + 1, m - 1)];
+      }
 #pragma unroll
       for (int u = 0; u < U; u++)
-        if (on[u]) {
 #pragma unroll
-          for (int v = 0; v < 4; v++) x.c[u][v] = pair_at(Cc[u], j + FU_CH * ch + 8 * v + 2 * g);
+        for (int v = 0; v < 4; v++) {
+          lo[4 + 4 * u + v] = Cc[u][min(r0 + 8 * v + 2 * g, m - 1)];
+          hi[4 + 4 * u + v] = Cc[u][min(r0 + 8 * v + 2 * g + 1, m - 1)];
         }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) x.v[i] = (fu_pair){lo[i], hi[i]};
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          x.c[u][v] = (fu_pair){lo[4 + 4 * u + v], hi[4 + 4 * u + v]};
     };
     auto store_v = [&](int ch, const fu_pair (&x)[4]) {
       if (ch < 0 || ch >= nch) return;

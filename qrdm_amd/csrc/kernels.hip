@@ -934,12 +934,19 @@ __device__ void apply_perm_rows(double* A, int lda, int m, double* work, int* jp
   const int tot = npair * PERM_ROWS;
   for (int q0 = 0; q0 < 2 * KMAX * PERM_ROWS / 256; q0 += 8) {
     if (q0 * 256 >= tot) break;
+    // (unconditional: a load under a condition that needs its pair's column
+    // first waited for both, eight times in a row)
     double v[8];
+    int src[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) {
       const int t = local_tid() + 256 * (q0 + q);
-      const int p = t / PERM_ROWS, r = rs + t % PERM_ROWS;
-      v[q] = (t < tot && r < m) ? A[(size_t)perm[2 * p + 1] * lda + r] : 0.0;
+      src[q] = perm[2 * min(t / PERM_ROWS, npair - 1) + 1];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int t = local_tid() + 256 * (q0 + q);
+      v[q] = A[(size_t)src[q] * lda + min(rs + t % PERM_ROWS, m - 1)];
     }
 #pragma unroll
     for (int q = 0; q < 8; q++) {
@@ -955,9 +962,16 @@ __device__ void apply_perm_rows(double* A, int lda, int m, double* work, int* jp
     if (jp) jv = jp[perm[2 * local_tid() + 1]];
   }
   __syncthreads();
-  for (int t = local_tid(); t < tot; t += 256) {
-    const int p = t / PERM_ROWS, r = rs + t % PERM_ROWS;
-    if (r < m) A[(size_t)perm[2 * p] * lda + r] = buf[t];
+  {
+    int dst[2 * KMAX * PERM_ROWS / 256];
+#pragma unroll
+    for (int q = 0; q < 2 * KMAX * PERM_ROWS / 256; q++)
+      dst[q] = npair > 0 ? perm[2 * min((local_tid() + 256 * q) / PERM_ROWS, npair - 1)] : 0;
+#pragma unroll
+    for (int q = 0; q < 2 * KMAX * PERM_ROWS / 256; q++) {
+      const int t = local_tid() + 256 * q, r = rs + t % PERM_ROWS;
+      if (t < tot && r < m) A[(size_t)dst[q] * lda + r] = buf[t];
+    }
   }
   if (side) {
     work[perm[2 * local_tid()]] = wv;

@@ -236,15 +236,19 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   const int ch0 = slab * G.slab_ch;
   const int ch1 = min(ch0 + G.slab_ch, G.nchunk);
   // the lane's column c0 + cbw + li (past ncol: a valid column, never stored)
-  const bool cok = cbw + li < ncol;
+  const bool cok = cbw + li < ncol, won = cbw < ncol;  // (won: some lane's)
   double* Cc = A + (size_t)(c0 + min(cbw + li, ncol - 1)) * lda;
   // the previous step's W tile, negated: wr[s] = -W(4s + g, column li) (lane
   // group g takes the k index 4s + g of step s of product 1)
+  // (every load unconditional and in flight together: a load under a condition,
+  // negated at once, waited for memory sixteen times in a row, about 10 us)
   double wr[16];
   if (APPLY) {
+    const double* wc = Wprev + (size_t)(c0 + min(cbw + li, ncol - 1)) * KMAX + g;
 #pragma unroll
-    for (int s = 0; s < 16; s++)
-      wr[s] = cok ? -Wprev[(size_t)(c0 + cbw + li) * KMAX + 4 * s + g] : 0.0;
+    for (int s = 0; s < 16; s++) wr[s] = wc[4 * s];
+#pragma unroll
+    for (int s = 0; s < 16; s++) wr[s] = cok ? -wr[s] : 0.0;
   }
   dbl4 acc[4];
 #pragma unroll
@@ -297,6 +301,8 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
       if (ACCUM) load_v(Vn, nn, c + 1);
       load_c(c + 1, x);
     }
+    __builtin_amdgcn_sched_barrier(0);  // the loads are issued before the stores
+    bool four = false;  // the wave's last four memory operations are its stores
     if (APPLY) {
 #pragma unroll
       for (int s = 0; s < 16; s++) {
@@ -308,6 +314,7 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
       cc[1] += cx[1];
       const int r0 = G.base + FU_CH * c;
       if (r0 >= r_lo && r0 + FU_CH <= m) {
+        four = won;
         if (cok) {
 #pragma unroll
           for (int v = 0; v < 4; v++)
@@ -337,7 +344,12 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
           acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t].y, cc[1][v], acc[t], 0, 0, 0);
       }
     }
-    __syncthreads();  // the next chunk of V is in LDS (every load has arrived)
+    // the next chunk of V is in LDS once every wave's loads have arrived; the
+    // stores behind them (vector memory operations complete in order) may still
+    // be on their way
+    if (four) __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4)
+    else __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0)
+    lds_barrier();
   };
   fu_pair x[4];
   if (ch1 > ch0) {
@@ -503,8 +515,7 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
   double va[KMAX / 4];
   const int rt = 16 * wv + li;
 #pragma unroll
-  for (int t = 0; t < KMAX / 4; t++)
-    va[t] = rt < kk ? -V[(size_t)(4 * t + g) * ldv + j + rt] : 0.0;
+  for (int t = 0; t < KMAX / 4; t++) va[t] = V[(size_t)(4 * t + g) * ldv + min(j + rt, ldv - 1)];
   dbl4 r12;
 #pragma unroll
   for (int v = 0; v < 4; v++) {
@@ -523,6 +534,8 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
     if (r == c) s_rd[r] = us[q];
   }
   lds_barrier();
+#pragma unroll
+  for (int t = 0; t < KMAX / 4; t++) va[t] = rt < kk ? -va[t] : 0.0;
   // one wave inverts the diagonal blocks while the others wait for their loads
   if (wv == 3) diag_inverse(Us, s_rd, Di);
   {
@@ -593,16 +606,16 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
       double vb[KMAX / 4];
 #pragma unroll
       for (int t = 0; t < KMAX / 4; t++)
-        vb[t] = (ra < m) ? -V[(size_t)(4 * t + g) * ldv + ra] : 0.0;  // V(ra, 4t + g)
+        vb[t] = V[(size_t)(4 * t + g) * ldv + min(ra, m - 1)];  // V(ra, 4t + g)
       dbl4 d;
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int r = rb + g + 4 * v;
-        d[v] = (rec && r < m) ? A[(size_t)cl * lda + r] : 0.0;
+        d[v] = A[(size_t)cl * lda + min(r, m - 1)];
       }
 #pragma unroll
       for (int t = 0; t < KMAX / 4; t++)
-        d = __builtin_amdgcn_mfma_f64_16x16x4f64(vb[t], S1[4 * t + g][li], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(-vb[t], S1[4 * t + g][li], d, 0, 0, 0);
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int r = rb + g + 4 * v;

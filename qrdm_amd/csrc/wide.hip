@@ -48,8 +48,10 @@ __global__ __launch_bounds__(256) void k_topk_wide(const double* __restrict__ va
   for (int u = 0; u < WT_KEYS / 256; u++) {
     const int e = tid + 256 * u, g = base + e;
     const bool in = g < L;
-    sv[e] = in ? val_in[g] : -1.0;  // norms are >= 0
-    si[e] = in ? (idx_in ? idx_in[g] : g) : INT_MAX;
+    const double v = val_in[min(g, L - 1)];
+    const int i = idx_in ? idx_in[min(g, L - 1)] : g;
+    sv[e] = in ? v : -1.0;  // norms are >= 0
+    si[e] = in ? i : INT_MAX;
   }
   __syncthreads();
   // thread: key 64 blockIdx.y + lane, against the quarter of the list of its wave
