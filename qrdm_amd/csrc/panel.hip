@@ -80,12 +80,19 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// 1/x for x in [1, 2]: the hardware estimate and two Newton steps.
-__device__ __forceinline__ double rcp_nr12(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = fma(y, fma(-x, y, 1.0), y);
-  y = fma(y, fma(-x, y, 1.0), y);
-  return y;
+// 1/x: the hardware estimate and one third-order step.
+__device__ __forceinline__ double rcp_nr3(double x) {
+  const double y = __builtin_amdgcn_rcp(x), r = fma(-x, y, 1.0);
+  return fma(fma(r, r, r), y, y);
+}
+
+// Of a 16-column block, lane r (= lane % 16) holding column r's stop code: the
+// columns before the first stop (bad: a stop, or past the end), and its code.
+__device__ __forceinline__ int block_stop(bool bad, int stc, int& code) {
+  const unsigned m = (unsigned)__ballot(bad) & 0xFFFFu;
+  const int done = m ? __builtin_ctz(m) : 16;
+  code = m ? __builtin_amdgcn_readlane(stc, done) : 0;
+  return done;
 }
 
 // S[r][c] -= sum_{t < 16} A(r, t) B(t, c) for r, c in [lo, nlim), 16 x 16
@@ -140,35 +147,33 @@ __device__ __forceinline__ int chol_blocked(double (*S)[LDP], int nlim, StopFn s
   // Wave 0 factors the diagonal block at bs: lane r (= lane % 16) holds row
   // bs + r of the symmetric block; both triangles are updated, so R(i, r) =
   // S(r, i) rs is the lane's own value and row i comes from lane i by a row
-  // broadcast.  Branch-free pivot steps: a pivot that is not taken updates
-  // nothing (zero multipliers; entries past the stop are not read), and lane
-  // r stores 1 / R(r, r) after the block.  (The row index is re-read per
-  // block: one fixed across the blocks lets the compiler hoist all 32 row
-  // masks out of the loop and spill them.)
+  // broadcast.  The instructions of one wave bound it, not their latency, so a
+  // pivot step is only the reciprocal and the update: every pivot of the block is
+  // taken, lane r then tests its own (what comes after a stop is garbage that is
+  // not read) and takes its square root.  At 8192 x 8192 this and the
+  // 64-bit row broadcasts took the kernel from 26.5 to 23.9 us, and the LU of the
+  // reconstruction, which does the same, from 18.7 to 14.5.  (The row index is re-read per block: one
+  // fixed across the blocks lets the compiler hoist all 32 row masks out of the
+  // loop and spill them.)
   auto diag = [&](int bs) {
     const int lane = local_tid() & 63, r = lane & 15;
     double w[BLK];
 #pragma unroll
     for (int c = 0; c < BLK; c++) w[c] = S[bs + r][bs + c];
-    double rsr = 0.0;  // 1 / sqrt(pivot) of this lane's row once eliminated
-    bool act = true;
-    int done = BLK, code = 0;
+    double d_r = 0.0;
 #pragma unroll
     for (int i = 0; i < BLK; i++) {
-      const int gi = bs + i;
-      const double d = row_bcast(w[i], i);
-      const int stc = (gi < nlim) ? stopfn(gi, d) : 0;
-      const double rs = rsqrt_nr(d);  // committed only when the pivot is accepted
-      const bool go = act && gi < nlim && stc == 0;
-      done = (act && !go) ? i : done;
-      code = (act && !go) ? stc : code;
-      act = go;
-      rsr = (r == i) ? rs : rsr;
-      // S(r, c) -= R(i, r) R(i, c) = S(r, i) rs^2 S(i, c) for rows r > i
-      const double a = (go && r > i) ? w[i] * rs * rs : 0.0;
+      d_r = r == i ? w[i] : d_r;
+      // S(r, c) -= R(i, r) R(i, c) = S(r, i) / S(i, i) S(i, c) for rows r > i
+      const double rc = rcp_nr3(row_bcast(w[i], i));
+      const double a = r > i ? w[i] * rc : 0.0;
 #pragma unroll
       for (int c = i + 1; c < BLK; c++) w[c] = fma(-a, row_bcast(w[c], i), w[c]);
     }
+    const int gi = bs + r, stc = gi < nlim ? stopfn(gi, d_r) : 0;
+    int code;
+    const int done = block_stop(stc != 0 || gi >= nlim, stc, code);
+    const double rsr = rsqrt_nr(d_r);  // 1 / sqrt(pivot) of the lane's row
     // rows < done: R(r, c) = S(r, c) / sqrt(pivot) on and above the diagonal
     if (lane < BLK) {
 #pragma unroll
@@ -238,62 +243,46 @@ __device__ __forceinline__ int lu_signed_blocked(double (*W)[LDP], int nlim, con
                                                  int* why) {
   const int tid = local_tid(), wave = tid >> 6;
   // Wave 0 factors the diagonal block at bs: lane r (= lane % 16) holds row
-  // bs + r; the pivot row comes from lane i by a row broadcast.  Branch-free
-  // pivot steps: the stop code is a select, and a pivot that is not taken
-  // updates nothing (its multipliers are zero; entries past the stop are not
-  // read).  Lane r keeps d, tau and the scale of its own column and stores
-  // them after the block.  (The row index is re-read per block: one fixed
-  // across the blocks lets the compiler hoist all 32 row masks out of the
-  // loop and spill them.)
+  // bs + r; the pivot row comes from lane i by a row broadcast.  As in chol_blocked
+  // every pivot is taken, then lane r tests its own column's and stores its d, tau
+  // and scale.  (The row index is re-read per block: one fixed across the blocks
+  // lets the compiler hoist all 32 row masks out of the loop and spill them.)
+  auto scale = [](double al) {  // d / (-1 - |a|), d = -1 for a >= 0
+    return copysign(rcp_nr3(1.0 + fabs(al)), al + 0.0);
+  };
   auto diag = [&](int bs) {
     const int lane = local_tid() & 63, r = lane & 15;
     double w[BLK];
 #pragma unroll
     for (int c = 0; c < BLK; c++) w[c] = W[bs + r][bs + c];
-    // ||x_i|| < thres  <=>  (1 - a^2) < (thres / R(i, i))^2: lane r holds the
-    // bound of column bs + r (R's diagonal is positive)
-    double rt2;
-    {
-      const double rt = thres / SR[bs + r][bs + r];
-      rt2 = rt * rt;
-    }
-    bool act = true;
-    int done = BLK, code = 0;
-    double d_r = 0.0, tl_r = 0.0, sc_r = 0.0;
+    const double rt2 = tl[bs + r];
+    double al = 0.0;  // the lane's own pivot
 #pragma unroll
     for (int i = 0; i < BLK; i++) {
-      const int gi = bs + i;
-      const double al = row_bcast(w[i], i);
-      const double aa = fabs(al);
-      const double om = 1.0 - aa;  // 2 - tau
-      const double x2 = fmax(om, 0.0) * (1.0 + aa);  // (||x_i|| / R(i, i))^2
-      const double di = (al >= 0.0) ? -1.0 : 1.0;
-      const double sc = -di * rcp_nr12(1.0 + aa);  // d_i / (-1 - |a_i|)
-      const double rt2i = row_bcast(rt2, i);
-      // non-finite pivot, the truncation test, tau near 2 (dlarfg's tau = 0
-      // branch or lost digits)
-      const int stc = (gi >= nlim) ? 0
-                                   : (!(al == al) ? 2 : ((gi >= 1 && x2 < rt2i) ? 1
-                                                                               : ((om < 1e-6) ? 2 : 0)));
-      const bool go = act && gi < nlim && stc == 0;
-      done = (act && !go) ? i : done;
-      code = (act && !go) ? stc : code;
-      act = go;
-      d_r = (r == i) ? di : d_r;
-      tl_r = (r == i) ? 1.0 + aa : tl_r;
-      sc_r = (r == i) ? sc : sc_r;
-      const double lv = (go && r > i) ? w[i] * sc : 0.0;  // L(r, i)
+      al = r == i ? w[i] : al;
+      const double sc = scale(row_bcast(w[i], i));
+      const double lv = r > i ? w[i] * sc : 0.0;  // L(r, i)
 #pragma unroll
       for (int c = i + 1; c < BLK; c++) w[c] = fma(-lv, row_bcast(w[c], i), w[c]);
-      w[i] = (go && r > i) ? lv : w[i];
+      w[i] = r > i ? lv : w[i];
     }
+    const int gi = bs + r;
+    const double aa = fabs(al), om = 1.0 - aa;  // om: 2 - tau
+    const double x2 = fmax(om, 0.0) * (1.0 + aa);  // (||x|| / R(gi, gi))^2
+    // non-finite pivot, the truncation test, tau near 2 (dlarfg's tau = 0 branch
+    // or lost digits)
+    const int stc = (gi >= nlim) ? 0
+                                 : (!(al == al) ? 2 : ((gi >= 1 && x2 < rt2) ? 1
+                                                                            : ((om < 1e-6) ? 2 : 0)));
+    int code;
+    const int done = block_stop(stc != 0 || gi >= nlim, stc, code);
     if (lane < BLK) {
 #pragma unroll
       for (int c = 0; c < BLK; c++) W[bs + r][bs + c] = w[c];
       if (r < done) {
-        dsg[bs + r] = d_r;
-        tl[bs + r] = tl_r;
-        scv[bs + r] = sc_r;
+        dsg[bs + r] = (al >= 0.0) ? -1.0 : 1.0;
+        tl[bs + r] = 1.0 + aa;
+        scv[bs + r] = scale(al);
       }
     }
     if (lane == 0) {
@@ -301,6 +290,13 @@ __device__ __forceinline__ int lu_signed_blocked(double (*W)[LDP], int nlim, con
       *s_why = code;
     }
   };
+  // ||x_i|| < thres  <=>  (1 - a^2) < (thres / R(i, i))^2: the bound of column i in
+  // tl[i] until wave 0 replaces it (R's diagonal is positive)
+  if (wave == 0) {
+    const double rt = thres / SR[tid][tid];
+    tl[tid] = rt * rt;
+    wave_lds_sync();
+  }
   for (int bs = 0; bs < nlim; bs += BLK) {
     // look-ahead: the previous block's trailing update, wave 0 on this
     // diagonal tile (then its factorisation), waves 1-3 on the other tiles
