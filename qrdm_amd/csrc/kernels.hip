@@ -334,10 +334,8 @@ __device__ __forceinline__ void block_merge_lists(double (*lv)[KMAX], int (*li)[
 
 // Whether the loop ends after the current step (src/dgeqrdm_work.c:782-785):
 // the last column reached, or the stop test met.
-__device__ __forceinline__ int step_done(const DevState* st, int m, int n, int enable_stop,
-                                         double eta) {
-  const int j = st->j, kk = st->fjb_cmp;
-  const double maxnrm = __longlong_as_double((long long)st->maxnrm_bits);
+__device__ __forceinline__ int step_done(int j, int kk, double maxnrm, int m, int n,
+                                         int enable_stop, double eta) {
   const int minmn = m < n ? m : n;
   int done = (j + kk >= minmn) ? 1 : 0;
   if (enable_stop && maxnrm * sqrt((double)(n - j - kk)) <= eta) done = 1;
@@ -346,37 +344,62 @@ __device__ __forceinline__ int step_done(const DevState* st, int m, int n, int e
 
 // End of a DM step (run once, by one thread): ncols, the step record and
 // work, the stop test (enable_stop, eta absolute), the next j, done.
-__device__ void step_end_apply(DevState* st, int* ncols_dev, int m, int n, int enable_stop,
-                               double eta) {
+// What the step's end reads of the state, all loads in flight together (read where
+// they are used, between stores to the same state, each waits for memory in turn).
+struct StepEnd {
+  int pend, done, j, kk, fjb, kmax, nc, nswap, panel, c0, npair, fused, kk_prev, it, flags;
+  double maxnrm, tau, delta;
+  StepWork work;
+};
+__device__ __forceinline__ StepEnd step_end_load(const DevState* st) {
+  StepEnd e;
+  e.pend = st->pend;
+  e.done = st->done;
+  e.j = st->j;
+  e.kk = st->fjb_cmp;
+  e.fjb = st->fjb;
+  e.kmax = st->kmax;
+  e.nc = st->nc;
+  e.nswap = st->nswap;
+  e.panel = st->fast;
+  e.c0 = st->c0;
+  e.npair = st->npair;
+  e.fused = st->fused;
+  e.kk_prev = st->kk_prev;
+  e.it = st->it;
+  e.flags = st->flags;
+  e.maxnrm = __longlong_as_double((long long)st->maxnrm_bits);
+  e.tau = st->tau_step;
+  e.delta = st->delta_step;
+  e.work = st->work;
+  return e;
+}
+__device__ __forceinline__ void step_end_apply(DevState* st, const StepEnd& e, int* ncols_dev,
+                                               int m, int n, int enable_stop, double eta) {
   st->pend = 0;
-  if (st->done) return;
-  const int j = st->j, kk = st->fjb_cmp, fjb = st->fjb;
-  double maxnrm;
-  {
-    const unsigned long long b = st->maxnrm_bits;
-    maxnrm = __longlong_as_double((long long)b);
-  }
+  if (e.done) return;
+  const int j = e.j, kk = e.kk, fjb = e.fjb;
   const int msub = m - j, nsub = n - j;
   StepRec& r = st->last;
   r.j = j;
-  r.kmax = st->kmax;
-  r.nc = st->nc;
+  r.kmax = e.kmax;
+  r.nc = e.nc;
   r.fjb = fjb;
   r.fjb_cmp = kk;
-  r.nswap = st->nswap;
-  r.panel = (st->fast && !(st->flags & 2)) ? 1 : 0;
-  r.maxnrm = maxnrm;
-  r.tau = st->tau_step;
-  r.delta = st->delta_step;
-  const double nct = (double)(n - st->c0);
-  StepWork& w = st->work;
-  w.select += 8.0 * nsub + 8.0 * (double)msub * st->kmax;
-  w.perm += 16.0 * (double)m * st->npair;
+  r.nswap = e.nswap;
+  r.panel = (e.panel && !(e.flags & 2)) ? 1 : 0;
+  r.maxnrm = e.maxnrm;
+  r.tau = e.tau;
+  r.delta = e.delta;
+  const double nct = (double)(n - e.c0);
+  StepWork w = e.work;
+  w.select += 8.0 * nsub + 8.0 * (double)msub * e.kmax;
+  w.perm += 16.0 * (double)m * e.npair;
   w.panel += 2.0 * msub * (double)fjb * fjb;
-  if (st->fused) {
+  if (e.fused) {
     // the step's fused pass: the previous step's update and this step's
     // V^T C on rows j..m of columns c0..n; W = T^T sum and the R12 rows
-    w.gemm1 += 2.0 * msub * nct * (double)(kk + st->kk_prev);
+    w.gemm1 += 2.0 * msub * nct * (double)(kk + e.kk_prev);
     w.wsum += 4.0 * kk * (double)kk * nct;
   } else {
     w.gemm1 += 2.0 * msub * nct * kk;
@@ -384,14 +407,15 @@ __device__ void step_end_apply(DevState* st, int* ncols_dev, int m, int n, int e
     w.gemm2 += 16.0 * msub * nct + 8.0 * msub * kk + 8.0 * kk * nct;
     w.norm += 8.0 * (double)(kk + 2) * (nsub - kk);
   }
+  st->work = w;
   st->kk_prev = kk;
-  const int done = step_done(st, m, n, enable_stop, eta);  // from j before the advance
-  ncols_dev[st->it] = kk;
-  st->it += 1;
+  const int done = step_done(j, kk, e.maxnrm, m, n, enable_stop, eta);  // before the advance
+  ncols_dev[e.it] = kk;
+  st->it = e.it + 1;
   st->j = j + kk;
   st->done = done;
   st->maxnrm_bits = 0ull;
-  st->flags &= ~6;
+  st->flags = e.flags & ~6;
 }
 
 // The step's candidates: the sorted first kmax keys of work[j..n) (value
@@ -415,15 +439,18 @@ __global__ __launch_bounds__(64 * TOPK_WAVES) void k_topk(const double* __restri
   __shared__ int li[TOPK_WAVES][KMAX];
   __shared__ int s_j, s_done, s_end, s_last;
   if (threadIdx.x == 0) {
-    int j = st->j, done = st->done;
-    if (!done && st->pend) {  // the previous step's end, as step_end_apply computes it
-      done = step_done(st, m_all, n_all, enable_stop, eta);
-      j += st->fjb_cmp;
+    // every load before any of them decides (one round trip)
+    const int j0 = st->j, done0 = st->done, pend = st->pend, kk = st->fjb_cmp, halt = st->halt;
+    const double maxnrm = __longlong_as_double((long long)st->maxnrm_bits);
+    int j = j0, done = done0;
+    if (!done0 && pend) {  // the previous step's end, as step_end_apply computes it
+      done = step_done(j0, kk, maxnrm, m_all, n_all, enable_stop, eta);
+      j += kk;
     }
     s_j = j;
-    s_done = dm_stopped(st);  // loop over or halted before this launch: nothing to do
+    s_done = done0 || halt;  // loop over or halted before this launch: nothing to do
     // a halted step's successors stop before their column moves as well
-    if (blockIdx.x == 0 && st->halt == 2) st->halt = 1;
+    if (blockIdx.x == 0 && halt == 2) st->halt = 1;
     s_end = done;       // the loop ends with the pending step: no sort
   }
   __syncthreads();
@@ -455,6 +482,10 @@ __global__ __launch_bounds__(64 * TOPK_WAVES) void k_topk(const double* __restri
   if (threadIdx.x == 0) s_last = last_to_arrive(ticket, nblk) ? 1 : 0;
   __syncthreads();
   if (!s_last) return;
+  // the last wave runs the pending step's end beside the first one's last part
+  const bool ender = threadIdx.x == 64 * (TOPK_WAVES - 1);
+  StepEnd se;
+  if (ender) se = step_end_load(st);
   if (sort) {
     // wave w merges lists w, w + TOPK_WAVES, ... into its own
     v = -1.0;  // a sorted list of padding keys
@@ -474,7 +505,7 @@ __global__ __launch_bounds__(64 * TOPK_WAVES) void k_topk(const double* __restri
     __syncthreads();
     block_merge_lists<TOPK_WAVES>(lv, li, v, ix);
   }
-  if (threadIdx.x == 0 && st->pend) step_end_apply(st, ncols_dev, m_all, n_all, enable_stop, eta);
+  if (ender && se.pend) step_end_apply(st, se, ncols_dev, m_all, n_all, enable_stop, eta);
   if (sort && wave == 0) {
     // k_max = min(nb, m_sub, n_sub) (src/dgeqrdm_work.c:703), at most KMAX here
     int kmax = nb < KMAX ? nb : KMAX;
@@ -1658,7 +1689,8 @@ void launch_norm_update(const double* A, int lda, int j0, int m, int n, double* 
 // otherwise).
 __global__ void k_step_end(DevState* st, int* ncols_dev, int m, int n, int enable_stop,
                            double eta) {
-  if (st->pend) step_end_apply(st, ncols_dev, m, n, enable_stop, eta);
+  const StepEnd e = step_end_load(st);
+  if (e.pend) step_end_apply(st, e, ncols_dev, m, n, enable_stop, eta);
 }
 
 void launch_step_end(DevState* st, int* ncols_dev, int m, int n, int enable_stop, double eta,
