@@ -748,12 +748,17 @@ __global__ __launch_bounds__(256) void k_gram_cand(double* A, int lda, int m, do
                                                    const DevState* st, StepBufs bufs) {
   __shared__ double Ws[KMAX][KMAX + 1];       // W_prev(i, candidate c) at Ws[i][c]
   __shared__ double Gp[4][10][4][64];         // each wave's tiles, in its lanes' layout
-  if (dm_stopped(st)) return;
-  const int j = st->j;
   // the greedy takes candidate 0 even when nc is 0 (all norms zero), so it
   // receives the update too; the cosines read the Gram only when nc > 1
-  const int nc = max(st->nc, 1);
   const int tid = local_tid(), lane = tid & 63, wv = tid >> 6, g = lane >> 4, li = lane & 15;
+  // all of the state in one round trip
+  const int j = st->j, nc = max(st->nc, 1), stopped = st->done | st->halt;
+  int cidx[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++) cidx[u] = st->cand_idx[16 * u + li];
+  asm volatile("" ::"s"(j), "s"(nc), "s"(stopped), "v"(cidx[0]), "v"(cidx[1]), "v"(cidx[2]),
+               "v"(cidx[3]));
+  if (stopped) return;
   // wave wv takes rows rb .. rb + 15 of the workgroup's 64-row slab, read
   // straight into the matrix cores' layout: X(rb + g + 4v, candidate 16u + li)
   const int rb = j + blockIdx.x * GRAM_ROWS + 16 * wv;
@@ -764,7 +769,7 @@ __global__ __launch_bounds__(256) void k_gram_cand(double* A, int lda, int m, do
   for (int u = 0; u < 4; u++) {
     const int c = 16 * u + li;
     cok[u] = c < nc;
-    cc[u] = A + (size_t)(j + (cok[u] ? st->cand_idx[c] : 0)) * lda;
+    cc[u] = A + (size_t)(j + (cok[u] ? cidx[u] : 0)) * lda;
   }
   dbl4 xb[4];
 #pragma unroll
@@ -1156,9 +1161,10 @@ __device__ __forceinline__ void larft_recurrence(const double* Ss, double* Ts, c
 // Trailing update (LAPACKE_dlarfb_mia, src/dlarfb.c:142 -> dlarfb 'L','T','F',
 // 'C'): C := C - V (C^T V T)^T on rows [j, m), columns [c0, n); with
 // trans = 0 the block reflector itself, C := C - V T V^T C.
-//   k_gemm1: W = op(T) V^T C, the rows split in slabs; each workgroup writes
-//            its slab's partial V^T C, the last one of a column tile (atomic
-//            ticket) sums the partials in slab order and applies op(T);
+// The three-kernel form of the reduced precisions and QRDM_TRAILING=3pass
+// (trailing.hip holds the merged pass that every other caller takes):
+//   k_gemm1: the partial products V^T C, the rows split in slabs;
+//   k_wsum:  W = op(T) sum of them in slab order;
 //   k_gemm2: C -= V W.
 // Matrix cores: v_mfma_f64_16x16x4f64, D(16x16) += A(16x4) B(4x16); lane l
 // holds A[l%16][l/16], B[l/16][l%16] and D[l/16 + 4*v][l%16], v = 0..3 (the

@@ -23,8 +23,9 @@
 //         src/dgeqr2.c:176-177);
 //   k_v2     V2 = P_bottom M (matrix cores), written into the panel and into
 //         the dense V the trailing update reads, with V^T V per slab;
-//   k_reduce_t  tau and T from V^T V (the compact WY identity), so that the
-//         block reflector is orthogonal for the V stored.
+// tau and T^-1 follow from V^T V (the compact WY identity), so that the block
+// reflector is orthogonal for the V stored: summed in the merged pass
+// (trailing.hip); for the three-kernel update k_reduce_t forms T.
 // Columns the truncation rejects keep their original values; the caller's
 // trailing update then starts at j + fjb_cmp and applies the kept reflectors
 // to them, as dlarf_ did inside the reference's panel.
@@ -753,9 +754,10 @@ __global__ __launch_bounds__(256) void k_qgram(const double* __restrict__ A, int
                                                const DevState* st, double* partial) {
   __shared__ double Ri[KMAX][LDP];
   __shared__ double Gp[4][10][4][64];
-  if (!step_runs(st, RUN_FAST)) return;
-  const int j = st->j;
-  const int k1 = st->k1;
+  const int j = st->j, k1 = st->k1;
+  const bool runs = step_runs(st, RUN_FAST);
+  asm volatile("" ::"s"(j), "s"(k1), "s"((int)runs));  // the state in one round trip
+  if (!runs) return;
   const int tid = local_tid(), lane = tid & 63, wv = tid >> 6, g = lane >> 4, li = lane & 15;
   const int rb = j + blockIdx.x * PR_ROWS + 16 * wv;
   load_mat(Ri, R1inv);
@@ -965,7 +967,7 @@ __device__ __forceinline__ int recon_core(double (*SR)[LDP], double (*SA)[LDP], 
   // 8. M = R^-1 D U^-1, upper triangular, computed transposed (lower) so that
   // consecutive lanes store consecutive rows: the TRI_UU jobs with the tile
   // indices swapped; the tiles below the diagonal blocks are zero.  (T and
-  // tau follow from the V that k_v2 stores, k_reduce_t.)
+  // tau follow from the V that k_v2 stores: the merged pass, or k_reduce_t.)
   {
     const int lane = tid & 63, wv = tid >> 6, li = lane & 15, g = lane >> 4;
     TileJob jt[4];
@@ -1036,9 +1038,9 @@ __device__ __forceinline__ void recon_inputs(ReconIn& in, const DevState* st,
 __device__ __forceinline__ void recon_body(const double* __restrict__ G2, const ReconIn& rin,
                                            double* A, int lda, double tau_dm, double* tau,
                                            DevState* st, double* M_out) {
-  __shared__ double SR[KMAX][LDP];  // R1, then R, then L^T, then U^-1 (rows scaled by D)
+  __shared__ double SR[KMAX][LDP];  // R1, then R, then U^-1 (rows scaled by D)
   __shared__ double SA[KMAX][LDP];  // R^-1
-  __shared__ double SW[KMAX][LDP];  // E, R2^-1, then Q11 and its LU, then L^-T
+  __shared__ double SW[KMAX][LDP];  // E, R2^-1, then Q11 and its LU
   __shared__ double SX[KMAX][LDP];  // G2, F or R2, R1^-1, then U
   __shared__ double Y[4][BLK][BLK + 1];
   __shared__ double rinv[KMAX], dsg[KMAX], tl[KMAX], scv[KMAX];
@@ -1126,11 +1128,12 @@ __global__ __launch_bounds__(256) void k_v2(double* A, int lda, int m,
                                             DevState* st, StepBufs bufs, double* gram_part) {
   __shared__ double Ms[KMAX][LDP];
   __shared__ double Gp[4][10][4][64];
-  if (!step_runs(st, RUN_FAST)) return;
-  double* V = v_cur(bufs, st);
   const int ldv = bufs.ldv;
-  const int j = st->j;
-  const int k = st->fjb_cmp;
+  const int j = st->j, k = st->fjb_cmp;
+  double* V = v_cur(bufs, st);
+  const bool runs = step_runs(st, RUN_FAST);
+  asm volatile("" ::"s"(j), "s"(k), "s"(V), "s"((int)runs));  // the state in one round trip
+  if (!runs) return;
   const int tid = local_tid(), lane = tid & 63, wv = tid >> 6, g = lane >> 4, li = lane & 15;
   const int rs = j + blockIdx.x * PR_ROWS;
   if (rs >= m) return;

@@ -211,14 +211,18 @@ __device__ __forceinline__ bool last_to_arrive(unsigned* ticket, unsigned n) {
 enum RunMode { RUN_ALWAYS = 0, RUN_DM = 1, RUN_EXACT = 2, RUN_FAST = 3 };
 
 // The DM loop has ended, or waits for the host to resume a halted step.
-__device__ __forceinline__ bool dm_stopped(const DevState* st) { return st->done || st->halt; }
+// (bitwise: the loads go out together; one after the other each is a round trip
+// before a kernel's first data load)
+__device__ __forceinline__ bool dm_stopped(const DevState* st) {
+  return (st->done | st->halt) != 0;
+}
 
 __device__ __forceinline__ bool step_runs(const DevState* st, int mode) {
   if (mode == RUN_ALWAYS) return true;
-  if (dm_stopped(st)) return false;
-  if (mode == RUN_EXACT) return !st->fast || (st->flags & 2);
-  if (mode == RUN_FAST) return st->fast && !(st->flags & 2);
-  return true;
+  const int stop = st->done | st->halt, fast = st->fast, fell = st->flags & 2;
+  const int form = (fast != 0) & (fell == 0);  // the Gram-based panel
+  const int runs = mode == RUN_EXACT ? form ^ 1 : (mode == RUN_FAST ? form : 1);
+  return ((stop == 0) & runs) != 0;
 }
 
 // ---- launchers (kernels.hip) ------------------------------------------------

@@ -18,8 +18,9 @@
 // diagonal, V to the left), through LDS; the rest is written once, at the end,
 // with the dense V of the trailing update.  One wave that holds no rows builds
 // T's diagonal blocks from those entries beside the others' updates.  Panels of
-// more than RP_ROWS rows take a workgroup per RP_HALF (or RP_ROWS) rows: every column's partial sums pass between the workgroups through
-// memory, each a slot of its own that holds a sentinel until it is written.
+// more than RP_ROWS rows take a workgroup per RP_HALF (or RP_ROWS) rows: every
+// column's partial sums pass between the workgroups through memory, each in a slot
+// that holds a sentinel until it is written.
 //
 // Measured for 64 columns, with V and T (rocprofv3): up to 128 rows 65 us, up
 // to 448 rows 104 us (memory-based: about 180 us for 64 rows, with T another

@@ -205,11 +205,14 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   // that a load on its way into one does not hold up reads of the other)
   __shared__ FuChunk vp0, vp1, vn0, vn1;
   if (st) {
-    if (dm_stopped(st)) return;
-    if (!st->given) {
-      r_lo = st->j;
-      c0 = st->c0;
-      cur = st->it & 1;
+    const int stopped = st->done | st->halt, given = st->given, j = st->j, sc0 = st->c0,
+              it = st->it;
+    asm volatile("" ::"s"(stopped), "s"(given), "s"(j), "s"(sc0), "s"(it));  // one round trip
+    if (stopped) return;
+    if (!given) {
+      r_lo = j;
+      c0 = sc0;
+      cur = it & 1;
       ns = fused_slabs_wave(r_lo, m, c0, n);
     }
   }
@@ -485,17 +488,19 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
   __shared__ double s_wk[WN_TC], s_wo[WN_TC];  // work, workold of the tile's columns
   __shared__ unsigned long long s_rows[4];
   __shared__ int s_rec[WN_TC];
-  if (dm_stopped(st)) return;
+  const int j = st->j, kk = st->fjb_cmp, c0 = st->c0, it = st->it;
+  const int stopped = st->done | st->halt;
+  asm volatile("" ::"s"(j), "s"(kk), "s"(c0), "s"(it), "s"(stopped));  // one round trip
+  if (stopped) return;
   // the step's end is pending from here on (run by the next k_topk or k_step_end)
   if (blockIdx.x == 0 && threadIdx.x == 0) st->pend = 1;
-  const int j = st->j, kk = st->fjb_cmp, c0 = st->c0;
   const int jn = j + kk;
   const int cb = jn + blockIdx.x * WN_TC;
   if (cb >= n) return;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, li = lane & 15;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const double* V = v_cur(bufs, st);
-  double* W = w_cur(bufs, st);
+  const double* V = bufs.V + (size_t)(it & 1) * bufs.vstride;
+  double* W = bufs.W + (size_t)(it & 1) * bufs.wstride;
   const int ldv = bufs.ldv, ldw = n - c0, ns = fused_slabs_wave(j, m, c0, n);
   const int col = cb + li, cl = min(col, n - 1);  // the lane's column
   // every global read of the prologue in flight together: T^-1, the first

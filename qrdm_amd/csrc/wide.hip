@@ -18,9 +18,10 @@
 //                  path: |G(q, t) / norm_q / norm_t| >= delta marks a conflict;
 //   k_swap_pairs   the column moves of permute_marked's walk (computed on the
 //                  host, src/dgeqrdm_work.c:149-262), with work and jpvt;
-// then the column-by-column panel (regpanel.hip), 64 columns at a time, the block reflector applied in 64-column chunks of the kept
-// reflectors (the same product H_0 .. H_{k-1} as one dlarfb of width k), and
-// the norm downdate over the step's fjb_cmp new rows.
+// then the column-by-column panel (regpanel.hip), 64 columns at a time, the block
+// reflector applied in 64-column chunks of the kept reflectors (the same product
+// H_0 .. H_{k-1} as one dlarfb of width k), and the norm downdate over the step's
+// fjb_cmp new rows.
 #include "qrdm_internal.h"
 
 #include <climits>
