@@ -626,24 +626,32 @@ int run_dm(const Args& x) {
       HIPCHK(hipMemcpyAsync(hb[q], B.st, sizeof(DevState), hipMemcpyDeviceToHost, s));
       if (evs) HIPCHK(hipEventRecord(evs[q], s));
     };
-    // Steps of a batch from column jl: as many as blocks of nb columns need to
-    // end the loop, and one more where several do (the truncation shortens
-    // blocks now and then), at most kBatch.  A step queued past the end still
-    // costs its eight launches, 20 us: 64 x 48 takes 1 step, not 8.
-    auto batch_steps = [&](int jl) {
+    // Steps of a batch that starts between the columns jl and jmax: as many as
+    // blocks of nb columns need to end the loop, and one more where several do (the
+    // truncation shortens blocks now and then), at most kBatch.  A step queued past
+    // the end still costs its eight launches, 20 us: 64 x 48 takes 1 step, not 8.
+    // A batch of tall panels ends before a step's panel could be a short one: that
+    // step halts, and the launches queued behind it cost as much.
+    const int nbw = std::min(nb, KMAX);
+    auto tall_from = [&](int jl) { return m - jl >= kFastPanelRows && !force_exact; };
+    auto batch_steps = [&](int jl, int jmax) {
       if (x.trace) return 1;
       const int blocks = (minmn - jl + nb - 1) / nb;
-      return std::min(kBatch, blocks > 1 ? blocks + 1 : 1);
+      const int steps = std::min(kBatch, blocks > 1 ? blocks + 1 : 1);
+      if (!tall_from(jl)) return steps;
+      const int room = m - kFastPanelRows - jmax;
+      return room < 0 ? 0 : std::min(steps, room / nbw + 1);
     };
-    auto queue_batch = [&](int jl, int q) {
+    auto queue_batch = [&](int jl, int jmax, int q) {
       // Tall panels: Gram-based Householder reconstruction (panel.hip), which
       // also leaves V and T for the trailing update, its first Cholesky beside
       // the column moves; the exact panel is not queued, and a step that
       // needs it (short panel, fjb < 2, or the Gram-based form falling back)
       // halts until the host resumes it.  Short panels: the column-by-column
       // exact panel, then dlarft.
-      const bool tall = m - jl >= kFastPanelRows && !force_exact;
-      const int steps = batch_steps(jl);
+      const bool tall = tall_from(jl);
+      const int steps = batch_steps(jl, jmax);
+      if (steps == 0) return 0;
       for (int b = 0; b < steps; b++) queue_step(jl, tall);
       readback(q);
       return steps;
@@ -658,13 +666,13 @@ int run_dm(const Args& x) {
     // is queued before its state is read back, so the device does not idle
     // through the readback; its grids are sized from the same lower bound.
     int q = 0, jend = j0;
-    int steps = queue_batch(j0, q);  // of the batch waited for
+    int steps = queue_batch(j0, j0, q);  // of the batch waited for
     while (true) {
       const bool ahead = !x.trace && !switch_wanted && j0 + steps * KMAX < minmn;
-      const int steps_ahead = ahead ? queue_batch(j0, q ^ 1) : 0;
+      const int steps_ahead = ahead ? queue_batch(j0, j0 + steps * nbw, q ^ 1) : 0;
       DevState* h = wait_slot(q);
       check_panels(h->flags);
-      bool in_flight = ahead;
+      bool in_flight = steps_ahead > 0;
       if (h->halt) {
         // the halted step (at h->j, selection and column moves done)
         // continues with the exact panel, after the batch queued behind it
@@ -723,7 +731,7 @@ int run_dm(const Args& x) {
           prec_now = low;
           switch_wanted = false;
         }
-        steps = queue_batch(j0, q);
+        steps = queue_batch(j0, j0, q);
       }
     }
     if (fused_now && it > 0) {
