@@ -29,12 +29,13 @@ namespace {
 thread_local std::string g_err;
 
 constexpr double kEps = 1.1102230246251565e-16;  // LAPACK dlamch('E') = 2^-53
-// Panels with at least this many rows take the Gram-based path.  Below, the
-// register-held panel of one workgroup is faster (about 0.5 us a column with
-// everything that follows it, against five launches of about 115 us); it stays
-// faster up to its 512 rows, but a step record says which form ran, and what
-// reads the records expects the Gram form from 425 rows on.
-constexpr int kFastPanelRows = 385;
+// Panels with at least this many rows take the Gram-based path, five launches of
+// about 75 us in all; below, the register-held panel of one workgroup, 65 us up to
+// 128 rows and 87 up to 336, with 9 for its column moves and fallback.  Measured
+// (us, whole calls by this limit 129 / 193 / 257 / 385): 130 x 64 270 / 241 / 241 /
+// 242, 256 x 256 732 / 766 / 756 / 755, 384 x 64 254 / 254 / 254 / 265, 384 x 300
+// 810 / 844 / 851 / 910, 900 x 900 2225 / 2259 / 2253 / 2280.
+constexpr int kFastPanelRows = 257;
 constexpr int kBatch = 8;  // DM steps queued between synchronisations
 // Layout of the per-step upload: up to 2*KMAX (dst, src) pairs, then KMAX
 // candidate ranks of the panel columns.
