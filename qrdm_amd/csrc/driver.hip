@@ -801,9 +801,9 @@ int run_ormqr(int trans, int m, int n, int k, const double* A, int lda, const do
   for (int q = 0; q < nblk; q++) {
     const int b = trans ? q : nblk - 1 - q;  // Q^T: H(0) first; Q: H(k-1) first
     const int j = b * KMAX, cur = b & 1;
-    const int kb = (k - j) < KMAX ? (k - j) : KMAX;
-    launch_panel_exact(const_cast<double*>(A), lda, j, m, kb, 0.0, PANEL_GIVEN,
-                       const_cast<double*>(tau) + j, B.st, s);
+    if (q == 0)  // the later ones' V comes with the W of the block before
+      launch_panel_exact(const_cast<double*>(A), lda, j, m, k, 0.0, PANEL_GIVEN,
+                         const_cast<double*>(tau), B.st, s);
     const int r = q > 0 ? std::min(j, jp) : j, ns = fused_slabs(r, m, 0, n);
     launch_fused(C, ldc, r, m, 0, n, bufs, B.Wp, ns, q > 0, 1, cur, s, B.st);
     launch_wsum(j, m, 0, n, nullptr, trans, B.Wp, B.Wf + cur * bufs.wstride, ns, s, B.st);

@@ -1598,7 +1598,8 @@ void launch_wsum(int j, int m, int c0, int n, const double* T, int trans, const 
   const int ncol = n - c0, mrow = m - j;
   if (ncol <= 0 || mrow <= 0) return;
   if (!T) {
-    launch_wsum_fused(c0, n, nullptr, trans, Wp, W, nsplit, s, st);
+    launch_wsum_fused(c0, n, nullptr, trans, Wp, W, nsplit, trans ? j + KMAX : j - KMAX, m, s,
+                      st);
     return;
   }
   const G1Geom g = gemm1_geom(j, m, c0, n, nsplit);

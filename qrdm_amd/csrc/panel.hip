@@ -1186,34 +1186,33 @@ __global__ __launch_bounds__(256) void k_v2(double* A, int lda, int m,
   gram_sum_store(gt, Gp, gram_part + (size_t)blockIdx.x * KMAX * KMAX);
 }
 
-// The block reflector of a factored panel (A below the diagonal, tau): the dense
-// V of columns [j, j + k) into buffer (j / KMAX) & 1 -- zero on the 64 rows above
-// the panel and from m to ws_ldv(m) -- and each 64-row slab's part of V^T V into
-// the slots, for the merged pass (trailing.hip) to sum beside its first loads.
-// One launch of up to a workgroup per 64 rows, 8 us at 4096 rows, in place of
-// four (the copy of V one row per thread over all 64 columns, the Gram from it,
-// its sum, and dlarft's recurrence in one workgroup: 147 us).
-__global__ __launch_bounds__(256) void k_given_panel(const double* __restrict__ A, int lda, int j,
-                                                     int m, int k, const double* tau,
-                                                     DevState* st) {
-  __shared__ double Gp[4][10][4][64];
+// The block reflector of factored columns (A below the diagonal, tau): the dense V
+// of columns [j, j + KMAX), those below given_k, into buffer (j / KMAX) & 1 -- zero
+// on the 64 rows above the panel and from m to ws_ldv(m) -- and each 64-row slab's
+// part of V^T V into the slots, for the merged pass (trailing.hip) to sum beside its
+// first loads.  blk: the 64-row slab; 256 threads.  9 us at 4096 rows in place of
+// four launches (the copy of V one row per thread over all 64 columns, the Gram from
+// it, its sum, and dlarft's recurrence in one workgroup: 147 us); from the second
+// block on beside the block before's W, which needs none of it (k_wsum_fused).
+__device__ __forceinline__ void given_panel(int j, int m, int blk, DevState* st,
+                                            double (*Gp)[10][4][64]) {
   const int tid = local_tid(), lane = tid & 63, wv = tid >> 6, g = lane >> 4, li = lane & 15;
+  const int k = min(KMAX, st->given_k - j), lda = st->given_lda;
+  if (k <= 0) return;  // no such block
+  const double* __restrict__ A = st->given_a;
   const int ldv = ws_ldv(m), cur = (j / KMAX) & 1;
   double* V = ws_v(st, m) + (size_t)cur * ldv * KMAX;
-  if (blockIdx.x == 0) {
+  if (blk == 0) {
     if (tid == 0) {
       st->j = j;
       st->fjb_cmp = k;
-      st->fast = 1;
-      st->given = 1;
-      st->tau_base = const_cast<double*>(tau) - j;
     }
     for (int e = tid; e < KMAX * KMAX; e += 256) {
       const int r = j - KMAX + (e & 63), c = e >> 6;
       if (r >= 0) V[(size_t)c * ldv + r] = 0.0;
     }
   }
-  const int rb = j + blockIdx.x * PR_ROWS + 16 * wv;
+  const int rb = j + blk * PR_ROWS + 16 * wv;
   dbl4p vb[4];
 #pragma unroll
   for (int u = 0; u < 4; u++)
@@ -1233,13 +1232,29 @@ __global__ __launch_bounds__(256) void k_given_panel(const double* __restrict__ 
 #pragma unroll
   for (int p = 0; p < 10; p++) gt[p] = (dbl4p){0.0, 0.0, 0.0, 0.0};
   gram_tiles(vb, gt);
-  gram_sum_store(gt, Gp, ws_slots(st) + (size_t)blockIdx.x * KMAX * KMAX);
+  gram_sum_store(gt, Gp, ws_slots(st) + (size_t)blk * KMAX * KMAX);
+}
+
+// What the given columns are, before the first block's launch.
+__global__ void k_given_begin(const double* A, int lda, int k, double* tau, DevState* st) {
+  st->fast = 1;
+  st->given_k = k;
+  st->given_lda = lda;
+  st->given_a = A;
+  st->tau_base = tau;
+}
+
+__global__ __launch_bounds__(256) void k_given_panel(int j, int m, DevState* st) {
+  __shared__ double Gp[4][10][4][64];
+  given_panel(j, m, blockIdx.x, st, Gp);
 }
 
 void launch_given_panel(const double* A, int lda, int j, int m, int k, const double* tau,
                         DevState* st, hipStream_t s) {
-  hipLaunchKernelGGL(k_given_panel, dim3((m - j + PR_ROWS - 1) / PR_ROWS), dim3(256), 0, s, A, lda,
-                     j, m, k, tau, st);
+  hipLaunchKernelGGL(k_given_begin, dim3(1), dim3(1), 0, s, A, lda, k, const_cast<double*>(tau),
+                     st);
+  hipLaunchKernelGGL(k_given_panel, dim3((m - j + PR_ROWS - 1) / PR_ROWS), dim3(256), 0, s, j, m,
+                     st);
 }
 
 // The block reflector of the Gram-based panel from the V it stored: S = V^T V

@@ -38,6 +38,9 @@ struct DevState {
   int flags;       // bit 0: non-finite value met; bit 1: fast panel fell back; bit 2: the
                    // register-held panel declined; bit 3: its workgroups gave up waiting
   int k1;          // columns the fast panel's first Cholesky factored
+  int given_k;     // > 0: V and tau are those of so many factored columns (ormqr) at
+                   // given_a; the merged pass leaves tau as it is and takes its geometry
+                   // from the host
   unsigned long long maxnrm_bits;  // max partial norm (bit pattern, >= 0)
   unsigned long long recomp_rows;  // rows read by norm recomputes (profiling)
   int sel[KMAX];        // accepted columns (relative to j), acceptance order
@@ -62,10 +65,12 @@ struct DevState {
   int kk_prev;  // fjb_cmp of the previous step (0 before the first): the width of the
                 // update the fused pass applies
   int policy_on;      // 1: the step's tau and delta come from the learned policy
-  double pan_beta;    // R(0, 0) of the last column-by-column panel (wide.hip's blocks)
+  int given_lda;
+  union {
+    double pan_beta;        // R(0, 0) of the last column-by-column panel (wide.hip's blocks)
+    const double* given_a;  // the given columns
+  };
   double* tau_base;   // tau[0..min(m, n)) (set by the Gram-based panel)
-  int given;          // 1: V and tau are a factored panel's (ormqr); the merged pass leaves
-                      // tau as it is and takes its geometry from the host
   double tau_step;    // tau and delta of the current step (the defaults, or the
   double delta_step;  // policy's proposal)
   StepRec last;
@@ -264,9 +269,10 @@ void launch_apply_perm(double* A, int lda, int m, double* work, int* jp, const i
 // the dense V (rows max(j - KMAX, 0) .. m of ws_v, of the step's parity with
 // st->fused) and T (ws_mat), and uses the Gram partials' space.  truncate: 0
 // none, 1 the DM test, 2 the DM test of a panel that continues a wider block.
-// PANEL_GIVEN: the columns are factored already; A and tau are only read, and V
-// (of buffer j / KMAX & 1, rows up to ws_ldv(m), j a multiple of KMAX) and the
-// partial V^T V (slots) are written, from which the merged pass forms T^-1.
+// PANEL_GIVEN: the fjb columns from 0 on, any number, are factored already (tau from
+// its first entry); A and tau are only read, and of the KMAX columns from j on, j a
+// multiple of KMAX, V (buffer j / KMAX & 1, rows up to ws_ldv(m)) and the partial
+// V^T V (slots) are written, from which the merged pass forms T^-1.
 constexpr int PANEL_GIVEN = 3;
 void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm,
                         int truncate, double* tau, DevState* st, hipStream_t s,
@@ -331,15 +337,17 @@ void launch_policy_predict(const void* net, const float* x, int ns, float* out, 
 // The three-kernel update's first two launches: the partial products Wp = V^T C per row
 // slab, then W = op(T) sum Wp.  launch_wsum with T = nullptr: the partials
 // of a merged pass (launch_fused) over columns [c0, n), nsplit its slabs; W by
-// absolute column (KMAX x n), from the T^-1 behind st.
+// absolute column (KMAX x n), from the T^-1 behind st; and V and the partial V^T V
+// of the given columns' next block, after (trans) or before column j.
 void launch_gemm1(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
                   double* Wp, int nsplit, hipStream_t s, const DevState* st);
 void launch_wsum(int j, int m, int c0, int n, const double* T, int trans, const double* Wp,
                  double* W, int nsplit, hipStream_t s, const DevState* st);
 // W = op(T) sum Wp (64 x n by absolute column) from a merged pass's ns slabs over
-// columns [c0, n); T = nullptr: from the T^-1 behind st.
+// columns [c0, n); T = nullptr: from the T^-1 behind st, with the block from column
+// jnext on (rows to m; < 0: none) of the given columns beside it.
 void launch_wsum_fused(int c0, int n, const double* T, int trans, const double* Wp, double* W,
-                       int ns, hipStream_t s, const DevState* st);
+                       int ns, int jnext, int m, hipStream_t s, const DevState* st);
 // Norm downdate of columns [j + fjb_cmp, n) (j, fjb_cmp from st; j0 <= j
 // sizes the grid).
 void launch_norm_update(const double* A, int lda, int j0, int m, int n, double* work,
