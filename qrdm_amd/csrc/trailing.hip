@@ -25,9 +25,11 @@
 // entries contiguous); V and W of two consecutive steps alternate between two
 // buffers (st->it & 1).
 //
-// Rounding: V W is summed from zero and then added to C, as in the one-step
-// form (summed into C on the matrix cores, formq 4096 x 2048 was off by 2.3e-15
-// of its norm instead of 1.7e-15, at the same speed).
+// Rounding: V W is summed from zero and then added to C, in every pass and at the
+// step's end (R12, the recomputed columns): an entry of C is rounded once.  Summed
+// into C on the matrix cores formq 4096 x 2048 was off by 2.3e-15 of its norm instead
+// of 1.7e-15, and a recomputed column's small rows by several units in the last
+// place instead of half a unit, at the same speed.
 #include "qrdm_internal.h"
 
 #include <algorithm>
@@ -544,7 +546,7 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
   }
   lds_barrier();
 #pragma unroll
-  for (int t = 0; t < KMAX / 4; t++) va[t] = rt < kk ? -va[t] : 0.0;
+  for (int t = 0; t < KMAX / 4; t++) va[t] = rt < kk ? va[t] : 0.0;
   // one wave inverts the diagonal blocks while the others wait for their loads
   if (wv == 3) diag_inverse(Us, s_rd, Di);
   {
@@ -564,9 +566,11 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
   lds_barrier();
   if (wv == 0) wy_solve<true>(Us, Di, S1);
   lds_barrier();
+  dbl4 vw = (dbl4){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int t = 0; t < KMAX / 4; t++)
-    r12 = __builtin_amdgcn_mfma_f64_16x16x4f64(va[t], S1[4 * t + g][li], r12, 0, 0, 0);
+    vw = __builtin_amdgcn_mfma_f64_16x16x4f64(va[t], S1[4 * t + g][li], vw, 0, 0, 0);
+  r12 -= vw;
   double sq = 0.0;
 #pragma unroll
   for (int v = 0; v < 4; v++) {
@@ -616,21 +620,22 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
 #pragma unroll
       for (int t = 0; t < KMAX / 4; t++)
         vb[t] = V[(size_t)(4 * t + g) * ldv + min(ra, m - 1)];  // V(ra, 4t + g)
-      dbl4 d;
+      dbl4 x, d = (dbl4){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int r = rb + g + 4 * v;
-        d[v] = A[(size_t)cl * lda + min(r, m - 1)];
+        x[v] = A[(size_t)cl * lda + min(r, m - 1)];
       }
 #pragma unroll
       for (int t = 0; t < KMAX / 4; t++)
-        d = __builtin_amdgcn_mfma_f64_16x16x4f64(-vb[t], S1[4 * t + g][li], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(vb[t], S1[4 * t + g][li], d, 0, 0, 0);
+      x -= d;
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int r = rb + g + 4 * v;
         if (rec && r < m) {
-          A[(size_t)cl * lda + r] = d[v];
-          ps = fma(d[v], d[v], ps);
+          A[(size_t)cl * lda + r] = x[v];
+          ps = fma(x[v], x[v], ps);
         }
       }
     }
