@@ -186,6 +186,13 @@ __device__ __forceinline__ void sum_gram(const DevState* st, int m) {
 // 1.64.  Odd leading dimensions run here too (3001 x 1777 DM 6.53 -> 6.06 ms
 // against the three-kernel form with 8-byte loads).
 //
+// V^T C is summed in pieces of two chunks: the error of one running sum grows with
+// its rows, and how many row slabs there are follows from the chip, not from that
+// (2 to 4 for 8192 columns and more, 2048 rows and more in one sum).  Relative error
+// of an update, pieces of 64 rows / slabs in one sum: Q C with C
+// 8192 x 8192, 256 reflectors 2.0e-16 / 6.6e-16, unpivoted QR 4096 x 8192 2.7e-16 /
+// 9.7e-16, DM 8192 x 8192 3.4e-16 / 1.3e-15; a pass takes as long with as without.
+//
 // V is zero above its panel (within 64 rows) and past m, which the callers
 // keep so: no masks in the products, only the stores look at r_lo and m.  W is
 // indexed by absolute columns; the partials, ns slabs, by the columns from c0 on (a
@@ -255,9 +262,9 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
 #pragma unroll
     for (int s = 0; s < 16; s++) wr[s] = cok ? -wr[s] : 0.0;
   }
-  dbl4 acc[4];
+  dbl4 acc[4], tot[4];  // V^T C of two chunks, of the slab
 #pragma unroll
-  for (int t = 0; t < 4; t++) acc[t] = (dbl4){0.0, 0.0, 0.0, 0.0};
+  for (int t = 0; t < 4; t++) acc[t] = tot[t] = (dbl4){0.0, 0.0, 0.0, 0.0};
   // chunk c of V into LDS: a wave takes the columns 16 w .. 16 w + 15, four
   // per load (lane: column lane / 16, unit lane % 16): the lane's byte offsets
   // from the wave's first column
@@ -372,6 +379,13 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   for (int c = ch0; c < ch1; c += 2) {
     step(c, vp0, vn0, vp1, vn1, x);
     if (c + 1 < ch1) step(c + 1, vp1, vn1, vp0, vn0, x);
+    if (ACCUM) {
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        tot[t] += acc[t];
+        acc[t] = (dbl4){0.0, 0.0, 0.0, 0.0};
+      }
+    }
   }
   if (!ACCUM || !cok) return;
   // partial tile: row 16t + g + 4w of the lane's column
@@ -379,7 +393,7 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
 #pragma unroll
   for (int t = 0; t < 4; t++)
 #pragma unroll
-    for (int w = 0; w < 4; w++) out[(size_t)(16 * t + g + 4 * w) * ldw] = acc[t][w];
+    for (int w = 0; w < 4; w++) out[(size_t)(16 * t + g + 4 * w) * ldw] = tot[t][w];
 }
 
 int fused_max_slabs() { return FU_MAX_SPLIT; }
