@@ -83,6 +83,10 @@ __device__ __forceinline__ double bt_v(const double* a, int lda, int j, int kk, 
 // matrices up to 1024 x 512 (8.87 -> 7.08 ms): 2.2 ms, about 11 GB in all, against
 // 2.95 with V read per wave and no loads in flight across chunks, and 4.7 with one
 // chunk in flight and 64 columns.
+//
+// P is summed in pieces of two chunks, as in the merged pass: one running sum down
+// the rows was off by 1.2e-15 of the result at 1024 x 512, this by 5.4e-16 (four
+// waves' sums 7.2e-16), for 0.06 ms of the launch above.
 template <int NW>
 __device__ __forceinline__ void bt_trailing(double* a, int lda, int j, int m, int kk, int c0, int n,
                             BatchLds<NW>& L) {
@@ -168,11 +172,11 @@ __device__ __forceinline__ void bt_trailing(double* a, int lda, int j, int m, in
         S[ch & 1][c][li ^ (c & 15)] = v;
       }
     };
-    dbl4 acc[U][4];
+    dbl4 acc[U][4], tot[U][4];  // P of two chunks, of all
 #pragma unroll
     for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int t = 0; t < 4; t++) acc[u][t] = (dbl4){0.0, 0.0, 0.0, 0.0};
+      for (int t = 0; t < 4; t++) acc[u][t] = tot[u][t] = (dbl4){0.0, 0.0, 0.0, 0.0};
     // chunk ch's products; x0: chunk ch (V stored already), x1: ch + 1, which
     // follows into LDS; ch + 2 is fetched over x0
     auto down = [&](int ch, Regs& x0, Regs& x1) {
@@ -209,11 +213,18 @@ __device__ __forceinline__ void bt_trailing(double* a, int lda, int j, int m, in
     for (int ch = 0; ch < nch; ch += 2) {
       down(ch, xa, xb);
       if (ch + 1 < nch) down(ch + 1, xb, xa);
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          tot[u][t] += acc[u][t];
+          acc[u][t] = (dbl4){0.0, 0.0, 0.0, 0.0};
+        }
     }
     // back from the last chunk, in LDS still
     load(nch - 1, xa);
     load(nch - 2, xb);
-    // P's rows 16 t + g + 4 v in acc[u][t][v], -W's in w[u][t][v]: W_t = sum over
+    // P's rows 16 t + g + 4 v in tot[u][t][v], -W's in w[u][t][v]: W_t = sum over
     // the blocks k <= t of T_kt^T P_k
     dbl4 w[U][4];
 #pragma unroll
@@ -227,7 +238,7 @@ __device__ __forceinline__ void bt_trailing(double* a, int lda, int j, int m, in
           const double x = -L.Ts[(16 * k + g + 4 * v) + (16 * t + li) * KMAX];
 #pragma unroll
           for (int u = 0; u < U; u++)
-            w[u][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, acc[u][k][v], w[u][t], 0, 0, 0);
+            w[u][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, tot[u][k][v], w[u][t], 0, 0, 0);
         }
     }
     auto up = [&](int ch, Regs& x0, Regs& x1) {

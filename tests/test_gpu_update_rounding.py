@@ -115,6 +115,29 @@ def test_dm_first_step(m, n, nb):
     check_block(a[cols].cpu().numpy().T, c0, unit_lower(fac, k), tau[:k].cpu().numpy(), 1, 16, k)
 
 
+def test_batched_first_step():
+    m, n = 1024, 512
+    it = (qrdm_amd.BatchItem * 1)(qrdm_amd.BatchItem(m, n, m, 0, 0, 0, 0))
+    lib = qrdm_amd.lib()
+    plan = lib.qrdm_batch_plan_create(1, it, 64)
+    assert plan
+    a = gaussian(m, n, 5)
+    a0 = a.clone()
+    tau = torch.zeros(n, dtype=torch.float64, device="cuda")
+    jp, nc, info = (torch.zeros(q, dtype=torch.int32, device="cuda") for q in (n, n, 1))
+    assert lib.qrdm_dgeqrdm_batched(plan, vp(a), vp(tau), vp(jp), vp(nc), vp(info),
+                                    TH.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), 0, 0,
+                                    None) == 0
+    torch.cuda.synchronize()
+    lib.qrdm_batch_plan_destroy(plan)
+    assert int(info[0]) == 0
+    k = int(nc[0])
+    cols = np.arange(n // 2, n, 8)
+    c0 = a0[(jp.long() - 1)[torch.from_numpy(cols).cuda()]].cpu().numpy().T
+    fac = a[:k].cpu().numpy().T
+    check_block(a[cols].cpu().numpy().T, c0, unit_lower(fac, k), tau[:k].cpu().numpy(), 1, 4, k)
+
+
 @pytest.mark.parametrize("left", [1e-5, 1e-2])
 def test_update_rounds_each_entry_once(left):
     # C is the panel's columns combined, and entries of size left / 16 on the lower
