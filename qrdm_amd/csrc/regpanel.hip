@@ -22,6 +22,14 @@
 // column's partial sums pass between the workgroups through memory, each in a slot
 // that holds a sentinel until it is written.
 //
+// The workgroups of such a panel wait for each other, so all of them have to be on
+// the chip at once.  They meet before column 0 (rp_all_here), while nothing is
+// written: where one does not arrive in time -- another kernel or process holds the
+// CUs -- all of them decline, and the memory-based panel, one workgroup that waits
+// for nobody, takes it.  Once all have met they stay, and every later wait ends.
+// Devices with fewer CUs than the panel has workgroups, and streams with a CU mask,
+// go to the memory-based panel at once.
+//
 // Measured for 64 columns, with V and T (rocprofv3): up to 128 rows 65 us, up
 // to 448 rows 104 us (memory-based: about 180 us for 64 rows, with T another
 // 60), 1024 rows on five workgroups 136 us, 4096 rows on nineteen 160 us
@@ -36,6 +44,11 @@
 // Sums of squares are taken plainly: where one leaves [1e-280, 1e280] (or is
 // not a number) the panel is declined before anything is written, and the
 // memory-based panel, which scales, takes it.
+#include <stdlib.h>
+#include <string.h>
+
+#include <algorithm>
+
 #include "qrdm_internal.h"
 
 namespace qrdm {
@@ -54,8 +67,15 @@ constexpr int RP_XCD = 28;
 // A slot not yet written: a NaN pattern no published value takes (published
 // NaNs are made the canonical one).
 __device__ constexpr unsigned long long kRpEmpty = 0x7ff4a5a5c3c30f0full;
-// Polls of one slot before a workgroup gives the panel up (about seconds).
+// Polls of one slot before a workgroup gives the panel up (about seconds; only a
+// workgroup that is gone could keep one empty).
 constexpr int RP_POLLS = 1 << 22;
+// Polls for the workgroups not here yet before all decline: about as long as the
+// memory-based panel takes at 4096 rows.
+constexpr int RP_MEET = 1 << 12;
+// The meeting's word (the first of the slots' space): how many are here, and whether
+// one has declined for all.
+constexpr unsigned kRpDeclined = 0x80000000u;
 
 // Two doubles at any multiple of eight bytes.
 typedef double rp_pair __attribute__((ext_vector_type(2), aligned(8)));
@@ -72,6 +92,7 @@ struct RegPanelLds {
   double X[KMAX][LDP];          // T
   double Y[4][BLK][BLK + 1];
   double tau[KMAX];
+  int here;
 };
 
 // (lane 16 g + li) := the sum over the four lane groups of s[g], column 16 g + li.
@@ -158,11 +179,27 @@ __device__ __forceinline__ bool rp_collect(const double* slots, int first, int s
   return true;
 }
 
+// Whether all nwg workgroups, each counted into *word, are here; false for all of
+// them when one has waited RP_MEET polls in vain.  (One thread.  The word goes from
+// "not all here" to one of the two answers once, by the last arrival's count or by
+// the exchange, and every workgroup, a late one too, reads that answer.)
+__device__ __forceinline__ bool rp_all_here(unsigned* word, unsigned nwg) {
+  for (int polls = 0;; polls++) {
+    unsigned v = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v & kRpDeclined) return false;
+    if (v == nwg) return true;
+    if (polls >= RP_MEET)
+      __hip_atomic_compare_exchange_strong(word, &v, v | kRpDeclined, __ATOMIC_RELAXED,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 // The panel's columns [0, fjb) at P (leading dimension lda, msub rows) by nwg
 // workgroups, this one the rows from wg * 16 QH NW.  Truncation: 5e-14 is the
 // bound of the columns after the first (tau_dm > 0: tau_dm |R(0, 0)| once
 // column 0 is done), unless truncate is 0; truncate = 2: beta0 is the block's
-// R(0, 0), and every column is tested.  slots (nwg > 1): four columns' sets
+// R(0, 0), and every column is tested.  slots (GRID): the meeting's word, in which
+// this workgroup is counted, and, from KMAX values on, four columns' sets
 // of (nwg + 1) x KMAX values, empty on entry; column i uses set i mod 4 and
 // empties its own slot of column i + 2, whose values (of column i - 2) every
 // workgroup has read before any publishes column i - 1.  Returns the columns reduced with
@@ -206,6 +243,12 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
       a[u][4 * h + 2] = hi.x;
       a[u][4 * h + 3] = hi.y;
     }
+  if constexpr (GRID) {
+    if (tid == 0) L.here = rp_all_here(reinterpret_cast<unsigned*>(slots), nwg) ? 1 : 0;
+    lds_barrier();
+    if (!L.here) return -1;
+    slots += KMAX;
+  }
   // column 16 u + ii to LDS: its owner lanes' rows, zero on and above the diagonal
   auto put_column = [&](int u, int ii) {
     if (li == ii) {
@@ -483,6 +526,10 @@ __global__ __launch_bounds__(64 * (NW + 1)) void k_panel_reg(double* A, int lda,
   const int wg = blockIdx.x / stride;
   // one workgroup in stride works; the grid is sized for the lowest j
   if (wg * stride != (int)blockIdx.x || wg >= nwg) return;
+  // (counted first: the panel's loads run beside the wait for the others)
+  if (GRID && threadIdx.x == 0)
+    __hip_atomic_fetch_add(reinterpret_cast<unsigned*>(ws_slots(st)), 1u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
   const double beta0 = truncate == 2 ? st->pan_beta : 0.0;
   const int k = reg_panel<QH, NW, GRID>(A + j + (size_t)j * lda, lda, msub, fjb, tau_dm, truncate,
                                         beta0, tau, V + j, ldv, min(j, KMAX),
@@ -574,18 +621,40 @@ __global__ __launch_bounds__(1024) void k_panel_slow(double* A, int lda, int j, 
   }
 }
 
-// Every slot of a panel by nwg workgroups empty (see kRpEmpty).
-__global__ __launch_bounds__(256) void k_panel_slots(DevState* st, int n, int mode) {
+// The meeting's word (nobody here, or declined), and every slot of a panel by several
+// workgroups empty (see kRpEmpty).
+__global__ __launch_bounds__(256) void k_panel_slots(DevState* st, int n, int mode,
+                                                     unsigned word) {
   if (!step_runs(st, mode)) return;
   unsigned long long* s = reinterpret_cast<unsigned long long*>(ws_slots(st));
-  for (int e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) s[e] = kRpEmpty;
+  for (int e = blockIdx.x * 256 + threadIdx.x; e < KMAX + n; e += gridDim.x * 256)
+    s[e] = e < KMAX ? word : kRpEmpty;
+}
+
+// The CUs that a panel's workgroups can count on: the device's, or none with a mask
+// on the stream.
+static int panel_cus(hipStream_t s) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 0;
+  // (the default streams have no mask, and the call is not for the named ones)
+  if (s == nullptr || s == hipStreamLegacy || s == hipStreamPerThread) return cus;
+  uint32_t mask[32] = {0};
+  if (hipExtStreamGetCUMask(s, 32, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return cus;  // (the meeting decides)
+  }
+  int on = 0;
+  for (uint32_t w : mask) on += __builtin_popcount(w);
+  return on < cus ? 0 : cus;
 }
 
 // The form by the panel's rows (m - j, j the lowest the step can have): up to
 // RP_SMALL rows four waves of 32 rows, up to RP_MID seven of 48, up to RP_ROWS
-// seven of 64 in one workgroup, then RP_ROWS rows per workgroup, all of which
-// have to be resident together: at most RP_WGS of the 256 CUs.  Larger ones
-// stay in memory.
+// seven of 64 in one workgroup, then RP_HALF or RP_ROWS rows per workgroup, at most
+// RP_WGS of them and no more than there are CUs for.  Larger ones stay in memory.
+// (QRDM_PANEL=alone: the panels of several workgroups decline where they meet.)
 void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm,
                         int truncate, double* tau, DevState* st, hipStream_t s, int mode) {
   if (truncate == PANEL_GIVEN) {
@@ -594,9 +663,16 @@ void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm
   }
   const int rows = m - j, nwg = (rows + RP_ROWS - 1) / RP_ROWS;
   const int half = (rows + RP_HALF - 1) / RP_HALF;
+  bool in_memory = nwg > RP_WGS;
   auto grid = [&](auto kernel, int n) {
-    const int stride = n <= RP_XCD ? 8 : 1;
-    hipLaunchKernelGGL(k_panel_slots, dim3(n + 1), dim3(256), 0, s, st, 4 * KMAX * (n + 1), mode);
+    const int cus = panel_cus(s);
+    in_memory = n > cus;
+    if (in_memory) return;
+    const int stride = n <= std::min(RP_XCD, cus / 8) ? 8 : 1;
+    const char* pe = getenv("QRDM_PANEL");
+    const unsigned word = pe && strcmp(pe, "alone") == 0 ? kRpDeclined : 0u;
+    hipLaunchKernelGGL(k_panel_slots, dim3(n + 2), dim3(256), 0, s, st, 4 * KMAX * (n + 1), mode,
+                       word);
     hipLaunchKernelGGL(kernel, dim3(n * stride), dim3(512), 0, s, A, lda, j, m, fjb, tau_dm,
                        truncate, tau, st, mode, stride);
   };
@@ -614,7 +690,7 @@ void launch_panel_exact(double* A, int lda, int j, int m, int fjb, double tau_dm
   else if (nwg <= RP_WGS)
     grid(k_panel_reg<4, 7, true>, nwg);
   hipLaunchKernelGGL(k_panel_slow, dim3(1), dim3(1024), 0, s, A, lda, j, m, fjb, tau_dm,
-                     truncate, tau, st, mode, nwg > RP_WGS ? 1 : 0);
+                     truncate, tau, st, mode, in_memory ? 1 : 0);
 }
 
 }  // namespace qrdm
