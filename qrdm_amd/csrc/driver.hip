@@ -745,8 +745,11 @@ int run_dm(const Args& x) {
     if (x.nsteps) *x.nsteps = it;
     HIPCHK(hipMemcpyAsync(x.jpvt, B.jp, sizeof(int) * n, hipMemcpyDeviceToHost, s));
     if (it > 0) HIPCHK(hipMemcpyAsync(x.ncols, B.ncols, sizeof(int) * it, hipMemcpyDeviceToHost, s));
+  } else {
+    HIPCHK(hipMemcpyAsync(hst, B.st, sizeof(DevState), hipMemcpyDeviceToHost, s));
   }
   HIPCHK(hipStreamSynchronize(s));
+  if (nfxd >= minmn) check_panels(hst->flags);
   if (g_prof.on) {
     g_prof.resolve();
     HIPCHK(hipMemcpy(hst, B.st, sizeof(DevState), hipMemcpyDeviceToHost));
