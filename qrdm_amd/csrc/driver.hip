@@ -345,7 +345,10 @@ int run_wide(const Args& x, Buffers& B, int nfxd, double eta, int enable_stop, d
     HIPCHK(hipStreamSynchronize(s));
     const int nc = hout[0], fjb = hout[1];
     sel.resize(fjb);
-    for (int q = 0; q < fjb; q++) sel[q] = hidx[hout[2 + q]];
+    for (int q = 0; q < fjb; q++) {
+      sel[q] = hidx[hout[2 + q]];
+      if (sel[q] < 0 || sel[q] >= nsub) throw HipError{hipErrorUnknown, "wide step's candidates"};
+    }
     // permute_marked (:149-262): the walk here, the moves on the device
     permute_walk(nsub, marked, sel.data(), fjb, swaps);
     pairs.resize(2 * swaps.size());

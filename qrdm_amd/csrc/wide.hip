@@ -51,7 +51,9 @@ __global__ __launch_bounds__(256) void k_topk_wide(const double* __restrict__ va
     const bool in = g < L;
     const double v = val_in[min(g, L - 1)];
     const int i = idx_in ? idx_in[min(g, L - 1)] : g;
-    sv[e] = in ? v : -1.0;  // norms are >= 0
+    // norms are >= 0; one that overflowed to a NaN counts as 0 (with a NaN among the
+    // keys they have no order, and places stay empty)
+    sv[e] = !in ? -1.0 : (v == v ? v : 0.0);
     si[e] = in ? i : INT_MAX;
   }
   __syncthreads();

@@ -1,5 +1,5 @@
-"""The host code's answers to a device state that is no result (tests/hostcheck/bad_state.cpp),
-on the CPU: the call fails."""
+"""The host code's answers to device states that are no results (tests/hostcheck/bad_state.cpp),
+on the CPU: the call fails, and nothing is indexed with them."""
 import os
 import subprocess
 
@@ -32,3 +32,6 @@ def result(program, what):
 def test_panel_given_up_with_every_column_fixed(program):
     assert result(program, "panel") <= -1000
 
+
+def test_wide_candidate_past_the_columns(program):
+    assert result(program, "index") <= -1000
