@@ -594,6 +594,7 @@ __device__ __forceinline__ int bt_factor(const BatchItem& it, double* A, double*
       for (int b = wave; 64 * b < nsub; b += NW) {
         const int t = 64 * b + lane;
         double bv = (t < nsub) ? L.work[j + t] : -1.0;
+        bv = bv == bv ? bv : 0.0;  // (as k_topk)
         int bi = (t < nsub) ? t : 0x40000000 + t;
         wave_sort64(bv, bi);
         wave_merge64(v, ix, bv, bi);

@@ -464,8 +464,11 @@ __global__ __launch_bounds__(64 * TOPK_WAVES) void k_topk(const double* __restri
   int ix = 0;
   if (sort) {
     const int t = blockIdx.x * TOPK_BLOCK + 64 * wave + lane;
-    // padding keys: -1 (norms are >= 0) with distinct indices past any column
+    // padding keys: -1 (norms are >= 0) with distinct indices past any column; a
+    // norm that overflowed to a NaN counts as 0 (a comparison with it would keep one
+    // key of a pair twice, and padding could come first)
     v = (t < nsub) ? work[j + t] : -1.0;
+    v = v == v ? v : 0.0;
     ix = (t < nsub) ? t : 0x40000000 + t;
     wave_sort64(v, ix);
     lv[wave][lane] = v;
