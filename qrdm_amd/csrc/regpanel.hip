@@ -43,7 +43,8 @@
 //
 // Sums of squares are taken plainly: where one leaves [1e-280, 1e280] (or is
 // not a number) the panel is declined before anything is written, and the
-// memory-based panel, which scales, takes it.
+// memory-based panel, which scales, takes it.  So are panels with a column below
+// that range that may never be summed itself.
 #include <stdlib.h>
 #include <string.h>
 
@@ -212,8 +213,8 @@ template <int QH, int NW, bool GRID>
 __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, double tau_dm,
                                          int truncate, double beta0, double* tau, double* V,
                                          int ldv, int z0, double* T_out, double* S_out,
-                                         double* slots, int nwg, int wg, DevState* st,
-                                         RegPanelLds<QH, NW>& L) {
+                                         double* slots, int nwg, int wg, bool scales,
+                                         DevState* st, RegPanelLds<QH, NW>& L) {
   constexpr int WR = 16 * QH, NQ = 4 * QH, NT = 64 * (NW + 1);
   const int tid = local_tid(), lane = tid & 63, g = lane >> 4, li = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -276,7 +277,7 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
   int k = fjb;
   bool ok = true;
   // After the data waves' partial sums of column i: sum := x^T (column lane),
-  // rv := row i's entry there.
+  // rv := row i's entry there.  (i = -1: any sums, before column 0's.)
   auto exchange = [&](int i, double& sum, double& rv) {
     const int buf = i & 1;
     lds_barrier();
@@ -365,6 +366,23 @@ __device__ __forceinline__ int reg_panel(double* P, int lda, int msub, int fjb, 
     }
     return true;
   };
+  // A column whose entries are all so small that their products with an accepted
+  // column could be lost (each entry counts 1 from 1e-140 on, below that 2^-30): the
+  // panel is declined.
+  if (scales) {
+    if (data) {
+      double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int q = 0; q < NQ; q++)
+          s[u] += fabs(a[u][q]) >= 1e-140 ? 1.0 : (a[u][q] != 0.0 ? 0x1p-30 : 0.0);
+      L.red[1][wave][lane] = group_sums(s);
+    }
+    double sum, rv;
+    exchange(-1, sum, rv);
+    if (__any(sum > 0.0 && sum < 1.0)) return -1;
+  }
   if (data) {
     put_column(0, 0);
     put_row(0, 0);
@@ -526,6 +544,11 @@ __global__ __launch_bounds__(64 * (NW + 1)) void k_panel_reg(double* A, int lda,
   const int wg = blockIdx.x / stride;
   // one workgroup in stride works; the grid is sized for the lowest j
   if (wg * stride != (int)blockIdx.x || wg >= nwg) return;
+  // Columns that no test of their own reaches: those the truncation rejects, and one
+  // with a single row left.  As DM candidates they are above tau_dm times the first
+  // column's norm, which is tested; otherwise the panel looks at their scale first.
+  const bool picked = truncate && tau_dm >= 1e-20 && !(mode != RUN_ALWAYS && st->policy_on);
+  const bool scales = (truncate || fjb >= msub) && !picked;
   // (counted first: the panel's loads run beside the wait for the others)
   if (GRID && threadIdx.x == 0)
     __hip_atomic_fetch_add(reinterpret_cast<unsigned*>(ws_slots(st)), 1u, __ATOMIC_RELAXED,
@@ -535,7 +558,8 @@ __global__ __launch_bounds__(64 * (NW + 1)) void k_panel_reg(double* A, int lda,
                                         beta0, tau, V + j, ldv, min(j, KMAX),
                                         mode != RUN_ALWAYS && st->fused ? nullptr
                                                                         : ws_mat(st, WS_T),
-                                        ws_mat(st, WS_S), ws_slots(st), nwg, wg, st, L);
+                                        ws_mat(st, WS_S), ws_slots(st), nwg, wg, scales, st,
+                                        L);
   if (wg == 0 && threadIdx.x == 0) {
     if (k < 0) {
       atomicOr(&st->flags, 4);
