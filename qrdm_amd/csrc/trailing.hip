@@ -33,6 +33,7 @@
 #include "qrdm_internal.h"
 
 #include <algorithm>
+#include <climits>
 
 namespace qrdm {
 
@@ -76,18 +77,21 @@ __host__ __device__ __forceinline__ int fused_per_xcd(int ns, int cgroups) {
 // Row slabs of a fused pass, at most one round of the chip's 64 workgroups per
 // XCD (two per CU): the cost of a count in chunks -- a slab's chunks and two for its
 // start and its partial tile, 1.7 times as long with a second workgroup on the CU,
-// and a twentieth per slab for the step's end -- or a large value where Wp (16 x 64
-// x n values) does not hold the partials.  Measured (us by workgroups per XCD, 4096
-// x 4096): 32 87, 48 104, 56 92, 64 79; 16384 x 512: 16 87, 32 50, 64 49; 1024 x
-// 1024: 16 16, 32 12, 64 15.  (Waves of 32 columns: 312 against 317 at 8192 x 8192,
-// 169 against 160 at 8192 x 4096; groups of 96 or 128 columns were slower
-// throughout.)
-__host__ __device__ __forceinline__ float fused_cost(int ns, int nchunk, int cgroups, int ncol,
-                                                     int n) {
+// and a twentieth per slab for the step's end -- in twentieths, or INT_MAX where Wp
+// (16 x 64 x n values) does not hold the partials.  Whole numbers: the pass and the
+// step's end each choose, and have to agree, and counts tie (72608 x 448: 36 and 64
+// slabs; in floats the choice there depends on how the sum is rounded).  Measured
+// (us by workgroups per XCD, 4096 x 4096): 32 87, 48 104, 56 92, 64 79; 16384 x 512:
+// 16 87, 32 50, 64 49; 1024 x 1024: 16 16, 32 12, 64 15.  (Waves of 32 columns: 312
+// against 317 at 8192 x 8192, 169 against 160 at 8192 x 4096; groups of 96 or 128
+// columns were slower throughout.)
+__host__ __device__ __forceinline__ int fused_cost(int ns, int nchunk, int cgroups, int ncol,
+                                                   int n) {
   const int per = fused_per_xcd(ns, cgroups);
-  if (ns > 1 && (per > 32 * FU_OCC || ns > nchunk || (long long)ns * ncol > 16LL * n)) return 1e9f;
-  const float chunks = (float)((nchunk + ns - 1) / ns) + 2.0f;
-  return (per > 32 ? 1.7f : 1.0f) * chunks + 0.05f * (float)ns;
+  if (ns > 1 && (per > 32 * FU_OCC || ns > nchunk || (long long)ns * ncol > 16LL * n))
+    return INT_MAX;
+  const int chunks = (nchunk + ns - 1) / ns + 2;
+  return (per > 32 ? 34 : 20) * chunks + ns;
 }
 
 // The count with the least cost, by a wave (lane: count lane + 1): the DM loop's
@@ -99,9 +103,7 @@ __device__ __forceinline__ int fused_slabs_wave(int r_lo, int m, int c0, int n) 
   const FuGeom g = fused_geom(r_lo, m, c0, n, 1);
   if (g.cgroups <= 0 || g.nchunk <= 0) return 1;
   const int ns = (local_tid() & 63) + 1;
-  const float cost = fused_cost(ns, g.nchunk, g.cgroups, n - c0, n);
-  // costs are positive: their bits are ordered as they are; equal ones, fewer slabs
-  int best = __float_as_int(cost), arg = ns;
+  int best = fused_cost(ns, g.nchunk, g.cgroups, n - c0, n), arg = ns;  // ties: fewer slabs
   auto take = [&](int ob, int oa) {
     const bool t = ob < best || (ob == best && oa < arg);
     best = t ? ob : best;
