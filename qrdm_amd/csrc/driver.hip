@@ -31,10 +31,13 @@ thread_local std::string g_err;
 constexpr double kEps = 1.1102230246251565e-16;  // LAPACK dlamch('E') = 2^-53
 // Panels with at least this many rows take the Gram-based path, five launches of
 // about 75 us in all; below, the register-held panel of one workgroup, 65 us up to
-// 128 rows and 87 up to 336, with 9 for its column moves and fallback.  Measured
-// (us, whole calls by this limit 129 / 193 / 257 / 385): 130 x 64 270 / 241 / 241 /
-// 242, 256 x 256 732 / 766 / 756 / 755, 384 x 64 254 / 254 / 254 / 265, 384 x 300
-// 810 / 844 / 851 / 910, 900 x 900 2225 / 2259 / 2253 / 2280.
+// 128 rows and 87 up to 336, with 9 for its column moves and fallback.  No limit is
+// best everywhere (us, whole calls by this limit 129 / 193 / 257): matrices of no more
+// than 256 rows and few columns want the register-held panel (200 x 32 229 / 229 / 188,
+// 256 x 64 254 / 253 / 231, 130 x 64 255 / 226 / 228, 200 x 100 377 / 361 / 354), the
+// last steps of larger ones the Gram-based one (256 x 256 668 / 702 / 690, 384 x 300
+// 789 / 821 / 828, 512 x 512 1277 / 1322 / 1326, 900 x 900 2175 / 2195 / 2201, 600 x 400
+// 1064 / 1050 / 1042).  257: the former gain 6 to 18 %, the latter lose 1 to 5.
 constexpr int kFastPanelRows = 257;
 constexpr int kBatch = 8;  // DM steps queued between synchronisations
 // Layout of the per-step upload: up to 2*KMAX (dst, src) pairs, then KMAX

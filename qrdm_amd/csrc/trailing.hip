@@ -269,18 +269,18 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
   for (int t = 0; t < 4; t++) acc[t] = tot[t] = (dbl4){0.0, 0.0, 0.0, 0.0};
   // chunk c of V into LDS: a wave takes the columns 16 w .. 16 w + 15, four
   // per load (lane: column lane / 16, unit lane % 16): the lane's byte offsets
-  // from the wave's first column
+  // from the load's first column
   unsigned voff[4];
 #pragma unroll
   for (int i = 0; i < 4; i++)
-    voff[i] = 8u * ((unsigned)(4 * i + g) * (unsigned)ldv + 2u * (unsigned)(li ^ (4 * i + g)));
+    voff[i] = 8u * ((unsigned)g * (unsigned)ldv + 2u * (unsigned)(li ^ (4 * i + g)));
   auto load_v = [&](const double* V, FuChunk& S, int c) {
-    const char* src =
-        reinterpret_cast<const char*>(V + (size_t)(16 * wave) * ldv + G.base + FU_CH * c);
+    const double* col = V + (size_t)(16 * wave) * ldv + G.base + FU_CH * c;
 #pragma unroll
     for (int i = 0; i < 4; i++)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(src + voff[i]),
+          (const __attribute__((address_space(1))) void*)(
+              reinterpret_cast<const char*>(col + (size_t)(4 * i) * ldv) + voff[i]),
           (__attribute__((address_space(3))) void*)&S[16 * wave + 4 * i][0], 16, 0, 0);
   };
   // chunk c of C as it lies in memory: rows base + 32c + 8v + 2g + (0, 1) in
