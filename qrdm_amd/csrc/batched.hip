@@ -48,7 +48,7 @@ struct BatchLds {
     } tk;                       // the top-k's per-wave lists
     double E[2][KMAX][LDP];     // the Gram-based panel's matrices
   } u;
-  double R1[KMAX * LDP];  // Gram slab / G / V^T V / trailing-update W
+  double R1[KMAX * LDP];  // candidate Gram / V^T V (the panel's scratch after it)
   double Ts[KMAX * LDP];  // T (column-major, leading dimension KMAX)
   double ts[KMAX], tmp[KMAX];
   double rinv[KMAX], dsg[KMAX], tl[KMAX], scv[KMAX];

@@ -169,8 +169,9 @@ struct Buffers {
 
 size_t layout_buffers(int m, int n, char* base, Buffers* b, int nb = KMAX) {
   char* p = base;
-  const int nsplit = 16;  // row slabs of the trailing update's partial products
-  static_assert(nsplit >= 16, "the fused pass uses up to 16 row slabs");
+  // row slabs of the three-kernel update's partial products; the merged pass takes
+  // as many as fit in the same 16 x KMAX x n values
+  const int nsplit = 16;
   Buffers t;
   // the head that kernels find from the state (ws_mat, ws_slots, ws_v)
   t.st = carve<DevState>(p, 1);

@@ -538,31 +538,6 @@ void launch_topk(const double* work, int j0, int m, int n, int nb, double tau, d
 }
 
 // ---------------------------------------------------------------------------
-// out = X^T X (64 x 64, column-major) for the 64-row slab X held in LDS as
-// X[c * (GRAM_ROWS + 1) + r]; 256 threads, wave w computes rows 16w..16w+15
-// on the matrix cores.
-__device__ __forceinline__ void gram_slab_acc(const double* X, dbl4 (&acc)[4]) {
-  const int lane = local_tid() & 63, wv = local_tid() >> 6;
-  const int g = lane >> 4, li = lane & 15;
-#pragma unroll 4
-  for (int k0 = 0; k0 < GRAM_ROWS; k0 += 4) {
-    const double a = X[(16 * wv + li) * (GRAM_ROWS + 1) + k0 + g];
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-      acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-          a, X[(16 * u + li) * (GRAM_ROWS + 1) + k0 + g], acc[u], 0, 0, 0);
-  }
-}
-
-__device__ __forceinline__ void gram_store(const dbl4 (&acc)[4], double* out) {
-  const int lane = local_tid() & 63, wv = local_tid() >> 6;
-  const int g = lane >> 4, li = lane & 15;
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) out[(16 * wv + g + 4 * v) + (16 * u + li) * KMAX] = acc[u][v];
-}
-
 // One 16-row block's contribution to a wave's Gram X^T X (64 x 64): xb[u]
 // holds X_blk(:, 16u .. 16u + 15) in the matrix cores' output layout (rows
 // g + 4v, column 16u + li for lane 16g + li), which is also the operand layout

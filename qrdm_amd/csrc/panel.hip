@@ -1101,7 +1101,7 @@ __global__ __launch_bounds__(256) void k_reduce_recon(const double* __restrict__
                                                       const double* __restrict__ R1,
                                                       const double* __restrict__ R1inv,
                                                       double* A, int lda, double tau_dm,
-                                                      double* tau, double* T_out, double* M_out,
+                                                      double* tau, double* M_out,
                                                       unsigned* ticket, DevState* st) {
   __shared__ double part[4][64];
   __shared__ int s_last;
@@ -1334,7 +1334,7 @@ void launch_panel_fast(double* A, int lda, int j0, int m, double tau_dm, double*
   const int nslab = (m - j0 + PR_ROWS - 1) / PR_ROWS;
   hipLaunchKernelGGL(k_qgram, dim3(nslab), dim3(256), 0, s, A, lda, m, R1inv, st, gram_part);
   hipLaunchKernelGGL(k_reduce_recon, dim3(KMAX * KMAX / 64), dim3(256), 0, s, gram_part, nslab,
-                     G2, R1, R1inv, A, lda, tau_dm, tau, T, M, ticket, st);
+                     G2, R1, R1inv, A, lda, tau_dm, tau, M, ticket, st);
   hipLaunchKernelGGL(k_v2, dim3(nslab), dim3(256), 0, s, A, lda, m, M, tau, st, bufs, gram_part);
   // the merged trailing pass sums V^T V itself (k_fused)
   if (bufs.vstride == 0)

@@ -123,9 +123,6 @@ __device__ __forceinline__ double* v_cur(const StepBufs& b, const DevState* st) 
 __device__ __forceinline__ double* v_prev(const StepBufs& b, const DevState* st) {
   return b.V + (size_t)((st->it & 1) ^ 1) * b.vstride;
 }
-__device__ __forceinline__ double* w_cur(const StepBufs& b, const DevState* st) {
-  return b.W + (size_t)(st->it & 1) * b.wstride;
-}
 __device__ __forceinline__ double* w_prev(const StepBufs& b, const DevState* st) {
   return b.W + (size_t)((st->it & 1) ^ 1) * b.wstride;
 }
@@ -406,10 +403,9 @@ void launch_zero(void* p, size_t bytes, hipStream_t s);
 void launch_set_fused(DevState* st, int fused, hipStream_t s);
 
 // ---- the merged trailing update (trailing.hip) -------------------------------
-// Row slabs of a fused pass over rows [r_lo, m), columns [c0, n) (at most
-// fused_max_slabs()); the partials Wp hold that many KMAX x n blocks.
+// Row slabs of a fused pass over rows [r_lo, m), columns [c0, n): as many KMAX x
+// (n - c0) partials as Wp's 16 x KMAX x n values hold, at most 64.
 int fused_slabs(int r_lo, int m, int c0, int n);
-int fused_max_slabs();
 // One pass over C (rows [r_lo, m), columns [c0, n)): apply: C -= V_prev
 // W_prev; accum: Wp[slab] = V_cur^T C.  With st (the DM loop) r_lo and c0
 // come from st (host values: lower bounds sizing the grid) and the buffers
@@ -421,7 +417,7 @@ void launch_fused(double* A, int lda, int r_lo, int m, int c0, int n, const Step
 // (zero below c0), the step's R12 rows C_top - V_top W (written), the norm
 // downdate and recompute of those columns (the recomputed ones get the whole
 // update now and a zero W column), into the current W buffer.  j0 <= j sizes
-// the grid; ns as the fused pass.
+// the grid.  (T, ns: not read; the step's T^-1 and slabs follow from st.)
 void launch_wsum_norm(double* A, int lda, int j0, int m, int n, const double* T,
                       const double* Wp, int ns, const StepBufs& bufs, double* work,
                       double* workold, DevState* st, double tol3z, hipStream_t s);

@@ -398,8 +398,6 @@ __global__ __launch_bounds__(64 * FU_NWG, FU_OCC) void k_fused(double* A, int ld
     for (int w = 0; w < 4; w++) out[(size_t)(16 * t + g + 4 * w) * ldw] = tot[t][w];
 }
 
-int fused_max_slabs() { return FU_MAX_SPLIT; }
-
 int fused_slabs(int r_lo, int m, int c0, int n) {
   const FuGeom g = fused_geom(r_lo, m, c0, n, 1);
   if (g.cgroups <= 0 || g.nchunk <= 0) return 1;
@@ -700,8 +698,10 @@ __global__ __launch_bounds__(256) void k_wsum_norm(double* A, int lda, int m, in
 void launch_wsum_norm(double* A, int lda, int j0, int m, int n, const double* T,
                       const double* Wp, int ns, const StepBufs& bufs, double* work,
                       double* workold, DevState* st, double tol3z, hipStream_t s) {
-  (void)T;   // the step's T^-1 lies behind the state (ws_mat WS_S)
-  (void)ns;  // the slabs as the pass chose them
+  // (T, ns: what the three-kernel update's W takes; here T^-1 lies behind the state
+  // (ws_mat WS_S) and the slabs are as the pass chose them)
+  (void)T;
+  (void)ns;
   // tiles of [j + kk, n), j + kk >= j0 + 1; one workgroup at least (it marks
   // the step's end pending).
   int tiles = (n - j0 - 1 + WN_TC - 1) / WN_TC;
@@ -822,7 +822,7 @@ void launch_wsum_fused(int c0, int n, const double* T, int trans, const double* 
 // A block reflector on its own: V^T C, W = op(T) V^T C, C -= V W.
 void launch_larfb(double* A, int lda, int j, int m, int c0, int n, const double* V, int ldv,
                   const double* T, int trans, double* Wp, double* W, int nsplit, hipStream_t s) {
-  (void)nsplit;  // Wp holds the slabs that fused_slabs chooses
+  (void)nsplit;  // the three-kernel update's slabs: fused_slabs chooses those here
   if (n - c0 <= 0 || m - j <= 0) return;
   const StepBufs bufs{const_cast<double*>(V), 0, ldv, W, 0};
   const int ns = fused_slabs(j, m, c0, n);
