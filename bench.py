@@ -36,7 +36,7 @@ HBM_PEAK_GBS = 8000.0
 # norm sweep reads the matrix once, the restore copy writes it once), averaged
 # over the launches of the workload (m, n, rank, nb); measured with
 # rocprofv3 --pmc, summary in profiles/k_fused_8192_pmc_traffic.md.
-FUSED_TRAFFIC = {(8192, 8192, 2048, 64): 364.9e6}
+FUSED_TRAFFIC = {(8192, 8192, 2048, 64): 397.8e6}
 
 
 def fused_algorithmic_bytes(m, n, ncols):

@@ -30,16 +30,16 @@
 // Devices with fewer CUs than the panel has workgroups, and streams with a CU mask,
 // go to the memory-based panel at once.
 //
-// Measured for 64 columns, with V and T (rocprofv3): up to 128 rows 65 us, up
-// to 448 rows 104 us (memory-based: about 180 us for 64 rows, with T another
+// Measured for 64 columns, with V and T (rocprofv3): up to 128 rows 67 us, up to 336
+// rows 87, up to 448 rows 105 us (memory-based: about 180 us for 64 rows, with T another
 // 60), 1024 rows on five workgroups 136 us, 4096 rows on nineteen 160 us
 // (memory-based 3.8 ms; on ten workgroups over all XCDs 189).  A column costs
 // about 2500 cycles at 128 rows and 3600 at 448, of which the reflector's scalars
 // take 280; between workgroups the exchange adds 2000 to 2500.  The loop is
 // unrolled over the four column groups so that every register index is static:
 // with uniform branches in their place the 448-row panel took 163 us.  Unpivoted
-// QR of 1024 x 1024 15.6 -> 2.2 ms, of 4096 x 2048 129 -> 6.7 ms; 2048 x 1024 DM
-// with 128-column blocks 68.4 -> 4.2 ms; 64 x 48 DM 0.53 -> 0.21 ms.
+// QR of 1024 x 1024 15.5 -> 2.3 ms, of 4096 x 2048 129 -> 6.6 ms; 2048 x 1024 DM
+// with 128-column blocks 68.2 -> 4.25 ms; 64 x 48 DM 0.51 -> 0.22 ms.
 //
 // Sums of squares are taken plainly: where one leaves [1e-280, 1e280] (or is
 // not a number) the panel is declined before anything is written, and the
@@ -71,8 +71,8 @@ __device__ constexpr unsigned long long kRpEmpty = 0x7ff4a5a5c3c30f0full;
 // Polls of one slot before a workgroup gives the panel up (about seconds; only a
 // workgroup that is gone could keep one empty).
 constexpr int RP_POLLS = 1 << 22;
-// Polls for the workgroups not here yet before all decline: about as long as the
-// memory-based panel takes at 4096 rows.
+// Polls for the workgroups not here yet before all decline: a few milliseconds, about
+// what the memory-based panel takes at 4096 rows.
 constexpr int RP_MEET = 1 << 12;
 // The meeting's word (the first of the slots' space): how many are here, and whether
 // one has declined for all.

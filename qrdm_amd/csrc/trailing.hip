@@ -181,12 +181,12 @@ __device__ __forceinline__ void sum_gram(const DevState* st, int m) {
 // next chunk of V goes from memory straight to the other LDS buffer and the
 // next chunk of C to registers while this one is multiplied (64 products per
 // wave and barrier), so nothing waits for a load issued in the same chunk.
-// Measured: the first pass at 8192 x 8192 317 us, 54 TF/s, the matrix cores busy
-// in 72 % of the cycles (2.23 GHz under this load); per 8192 x 8192
-// factorisation 17.2 ms against 18.2 with 16-row chunks, V stored to LDS
-// through registers and a barrier every 32 products, 16384 x 1024 1.36 against
-// 1.64.  Odd leading dimensions run here too (3001 x 1777 DM 6.53 -> 6.06 ms
-// against the three-kernel form with 8-byte loads).
+// Measured: the first pass at 8192 x 8192 325 us, 52 TF/s of products, the matrix
+// cores busy in 75 % of the cycles, 62 % over all passes (117 us on average); per 8192
+// x 8192 factorisation 15.1 ms, against 18.2 with 16-row chunks, V stored to LDS
+// through registers and a barrier every 32 products, 16384 x 1024 0.85 against 1.64.
+// Odd leading dimensions run here too (3001 x 1777 DM 6.53 -> 6.06 ms against the
+// three-kernel form with 8-byte loads).
 //
 // V^T C is summed in pieces of two chunks: the error of one running sum grows with
 // its rows, and how many row slabs there are follows from the chip, not from that
